@@ -160,14 +160,51 @@ __device__ __forceinline__ int xcd_brick(int block, int nblocks) {
     return (block & 7) * per + (block >> 3);
 }
 
+// Sum / max over a wavefront: the xor butterfly 32, 16, 8, 4, 2, 1, so every lane ends with the same
+// bits.  The exchanges are register moves (gfx950's half and row swaps, DPP) instead of a shuffle
+// through LDS, about 130 cycles for each of twelve 32-bit halves: most of what a small reducing
+// kernel takes.  After the steps 32, 16 and 8 a value depends on its lane modulo 8 only, so that a
+// rotation by 4 within 16 lanes is the exchange with lane ^ 4.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xF, 0xF, true);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+// v of this lane's half (HALF) or even/odd row pair and of the other one, in a fixed order.
+template <bool HALF>
+__device__ __forceinline__ double2 swap_pair(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)u, hi = (unsigned)(u >> 32);
+    const auto l = HALF ? __builtin_amdgcn_permlane32_swap(lo, lo, false, false)
+                        : __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = HALF ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false)
+                        : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return make_double2(__builtin_bit_cast(double, (unsigned long long)h[0] << 32 | l[0]),
+                        __builtin_bit_cast(double, (unsigned long long)h[1] << 32 | l[1]));
+}
+constexpr int DPP_ROR8 = 0x128, DPP_ROR4 = 0x124, DPP_QUAD_2301 = 0x4E, DPP_QUAD_1032 = 0xB1;
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    const double2 a = swap_pair<true>(v);
+    v = a.x + a.y;
+    const double2 b = swap_pair<false>(v);
+    v = b.x + b.y;
+    v += dpp_move<DPP_ROR8>(v);
+    v += dpp_move<DPP_ROR4>(v);
+    v += dpp_move<DPP_QUAD_2301>(v);
+    v += dpp_move<DPP_QUAD_1032>(v);
     return v;
 }
 __device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+    const double2 a = swap_pair<true>(v);
+    v = fmax(a.x, a.y);
+    const double2 b = swap_pair<false>(v);
+    v = fmax(b.x, b.y);
+    v = fmax(v, dpp_move<DPP_ROR8>(v));
+    v = fmax(v, dpp_move<DPP_ROR4>(v));
+    v = fmax(v, dpp_move<DPP_QUAD_2301>(v));
+    v = fmax(v, dpp_move<DPP_QUAD_1032>(v));
     return v;
 }
 
