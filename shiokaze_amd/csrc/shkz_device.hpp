@@ -45,6 +45,8 @@ struct GridLevel {
 enum {
     BM_COARSEST = 1,  // the brick's grid ends on this level (its coarse solve handles it)
     BM_UNIFORM = 2,   // level 0: the operator is one constant on the brick (UniCoef)
+    BM_BOTTOM = 4,    // a level of the grid's bottom (BottomGrid): k_bottom works on it
+    BM_BELOW = 8      // ... and not the bottom's first level, whose right-hand side the restriction forms
 };
 struct __align__(32) BrickMeta {
     int nbr[6];
@@ -141,9 +143,32 @@ struct BatchCtl {
 
 // What a V-cycle launch may skip: everything once all grids are done, and the bricks of a grid
 // that is done.  S may be NULL (no per-grid test).
+// skip: the brick flags (BM_*) whose bricks the smoothing kernels leave to another kernel.
 struct Gate {
     const BatchCtl *ctl;
     const SolveScalars *S;
+    int skip;
+};
+
+// The bottom of one grid's hierarchy: its last levels, each of at most BOTTOM_BRICKS stored bricks,
+// down to the single brick of the coarsest one.  One workgroup runs that whole part of the V-cycle
+// (k_bottom), whose arrays and tables these records name.
+constexpr int BOTTOM_BRICKS = 8;
+constexpr int BOTTOM_LEVELS = 4;
+struct BottomLevel {
+    const float *dir, *gx, *gy, *gz, *idiag;  // from the grid's first brick of the level on
+    float *rhs, *z, *tmp;
+    const BrickMeta *meta;
+    const int *bxyz, *child64, *parent8;
+    int brick_start, nb;
+    int deepest;  // the batch's last level (its result is always in z)
+    int flat;
+};
+struct BottomGrid {
+    int n;  // levels (0: the grid has no level below the finest)
+    int pad[3];
+    const int16_t *code;  // component codes of the coarsest brick (k_coarse_components)
+    BottomLevel lev[BOTTOM_LEVELS];
 };
 
 // Deterministic two-pass reduction: every brick of a reducing kernel stores two partials (plain

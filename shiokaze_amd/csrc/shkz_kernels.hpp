@@ -111,10 +111,10 @@ __device__ __forceinline__ bool grid_done(const Gate &Q, const LevelDesc &L, con
     return L.ngrids > 1 && Q.S && Q.S[m.grid].done;
 }
 
-// Smoothing-side V-cycle work on a brick is skipped for a grid that is done or whose last level
-// this is (its coarse solve handles it).
+// Smoothing-side V-cycle work on a brick is skipped for a grid that is done, or where another kernel
+// does it: on the grid's last level (the coarse solve), or on any level of its bottom (k_bottom).
 __device__ __forceinline__ bool skip_smooth(const Gate &Q, const LevelDesc &L, const BrickMeta &m) {
-    return (m.flags & BM_COARSEST) || grid_done(Q, L, m);
+    return (m.flags & Q.skip) || grid_done(Q, L, m);
 }
 
 // Value of level vector v at cell (i,j,k) of the grid described by G (0 outside or unstored).
@@ -1228,43 +1228,25 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_jacobi4_dot(LevelDesc L, OpDes
 constexpr int LOCAL_SGS_SWEEPS = 2;         // finest level: the default (2 or 3, a tuned control)
 constexpr int LOCAL_SGS_SWEEPS_COARSE = 3;  // coarse levels (one application per smoothing step)
 
-// The couplings of the lane's four cells to cells of the same brick (0 across the brick's faces):
-// from the loaded Row4Coef of the level (whose high couplings may come from neighbour bricks).
-__device__ __forceinline__ Row4Coef<float> row4_local(const Row4Coef<float> &g, int q) {
-    const int li = q >> 4, lj = (q >> 1) & 7, h = q & 1;
-    Row4Coef<float> o;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        o.gxm[j] = li > 0 ? g.gxm[j] : 0.0f;
-        o.gxp[j] = li < 7 ? g.gxp[j] : 0.0f;
-        o.gym[j] = lj > 0 ? g.gym[j] : 0.0f;
-        o.gyp[j] = lj < 7 ? g.gyp[j] : 0.0f;
-        const int lk = 4 * h + j;
-        o.gzm[j] = lk > 0 ? g.gzm[j] : 0.0f;
-        o.gzp[j] = lk < 7 ? g.gzp[j] : 0.0f;
-    }
-    return o;
-}
-__device__ __forceinline__ Row4Coef<float> row4_local_uniform(float g, int q) {
+// Row4Coef of a BM_UNIFORM brick.
+__device__ __forceinline__ Row4Coef<float> row4_uniform(float g) {
     Row4Coef<float> u;
 #pragma unroll
     for (int j = 0; j < 4; ++j) u.gxm[j] = u.gxp[j] = u.gym[j] = u.gyp[j] = u.gzm[j] = u.gzp[j] = g;
-    return row4_local(u, q);
+    return u;
 }
 
-// One cell of a lane in the brick-local sweep: what its update needs besides the neighbour values
-// (its x couplings and LDS slots, y couplings, three z weights, inverse diagonal and right-hand side).
+// One cell of a lane in the brick-local sweep: its couplings to the x and y neighbours, the weights of
+// the z terms (the two own cells of the other group and the partner
+// lane's swapped value, see sgs_cells) and its inverse diagonal.
 struct SgsCell {
-    float ax_m, ax_p, ay_m, ay_p;  // couplings to the x and y neighbours (0 across the brick's faces)
-    float za, zb, zs;              // weights of the z terms: the two own cells of the other group and
-                                   // the partner lane's swapped value (see local_sgs4)
-    float id, r;
-    int xm, xp, st;                // LDS slots: x neighbours (clamped in-bounds where the coupling is
-                                   // 0) and the cell's own slot
+    float ax_m, ax_p, ay_m, ay_p;
+    float za, zb, zs;
+    float id;
 };
 
-// e = M_b r on the brick of a 128-thread workgroup (lane q: cells 4q .. 4q+3 of the brick, the
-// storage order).  lds: 512 floats.  Every lane of the workgroup must call it (barriers, DPP).
+// The brick-local sweep on the brick of a 128-thread group (lane q: cells 4q .. 4q+3 of the brick, the
+// storage order).
 //
 // Cell j of the lane has colour col0 ^ (j & 1) (col0 = (li + lj) & 1), so each half-sweep updates
 // two cells of every lane: group P (j = col0, col0 + 2) in the even half-sweeps (the first one, from
@@ -1276,38 +1258,72 @@ struct SgsCell {
 //    the row: lj = 0 / 7, outside the brick);
 //  - z: the lane's own cells of the other group, and at the row's ends the partner lane's
 //    (q ^ 1, same col0) by a DPP lane swap; the weights za, zb, zs place the two couplings;
-//  - x: lanes q -+ 16 (other wavefront at li = 3 / 4), through LDS.
-// A coupling across the brick's faces is 0 and its value is read from an in-bounds slot that holds
-// a sweep value, so the product is a zero.  The sums use fused multiply-adds in a fixed order.
+//  - x: lanes q -+ 16 (other wavefront at li = 3 / 4), through LDS.  Their col0 is opposite too, so the
+//    neighbours of a group's two cells are the other group's two of that lane: LDS holds each group as
+//    one pair of floats per lane, and a half-sweep writes one pair and reads two (8-byte accesses; one
+//    slot per cell took twice the LDS instructions and a select for every address).
+// The sweeps take 0 for the cells across the brick's faces: along y from the DPP shift, along x from a
+// slot of zeros past the group's pairs, along z by a zero weight.  So the couplings need no selects.
+// The sums use fused multiply-adds in a fixed order.
 constexpr int DPP_ROW_SHR2 = 0x112, DPP_ROW_SHL2 = 0x102, DPP_SWAP_PAIRS = 0xB1;  // quad_perm [1,0,3,2]
 template <int CTRL>
 __device__ __forceinline__ float sgs_dpp(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
-__device__ __forceinline__ float sgs_update(const SgsCell &c, const float *lds, float ym, float yp, float z0, float z1,
-                                            float zsw) {
-    float acc = c.r;
-    acc = __builtin_fmaf(c.ax_m, lds[c.xm], acc);
-    acc = __builtin_fmaf(c.ax_p, lds[c.xp], acc);
-    acc = __builtin_fmaf(c.ay_m, ym, acc);
-    acc = __builtin_fmaf(c.ay_p, yp, acc);
-    acc = __builtin_fmaf(c.za, z0, acc);
-    acc = __builtin_fmaf(c.zb, z1, acc);
-    acc = __builtin_fmaf(c.zs, zsw, acc);
-    return c.id * acc;
+// A lane's four cells by group: p0, p1 (group P), q0, q1 (group Q); from the row and back.
+struct SgsRow {
+    float p0, p1, q0, q1;
+};
+__device__ __forceinline__ SgsRow sgs_group(const float v[4], bool c1) {
+    return SgsRow{c1 ? v[1] : v[0], c1 ? v[3] : v[2], c1 ? v[0] : v[1], c1 ? v[2] : v[3]};
+}
+__device__ __forceinline__ void sgs_ungroup(const SgsRow &g, bool c1, float v[4]) {
+    v[0] = c1 ? g.q0 : g.p0;
+    v[1] = c1 ? g.p0 : g.q0;
+    v[2] = c1 ? g.q1 : g.p1;
+    v[3] = c1 ? g.p1 : g.q1;
+}
+__device__ __forceinline__ bool sgs_col1(int q) { return (((q >> 4) + (q >> 1)) & 1) != 0; }
+
+struct SgsCells {
+    SgsCell P0, P1, Q0, Q1;
+};
+
+// Adds the couplings times the neighbours of a group's cells a, b, the other group being (v0, v1), in
+// the sweep's order: x, y, z.  The terms of other lanes (y: rows -+2; z: the pair's swap) use the
+// multiply-add's own DPP operand.  The compiler moves a DPP
+// value to a register first, 6 of 28 instructions of a half-sweep, and these kernels are bound by
+// their issue.  The wait states cover a value written just before.
+__device__ __forceinline__ void sgs_pair(const SgsCell &a, const SgsCell &b, float &accA, float &accB, float2 xm,
+                                         float2 xp, float v0, float v1) {
+    accA = __builtin_fmaf(a.ax_m, xm.x, accA);
+    accB = __builtin_fmaf(b.ax_m, xm.y, accB);
+    accA = __builtin_fmaf(a.ax_p, xp.x, accA);
+    accB = __builtin_fmaf(b.ax_p, xp.y, accB);
+    asm volatile("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %2, %4 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+        "v_fmac_f32_dpp %1, %3, %6 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+        "v_fmac_f32_dpp %0, %2, %5 row_shl:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+        "v_fmac_f32_dpp %1, %3, %7 row_shl:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+        "v_fmac_f32 %0, %2, %8\n\t"
+        "v_fmac_f32 %1, %2, %11\n\t"
+        "v_fmac_f32 %0, %3, %9\n\t"
+        "v_fmac_f32 %1, %3, %12\n\t"
+        "v_fmac_f32_dpp %0, %3, %10 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+        "v_fmac_f32_dpp %1, %2, %13 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf bound_ctrl:0"
+        : "+&v"(accA), "+&v"(accB)
+        : "v"(v0), "v"(v1), "v"(a.ay_m), "v"(a.ay_p), "v"(b.ay_m), "v"(b.ay_p), "v"(a.za), "v"(a.zb), "v"(a.zs),
+          "v"(b.za), "v"(b.zb), "v"(b.zs));
 }
 
-template <int K>
-__device__ __forceinline__ void local_sgs4(const Row4Coef<float> &c, const float id[4], const float r[4], float e[4],
-                                           float *lds, int q) {
-    const int li = q >> 4, lj = (q >> 1) & 7;
-    const int base = 4 * q;
-    const bool c1 = ((li + lj) & 1) != 0;  // col0
-    // The lane's choice between its cells is made on loaded values (one select per field), never on
-    // an array index: an index chosen per lane would keep the arrays in memory (LDS, addressed
-    // through the dispatch packet), on the critical path of every launch.
-    float gxm[4], gxp[4], gym[4], gyp[4], gzm[4], gzp[4], idv[4], rv[4];
+// The lane's cells by group from its couplings and inverse diagonals.
+// The lane's choice between its cells is made on loaded values (one select per field), never on an
+// array index: an index chosen per lane would keep the arrays in memory (LDS, addressed through the
+// dispatch packet), on the critical path of every launch.
+__device__ __forceinline__ SgsCells sgs_cells(const Row4Coef<float> &c, const float id[4], int q) {
+    const bool c1 = sgs_col1(q);
+    float gxm[4], gxp[4], gym[4], gyp[4], gzm[4], gzp[4], idv[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         gxm[j] = c.gxm[j];
@@ -1317,8 +1333,9 @@ __device__ __forceinline__ void local_sgs4(const Row4Coef<float> &c, const float
         gzm[j] = c.gzm[j];
         gzp[j] = c.gzp[j];
         idv[j] = id[j];
-        rv[j] = r[j];
     }
+    if (q & 1) gzp[3] = 0.0f;
+    else gzm[0] = 0.0f;
     // cell ja when col0 = 0, jb when col0 = 1, with the z weights of each case
     auto cell_of = [&](int ja, float za_a, float zb_a, float zs_a, int jb, float za_b, float zb_b, float zs_b) {
         SgsCell o;
@@ -1330,11 +1347,6 @@ __device__ __forceinline__ void local_sgs4(const Row4Coef<float> &c, const float
         o.zb = c1 ? zb_b : zb_a;
         o.zs = c1 ? zs_b : zs_a;
         o.id = c1 ? idv[jb] : idv[ja];
-        o.r = c1 ? rv[jb] : rv[ja];
-        const int j = c1 ? jb : ja;
-        o.st = base + j;
-        o.xm = li > 0 ? base + j - 64 : base + j + 64;
-        o.xp = li < 7 ? base + j + 64 : base + j - 64;
         return o;
     };
     // group P: cells 0, 2 (col0 = 0) or 1, 3 (col0 = 1); group Q: the others.  For col0 = 0:
@@ -1348,40 +1360,113 @@ __device__ __forceinline__ void local_sgs4(const Row4Coef<float> &c, const float
     //   Q0 = cell 0: z- partner's cell 3 (= its P1), z+ cell 1 (P0)
     //   Q1 = cell 2: z- cell 1 (P0), z+ cell 3 (P1)
     // P0 and P1 take the swap of Q1 and Q0, Q0 and Q1 the swap of P1 and P0.
-    const SgsCell P0 = cell_of(0, gzp[0], 0.0f, gzm[0], 1, gzm[1], gzp[1], 0.0f);
-    const SgsCell P1 = cell_of(2, gzm[2], gzp[2], 0.0f, 3, 0.0f, gzm[3], gzp[3]);
-    const SgsCell Q0 = cell_of(1, gzm[1], gzp[1], 0.0f, 0, gzp[0], 0.0f, gzm[0]);
-    const SgsCell Q1 = cell_of(3, 0.0f, gzm[3], gzp[3], 2, gzm[2], gzp[2], 0.0f);
+    return SgsCells{cell_of(0, gzp[0], 0.0f, gzm[0], 1, gzm[1], gzp[1], 0.0f),
+                    cell_of(2, gzm[2], gzp[2], 0.0f, 3, 0.0f, gzm[3], gzp[3]),
+                    cell_of(1, gzm[1], gzp[1], 0.0f, 0, gzp[0], 0.0f, gzm[0]),
+                    cell_of(3, 0.0f, gzm[3], gzp[3], 2, gzm[2], gzp[2], 0.0f)};
+}
+
+// M_b r (K sweeps from zero).  lds: SGS_PAIRS pairs per group.  Every lane of the workgroup must call it
+// (barriers, DPP).
+constexpr int SGS_PAIRS = ROW4_THREADS + 1, SGS_LDS = 4 * SGS_PAIRS;  // (in floats)
+template <int K>
+__device__ __forceinline__ SgsRow sgs_sweeps(const SgsCells &C, const SgsRow &r, float2 *lds, int q) {
+    const int qm = q >= 16 ? q - 16 : ROW4_THREADS, qp = q < ROW4_THREADS - 16 ? q + 16 : ROW4_THREADS;
+    float2 *const lp = lds, *const lq = lds + SGS_PAIRS;
     // the first half-sweep, from zero: no neighbour values yet
-    float p0 = P0.id * P0.r, p1 = P1.id * P1.r, q0 = 0.0f, q1 = 0.0f;
-    lds[P0.st] = p0;
-    lds[P1.st] = p1;
+    SgsRow e{C.P0.id * r.p0, C.P1.id * r.p1, 0.0f, 0.0f};
+    lp[q] = make_float2(e.p0, e.p1);
+    if (q == 0) lp[ROW4_THREADS] = lq[ROW4_THREADS] = make_float2(0.0f, 0.0f);
     __syncthreads();
 #pragma unroll
     for (int s = 1; s <= 2 * K; ++s) {
         if (s & 1) {
-            const float ym0 = sgs_dpp<DPP_ROW_SHR2>(p0), yp0 = sgs_dpp<DPP_ROW_SHL2>(p0);
-            const float ym1 = sgs_dpp<DPP_ROW_SHR2>(p1), yp1 = sgs_dpp<DPP_ROW_SHL2>(p1);
-            const float sw0 = sgs_dpp<DPP_SWAP_PAIRS>(p0), sw1 = sgs_dpp<DPP_SWAP_PAIRS>(p1);
-            q0 = sgs_update(Q0, lds, ym0, yp0, p0, p1, sw1);
-            q1 = sgs_update(Q1, lds, ym1, yp1, p0, p1, sw0);
-            lds[Q0.st] = q0;
-            lds[Q1.st] = q1;
+            float a = r.q0, b = r.q1;
+            sgs_pair(C.Q0, C.Q1, a, b, lp[qm], lp[qp], e.p0, e.p1);
+            e.q0 = C.Q0.id * a;
+            e.q1 = C.Q1.id * b;
+            if (s < 2 * K) lq[q] = make_float2(e.q0, e.q1);
         } else {
-            const float ym0 = sgs_dpp<DPP_ROW_SHR2>(q0), yp0 = sgs_dpp<DPP_ROW_SHL2>(q0);
-            const float ym1 = sgs_dpp<DPP_ROW_SHR2>(q1), yp1 = sgs_dpp<DPP_ROW_SHL2>(q1);
-            const float sw0 = sgs_dpp<DPP_SWAP_PAIRS>(q0), sw1 = sgs_dpp<DPP_SWAP_PAIRS>(q1);
-            p0 = sgs_update(P0, lds, ym0, yp0, q0, q1, sw1);
-            p1 = sgs_update(P1, lds, ym1, yp1, q0, q1, sw0);
-            lds[P0.st] = p0;
-            lds[P1.st] = p1;
+            float a = r.p0, b = r.p1;
+            sgs_pair(C.P0, C.P1, a, b, lq[qm], lq[qp], e.q0, e.q1);
+            e.p0 = C.P0.id * a;
+            e.p1 = C.P1.id * b;
+            if (s < 2 * K) lp[q] = make_float2(e.p0, e.p1);
+        }
+        if (s < 2 * K) __syncthreads();
+    }
+    return e;
+}
+
+// The sum of a cell's couplings times its neighbours in the order x-, x+, y-, y+, z-, z+ of the
+// residual (offdiag_sum) and of local_sgs1.  Which of the z weights is the lower and which the upper
+// coupling depends on the cell and col0 (sgs_cells): v0, v1 are the other group's cells of the lane,
+// end the cell across the row's end (of the pair's lane or of the next brick) and ce its coupling.
+enum SgsPlace { AT_P0, AT_P1, AT_Q0, AT_Q1 };
+template <SgsPlace AT>
+__device__ __forceinline__ float sgs_ordered(const SgsCell &c, bool c1, float xm, float xp, float ym, float yp, float v0,
+                                             float v1, float end, float ce) {
+    float cm, cp, zm, zp;
+    if (AT == AT_P0 || AT == AT_Q0) {
+        const bool inner = AT == AT_P0 ? c1 : !c1;  // cell 1, else cell 0 (the row's lower end)
+        cm = inner ? c.za : ce;
+        zm = inner ? v0 : end;
+        cp = inner ? c.zb : c.za;
+        zp = inner ? v1 : v0;
+    } else {
+        const bool inner = AT == AT_P1 ? !c1 : c1;  // cell 2, else cell 3 (the row's upper end)
+        cm = inner ? c.za : c.zb;
+        zm = inner ? v0 : v1;
+        cp = inner ? c.zb : ce;
+        zp = inner ? v1 : end;
+    }
+    return c.ax_m * xm + c.ax_p * xp + c.ay_m * ym + c.ay_p * yp + cm * zm + cp * zp;
+}
+
+// local_sgs1's sweeps (its operations in its order) on a lane's row by group.
+template <int K>
+__device__ __forceinline__ SgsRow sgs_sweeps_ordered(const SgsCells &C, const SgsRow &r, float2 *lds, int q, bool c1) {
+    const int qm = q >= 16 ? q - 16 : ROW4_THREADS, qp = q < ROW4_THREADS - 16 ? q + 16 : ROW4_THREADS;
+    float2 *const lp = lds, *const lq = lds + SGS_PAIRS;
+    SgsRow e{C.P0.id * r.p0, C.P1.id * r.p1, 0.0f, 0.0f};
+    lp[q] = make_float2(e.p0, e.p1);
+    if (q == 0) lp[ROW4_THREADS] = lq[ROW4_THREADS] = make_float2(0.0f, 0.0f);
+    __syncthreads();
+#pragma unroll 1
+    for (int s = 0; s < K; ++s) {
+        {
+            const float2 xm = lp[qm], xp = lp[qp];
+            const float n0 = sgs_ordered<AT_Q0>(C.Q0, c1, xm.x, xp.x, sgs_dpp<DPP_ROW_SHR2>(e.p0), sgs_dpp<DPP_ROW_SHL2>(e.p0),
+                                                e.p0, e.p1, sgs_dpp<DPP_SWAP_PAIRS>(e.p1), C.Q0.zs);
+            const float n1 = sgs_ordered<AT_Q1>(C.Q1, c1, xm.y, xp.y, sgs_dpp<DPP_ROW_SHR2>(e.p1), sgs_dpp<DPP_ROW_SHL2>(e.p1),
+                                                e.p0, e.p1, sgs_dpp<DPP_SWAP_PAIRS>(e.p0), C.Q1.zs);
+            e.q0 = C.Q0.id * (r.q0 + n0);
+            e.q1 = C.Q1.id * (r.q1 + n1);
+            lq[q] = make_float2(e.q0, e.q1);
+        }
+        __syncthreads();
+        {
+            const float2 xm = lq[qm], xp = lq[qp];
+            const float n0 = sgs_ordered<AT_P0>(C.P0, c1, xm.x, xp.x, sgs_dpp<DPP_ROW_SHR2>(e.q0), sgs_dpp<DPP_ROW_SHL2>(e.q0),
+                                                e.q0, e.q1, sgs_dpp<DPP_SWAP_PAIRS>(e.q1), C.P0.zs);
+            const float n1 = sgs_ordered<AT_P1>(C.P1, c1, xm.y, xp.y, sgs_dpp<DPP_ROW_SHR2>(e.q1), sgs_dpp<DPP_ROW_SHL2>(e.q1),
+                                                e.q0, e.q1, sgs_dpp<DPP_SWAP_PAIRS>(e.q0), C.P1.zs);
+            e.p0 = C.P0.id * (r.p0 + n0);
+            e.p1 = C.P1.id * (r.p1 + n1);
+            lp[q] = make_float2(e.p0, e.p1);
         }
         __syncthreads();
     }
-    e[0] = c1 ? q0 : p0;
-    e[1] = c1 ? p0 : q0;
-    e[2] = c1 ? q1 : p1;
-    e[3] = c1 ? p1 : q1;
+    return e;
+}
+
+// e = M_b r on rows.  lds: SGS_LDS floats (8-byte aligned).
+template <int K>
+__device__ __forceinline__ void local_sgs4(const Row4Coef<float> &c, const float id[4], const float r[4], float e[4],
+                                           float *lds, int q) {
+    const SgsCells C = sgs_cells(c, id, q);
+    const bool c1 = sgs_col1(q);
+    sgs_ungroup(sgs_sweeps<K>(C, sgs_group(r, c1), reinterpret_cast<float2 *>(lds), q), c1, e);
 }
 
 // Pre-smoothing from zero on the finest level: z = M_b rhs (one brick per 128-thread workgroup), K
@@ -1391,7 +1476,7 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_pre_local4(LevelDesc L, OpDesc
                                                              const float *__restrict__ idiag,
                                                              const float *__restrict__ rhs, float *__restrict__ z,
                                                              Gate Q) {
-    __shared__ float lds[BRICK_CELLS];
+    __shared__ __align__(16) float lds[SGS_LDS];
     const int br = brick_or_idle(L);
     if (br < 0) return;
     const BrickMeta m = L.meta[br];
@@ -1403,11 +1488,11 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_pre_local4(LevelDesc L, OpDesc
     Row4Coef<float> c;
     if (m.flags & BM_UNIFORM) {
         const UniT<float> u = uni_load<float>(L, br);
-        c = row4_local_uniform(u.g, q);
+        c = row4_uniform(u.g);
 #pragma unroll
         for (int j = 0; j < 4; ++j) id[j] = u.id;
     } else {
-        c = row4_local(row4_coef(A, N), q);
+        c = row4_coef(A, N);
         unpack4(ld4(idiag, N.c), id);
     }
     local_sgs4<K>(c, id, r, e, lds, q);
@@ -1424,7 +1509,7 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_post_local4(LevelDesc L, OpDes
                                                               const float *__restrict__ rhs,
                                                               const float *__restrict__ zin, float *__restrict__ zout,
                                                               Gate Q, RedBuf R) {
-    __shared__ float lds[BRICK_CELLS];
+    __shared__ __align__(16) float lds[SGS_LDS];
     __shared__ double red[2];
     const int br = brick_or_idle(L);
     if (br < 0) return;
@@ -1448,7 +1533,7 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_post_local4(LevelDesc L, OpDes
             id[j] = u.id;
             unk[j] = true;
         }
-        c = row4_local_uniform(u.g, q);
+        c = row4_uniform(u.g);
     } else {
         const Row4Coef<float> g = row4_coef(A, N);
         float dir[4];
@@ -1462,7 +1547,7 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_post_local4(LevelDesc L, OpDes
             unk[j] = dir[j] >= 0;
             res[j] = unk[j] ? r[j] - (diag * v.c[j] - off) : 0.0f;
         }
-        c = row4_local(g, q);
+        c = g;
     }
     local_sgs4<K>(c, id, res, e, lds, q);
     float out[4];
@@ -1728,10 +1813,10 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_cg_update4(LevelDesc L, double
             const UniT<float> u = uni_load<float>(L, br);
 #pragma unroll
             for (int j = 0; j < 4; ++j) id[j] = u.id;
-            if (ZFIRST == 2) cf = row4_local_uniform(u.g, threadIdx.x);
+            if (ZFIRST == 2) cf = row4_uniform(u.g);
         } else {
             unpack4(ld4(idiag, c), id);
-            if (ZFIRST == 2) cf = row4_local(row4_coef(A32, row4_nbrs(m, br, threadIdx.x)), threadIdx.x);
+            if (ZFIRST == 2) cf = row4_coef(A32, row4_nbrs(m, br, threadIdx.x));
         }
     }
     const SolveScalars &Sg = S[g];
@@ -1756,7 +1841,7 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_cg_update4(LevelDesc L, double
     }
     if (ZFIRST == 2 && !(m.flags & BM_COARSEST)) {
         // the brick-local smoother's pre-smoothing from zero (k_pre_local4) on the updated residual
-        __shared__ float zl[BRICK_CELLS];
+        __shared__ __align__(16) float zl[SGS_LDS];
         float e[4];
         local_sgs4<K>(cf, id, rv, e, zl, threadIdx.x);
         *reinterpret_cast<float4 *>(z + c) = make_float4(e[0], e[1], e[2], e[3]);
@@ -1910,7 +1995,7 @@ __global__ __launch_bounds__(BLOCK) void k_restrict_pre(LevelDesc Lc, OpDesc<flo
     const float dirc = Ac.dir[c];
     const int cid = t < 64 ? Lc.child64[64 * br + t] : -1;
     const BrickMeta m = Lc.meta[br];
-    if (all_done(Q) || grid_done(Q, Lc, m)) return;
+    if (all_done(Q) || grid_done(Q, Lc, m) || (m.flags & Q.skip & BM_BELOW)) return;
     if (t < 64) bid[t] = cid;
     __syncthreads();
     constexpr int NQ = (E * E * E + BLOCK - 1) / BLOCK;
@@ -2403,6 +2488,33 @@ __global__ __launch_bounds__(BRICK_CELLS) void k_coarse_components(LevelDesc L, 
     code[c] = !unk ? (int16_t)-1 : (hasd[lab[e]] ? (int16_t)-2 : (int16_t)lab[e]);
 }
 
+// Sums and sizes of the components of one brick in LDS, one entry per root cell.  The values are added
+// as integers, scaled so that the largest has 53 bits: integer sums do not depend on the order of the
+// atomic adds, 512 of them fit 64 bits, and the scaling loses at most 2^-54 of the largest value per
+// term, no more than a sum in FP64 does.  (One thread adding a component of the whole brick in cell
+// order took 35 us of the 47 us coarse solve of an all-fluid box; this takes about 1 us.)
+struct ComponentSums {
+    unsigned long long s[BRICK_CELLS];
+    int n[BRICK_CELLS];
+    __device__ __forceinline__ void clear(int e) {
+        s[e] = 0;
+        n[e] = 0;
+    }
+    __device__ __forceinline__ static int shift(double mx) {
+        int ex = 0;
+        (void)frexp(mx, &ex);
+        return 53 - ex;
+    }
+    __device__ __forceinline__ void add(int root, double v, int sh) {
+        if (root < 0) return;
+        atomicAdd(&s[root], (unsigned long long)(long long)rint(ldexp(v, sh)));
+        atomicAdd(&n[root], 1);
+    }
+    __device__ __forceinline__ double mean(int root, int sh) const {
+        return ldexp((double)(long long)s[root], -sh) / n[root];
+    }
+};
+
 // Coarse solve of every grid whose last level L is (one brick): block g handles grid g with
 // `sweeps` damped-Jacobi sweeps from zero, in LDS.  DOT (finest level only): also the r.z partial
 // of the grid's brick, as k_jacobi<..., DOT> stores it for grids with coarser levels.  CPT cells per
@@ -2417,6 +2529,7 @@ __global__ __launch_bounds__(BRICK_CELLS / CPT) void k_coarse_solve(LevelDesc L,
     __shared__ T zs[2][BRICK_CELLS];
     __shared__ double lds[32];
     __shared__ int16_t cc[BRICK_CELLS];
+    __shared__ ComponentSums sums;
     if (all_done(Q)) return;
     const int g = blockIdx.x;
     const GridLevel G = L.gl[g];
@@ -2453,31 +2566,19 @@ __global__ __launch_bounds__(BRICK_CELLS / CPT) void k_coarse_solve(LevelDesc L,
 #pragma unroll
     for (int u = 0; u < CPT; ++u) rs[u] = r[u];
     if (__syncthreads_or(sing)) {
-#pragma unroll
-        for (int u = 0; u < CPT; ++u) zs[0][t + u * NT] = r[u];
-        __syncthreads();
-        // the root of each singular component sums it in cell order and stores its mean
+        double mx = 0.0;
 #pragma unroll
         for (int u = 0; u < CPT; ++u) {
-            const int e = t + u * NT;
-            if (cc[e] == e) {
-                double sum = 0.0;
-                int cnt = 0;
-                for (int k = e; k < BRICK_CELLS; ++k)
-                    if (cc[k] == e) {
-                        sum += (double)zs[0][k];
-                        ++cnt;
-                    }
-                zs[1][e] = (T)(sum / cnt);
-            }
+            if (cc[t + u * NT] >= 0) mx = fmax(mx, fabs((double)r[u]));
+            sums.clear(t + u * NT);
         }
+        const int sh = ComponentSums::shift(block_max(mx, lds));  // its barriers follow the clearing
+#pragma unroll
+        for (int u = 0; u < CPT; ++u) sums.add(cc[t + u * NT], (double)r[u], sh);
         __syncthreads();
 #pragma unroll
-        for (int u = 0; u < CPT; ++u) {
-            const int e = t + u * NT;
-            if (cc[e] >= 0) rs[u] = r[u] - zs[1][cc[e]];
-        }
-        __syncthreads();
+        for (int u = 0; u < CPT; ++u)
+            if (cc[t + u * NT] >= 0) rs[u] = r[u] - (T)sums.mean(cc[t + u * NT], sh);
     }
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
@@ -2518,6 +2619,413 @@ __global__ __launch_bounds__(BRICK_CELLS / CPT) void k_coarse_solve(LevelDesc L,
     if (DOT) {
         part = block_sum(part, lds);
         store_partials(R, G.brick_start, part, 0.0);
+    }
+}
+
+// The bottom of the V-cycle (BottomGrid) of one grid in one 1024-thread workgroup: from the first
+// level of at most 8 stored bricks, whose right-hand side and pre-smoothing from zero the restriction
+// has written, down to the coarsest brick and back up.  128 threads per brick hold its cells as rows of
+// four (Row4), with the operator in registers and the vectors that neighbours read in LDS.
+//
+// These levels are a few thousand cells: each launch on them costs its boundary and two to three
+// dependent trips to memory (another XCD wrote the data), 3 to 5 us for well under 1 us of work, and
+// the coarsest brick's sweeps a barrier of eight wavefronts each.  In one workgroup only the first
+// loads go to memory.  Measured per V-cycle on the last two levels of a 32^3 grid (V(1,1), 48 sweeps on
+// the coarsest brick): 26 us in five launches, 17 us here, of which 8 us are those sweeps; of a 256^3
+// grid (V(2,2), 4 sweeps): 35 us in eight launches, 17 us here.  Eight bricks fill the 1024 threads with one brick each; a level of 16 or more
+// would make the one CU's issue the bound (about 2 us of it per smoothing step and 8 bricks, as long
+// as the launch it saves).
+// Every value is formed by the operations of the kernels for larger levels in their order
+// (k_post_local4, k_residual4, k_restrict_pre, k_prolong4, k_coarse_solve; the restriction's nested
+// sums one axis at a time), so both forms give the same bits.
+constexpr int BOTTOM_THREADS = BOTTOM_BRICKS * ROW4_THREADS;
+
+// Damped-Jacobi sweeps from zero on the coarsest brick (k_coarse_solve's operations in its order), two
+// cells (z[0], z[1]) per lane of the first four wavefronts; every thread of the workgroup calls it
+// (barriers).  A 16-lane DPP row holds the eight y rows of one x and one half of z: lane bits kqlo, lj
+// (3), kqhi, li (3), cells 4 kqhi + 2 kqlo and the next.  So the y neighbours are two lanes away in the
+// DPP row, one z neighbour is the lane's other cell, the other the pair's or, across the halves, through
+// LDS (zb: 2 x 512 floats), as the x neighbours are.  One wavefront per SIMD: with four cells per lane of
+// two wavefronts a sweep took 500 cycles, its 76 instructions issued one after the other.
+struct BottomCells {
+    float xm, xp, ym, yp, zm, zp;  // couplings
+    float diag, inv, rs;
+};
+__device__ __forceinline__ void bottom_solve(const BottomCells (&c)[2], float z[2], float *zb, int sweeps, bool mine,
+                                             int base, int kqlo) {
+    if (mine) {
+        z[0] = c[0].inv * c[0].rs;
+        z[1] = c[1].inv * c[1].rs;
+        *reinterpret_cast<float2 *>(zb + base) = make_float2(z[0], z[1]);
+    }
+    __syncthreads();
+    if (!mine) {  // the other wavefronts only keep the barriers
+        for (int s = 1; s < sweeps; ++s) __syncthreads();
+        return;
+    }
+    // (a coupling is 0 across the brick's faces; its value is then the cell's own)
+    const int ixm = base >= 64 ? base - 64 : base, ixp = base < 448 ? base + 64 : base;
+    const int iz = kqlo ? ((base & 7) < 6 ? base + 2 : base) : ((base & 7) ? base - 1 : base);
+    for (int s = 1; s < sweeps; ++s) {
+        const float *zc = zb + ((s & 1) ? 0 : BRICK_CELLS);
+        float *zn = zb + ((s & 1) ? BRICK_CELLS : 0);
+        const float2 xm = *reinterpret_cast<const float2 *>(zc + ixm), xp = *reinterpret_cast<const float2 *>(zc + ixp);
+        const float far = zc[iz];
+        const float sw0 = sgs_dpp<DPP_SWAP_PAIRS>(z[0]), sw1 = sgs_dpp<DPP_SWAP_PAIRS>(z[1]);
+        float ym[2], yp[2], d[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            ym[j] = c[j].ym * sgs_dpp<DPP_ROW_SHR2>(z[j]);
+            yp[j] = c[j].yp * sgs_dpp<DPP_ROW_SHL2>(z[j]);
+            d[j] = c[j].diag * z[j];
+        }
+        const float zp0 = c[0].zp * z[1], zm1 = c[1].zm * z[0];
+        __builtin_amdgcn_sched_barrier(0);  // the products of registers cover the LDS reads
+        const float zm0 = c[0].zm * (kqlo ? sw1 : far), zp1 = c[1].zp * (kqlo ? far : sw0);
+        const float off0 = c[0].xm * xm.x + c[0].xp * xp.x + ym[0] + yp[0] + zm0 + zp0;
+        const float off1 = c[1].xm * xm.y + c[1].xp * xp.y + ym[1] + yp[1] + zm1 + zp1;
+        z[0] = z[0] + c[0].inv * (c[0].rs - (d[0] - off0));
+        z[1] = z[1] + c[1].inv * (c[1].rs - (d[1] - off1));
+        *reinterpret_cast<float2 *>(zn + base) = make_float2(z[0], z[1]);
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(BOTTOM_THREADS) void k_bottom(const BottomGrid *__restrict__ grids, int pre, int post,
+                                                           int sweeps, float omega, int slot, Gate Q) {
+    constexpr int E = 18, NC = BOTTOM_BRICKS * BRICK_CELLS;
+    __shared__ __align__(16) float zl[NC];  // z of the level in hand
+    __shared__ __align__(16) float ex[BOTTOM_BRICKS * SGS_LDS];  // the smoother's exchange; the residual that is restricted
+    __shared__ __align__(16) float rc[NC];  // the next level's right-hand side, then its z
+    __shared__ __align__(16) float t1[E * E * 8];  // the restriction's partial sums along z (and the coarse sweeps'
+    __shared__ float t2[E * 8 * 8];    // buffers), then along y
+    __shared__ __align__(16) float cop[4][BRICK_CELLS];  // the coarsest brick's gx, gy, gz, dir
+    __shared__ __align__(16) int cid[64 * BOTTOM_BRICKS];  // child64 and parent8 of the level in hand
+    __shared__ __align__(16) int pb[BOTTOM_BRICKS][8];
+    __shared__ int16_t code[BRICK_CELLS];
+    __shared__ int any[4];
+    __shared__ double red[32];
+    __shared__ ComponentSums sums;
+    const BottomGrid &G = grids[blockIdx.x];
+    const int n = G.n;
+    if (n == 0 || all_done(Q) || (Q.S && Q.S[blockIdx.x].done)) return;
+    const int t = threadIdx.x, q = t % ROW4_THREADS;
+    const int own = __builtin_amdgcn_readfirstlane(t / ROW4_THREADS);  // (a wavefront works on one brick)
+    const int li = q >> 4, lj = (q >> 1) & 7, h = q & 1;
+
+    // the coarsest brick's operator, kept in LDS
+    if (own < 4) {
+        const BottomLevel &L = G.lev[n - 1];
+        const float *const from[4] = {L.gx, L.gy, L.gz, L.dir};
+        *reinterpret_cast<float4 *>(&cop[own][4 * q]) = ld4(from[own], 4 * q);
+    }
+    if (t >= BOTTOM_THREADS - BRICK_CELLS) code[t - (BOTTOM_THREADS - BRICK_CELLS)] = G.code[t - (BOTTOM_THREADS - BRICK_CELLS)];
+
+    // The level in hand: the thread's four cells by colour group (SgsRow) with all of their couplings, so
+    // that neither the sweeps nor the residual select or reload anything.  Neighbour bricks count from
+    // the grid's first brick of the level.  The wavefronts of bricks the level does not have keep zeros
+    // and the barriers.
+    const bool c1 = sgs_col1(q);
+    const int me = own * ROW4_THREADS + q;
+    SgsCells A{};
+    SgsRow diag{}, ez{};  // diagonal; couplings across the brick's z faces
+    SgsRow r{}, z{};
+    int ixm = me, ixp = me, iym = me, iyp = me, iz = 4 * me;  // the rows beside the thread's, the cell across z
+    int unk = 0;                        // bit j: the row's cell j is an unknown
+    bool work = false;
+    int parity = 0;  // of the brick's position (x, y, z)
+    auto load = [&](const BottomLevel &L, const BottomLevel &C) {
+        work = own < L.nb;
+        A = SgsCells{};
+        diag = ez = r = z = SgsRow{};
+        ixm = ixp = iym = iyp = me;
+        iz = 4 * me;
+        // every load of the level at once, its tables included; the operator's rows to LDS
+        const int nc = C.nb;
+        const int id64 = t < 64 * nc ? C.child64[t] : -1, id8 = t < 8 * L.nb ? L.parent8[t] : -1;
+        BrickMeta m{};
+        float own_gz[4] = {0.0f, 0.0f, 0.0f, 0.0f}, own_dir[4] = {0.0f, 0.0f, 0.0f, 0.0f}, own_id[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (work) {
+            m = L.meta[own];
+            parity = (L.bxyz[3 * own] & 1) << 2 | (L.bxyz[3 * own + 1] & 1) << 1 | (L.bxyz[3 * own + 2] & 1);
+            const float4 gx0 = ld4(L.gx, 4 * me), gy0 = ld4(L.gy, 4 * me);
+            load4(L.gz, 4 * me, own_gz);
+            load4(L.dir, 4 * me, own_dir);
+            load4(L.idiag, 4 * me, own_id);
+            reinterpret_cast<float4 *>(zl)[me] = gx0;
+            reinterpret_cast<float4 *>(ex)[me] = gy0;
+            t1[me] = own_gz[0];
+        }
+        if (t < 64 * nc) cid[t] = id64 >= 0 ? id64 - L.brick_start : -1;
+        if (t < 8 * L.nb) pb[t >> 3][t & 7] = id8 >= 0 ? id8 - C.brick_start : -1;
+        __syncthreads();
+        if (!work) return;
+#pragma unroll
+        for (int d = 0; d < 6; ++d) m.nbr[d] = m.nbr[d] >= 0 ? m.nbr[d] - L.brick_start : -1;
+        float dg[4], gz[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        // the high couplings are the next cells' low ones, in rows of other threads
+        Row4Coef<float> g;
+        const float4 *lx = reinterpret_cast<const float4 *>(zl), *ly = reinterpret_cast<const float4 *>(ex);
+        unpack4(lx[me], g.gxm);
+        unpack4(ly[me], g.gym);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) g.gzm[j] = own_gz[j];
+        // the rows beside the thread's, in the brick or across its faces; where no brick is stored the
+        // coupling is 0, and the row the thread's own
+        const int jxp = li < 7 ? me + 16 : m.nbr[NB_XP] >= 0 ? m.nbr[NB_XP] * ROW4_THREADS + q - 112 : -1;
+        const int jyp = lj < 7 ? me + 2 : m.nbr[NB_YP] >= 0 ? m.nbr[NB_YP] * ROW4_THREADS + q - 14 : -1;
+        const int jz = !h ? me + 1 : m.nbr[NB_ZP] >= 0 ? m.nbr[NB_ZP] * ROW4_THREADS + q - 1 : -1;
+        unpack4(jxp >= 0 ? lx[jxp] : make_float4(0.0f, 0.0f, 0.0f, 0.0f), g.gxp);
+        unpack4(jyp >= 0 ? ly[jyp] : make_float4(0.0f, 0.0f, 0.0f, 0.0f), g.gyp);
+        if (jxp >= 0) ixp = jxp;
+        if (jyp >= 0) iyp = jyp;
+        if (li > 0) ixm = me - 16;
+        else if (m.nbr[NB_XM] >= 0) ixm = m.nbr[NB_XM] * ROW4_THREADS + q + 112;
+        if (lj > 0) iym = me - 2;
+        else if (m.nbr[NB_YM] >= 0) iym = m.nbr[NB_YM] * ROW4_THREADS + q + 14;
+        g.gzp[0] = g.gzm[1];
+        g.gzp[1] = g.gzm[2];
+        g.gzp[2] = g.gzm[3];
+        g.gzp[3] = jz >= 0 ? t1[jz] : 0.0f;
+        unk = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            dg[j] = own_dir[j] >= 0 ? own_dir[j] + ((g.gxm[j] + g.gxp[j]) + (g.gym[j] + g.gyp[j]) + (g.gzm[j] + g.gzp[j]))
+                                    : 0.0f;
+            unk |= own_dir[j] >= 0 ? 1 << j : 0;
+        }
+        A = sgs_cells(g, own_id, q);
+        diag = sgs_group(dg, c1);
+        // across z the row's col0 is the same (across x and y the other one)
+        const int nz = h ? m.nbr[NB_ZP] : m.nbr[NB_ZM];
+        if (h) gz[3] = g.gzp[3];
+        else gz[0] = g.gzm[0];
+        ez = sgs_group(gz, c1);
+        if (nz >= 0) iz = 4 * (nz * ROW4_THREADS + (q ^ 1)) + (h ? (c1 ? 2 : 0) : (c1 ? 1 : 3));
+    };
+    // rhs - A z of the thread's cells; zl: z by row and group
+    auto residual = [&]() {
+        const float4 *zr = reinterpret_cast<const float4 *>(zl);
+        const float4 xm = zr[ixm], xp = zr[ixp], ym = zr[iym], yp = zr[iyp];
+        const float fz = zl[iz];
+        const float sp0 = sgs_dpp<DPP_SWAP_PAIRS>(z.p0), sp1 = sgs_dpp<DPP_SWAP_PAIRS>(z.p1);
+        const float sq0 = sgs_dpp<DPP_SWAP_PAIRS>(z.q0), sq1 = sgs_dpp<DPP_SWAP_PAIRS>(z.q1);
+        // across the row's lower end (h = 0) or upper end (h = 1) lies the next brick, else the pair's lane
+        const float lo0 = h ? sp1 : fz, hi0 = h ? fz : sp0, lo1 = h ? sq1 : fz, hi1 = h ? fz : sq0;
+        SgsRow o;
+        o.p0 = r.p0 - (diag.p0 * z.p0 - sgs_ordered<AT_P0>(A.P0, c1, xm.z, xp.z, ym.z, yp.z, z.q0, z.q1, lo1, A.P0.zs + ez.p0));
+        o.p1 = r.p1 - (diag.p1 * z.p1 - sgs_ordered<AT_P1>(A.P1, c1, xm.w, xp.w, ym.w, yp.w, z.q0, z.q1, hi1, A.P1.zs + ez.p1));
+        o.q0 = r.q0 - (diag.q0 * z.q0 - sgs_ordered<AT_Q0>(A.Q0, c1, xm.x, xp.x, ym.x, yp.x, z.p0, z.p1, lo0, A.Q0.zs + ez.q0));
+        o.q1 = r.q1 - (diag.q1 * z.q1 - sgs_ordered<AT_Q1>(A.Q1, c1, xm.y, xp.y, ym.y, yp.y, z.p0, z.p1, hi0, A.Q1.zs + ez.q1));
+        return o;
+    };
+    auto publish = [&]() {
+        reinterpret_cast<float4 *>(zl)[me] = make_float4(z.p0, z.p1, z.q0, z.q1);
+        __syncthreads();
+    };
+    float2 *const exq = reinterpret_cast<float2 *>(ex) + own * 2 * SGS_PAIRS;
+    // z += M_b (rhs - A z)
+    auto smooth = [&]() {
+        const SgsRow e = sgs_sweeps<LOCAL_SGS_SWEEPS_COARSE>(A, residual(), exq, q);
+        z = SgsRow{z.p0 + e.p0, z.p1 + e.p1, z.q0 + e.q0, z.q1 + e.q1};
+        publish();  // (every read of zl lies before the sweeps' barriers)
+    };
+    auto take = [&](const float *from) {  // the thread's row, by group
+        float v[4];
+        load4(from, (long)4 * me, v);
+        return sgs_group(v, c1);
+    };
+    auto give = [&](float *to, const SgsRow &g) {
+        float v[4];
+        sgs_ungroup(g, c1, v);
+        store4(to, (long)4 * me, v);
+    };
+
+    for (int d = 0; d + 1 < n; ++d) {
+        const BottomLevel &L = G.lev[d], &C = G.lev[d + 1];
+        load(L, C);
+        if (work) {
+            if (d == 0) {
+                r = take(L.rhs);
+                z = take(L.z);
+            } else {
+                float v[4];
+                load4((const float *)rc, (long)4 * me, v);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = (unk >> j) & 1 ? v[j] : 0.0f;
+                r = sgs_group(v, c1);
+            }
+        }
+        __syncthreads();  // the operator's rows in zl and ex have been read
+        if (d > 0) z = sgs_sweeps_ordered<LOCAL_SGS_SWEEPS_COARSE>(A, r, exq, q, c1);  // from zero, as k_restrict_pre
+        publish();
+        for (int s = 1; s < pre; ++s) smooth();
+        give(ex, residual());
+        if (work && d + 2 < n) {  // for the way up (this thread reads them back)
+            give(L.z, z);
+            if (d > 0) give(L.rhs, r);
+        }
+        __syncthreads();
+        // k_restrict_pre's sums, one coarse brick after another.  Along z first: thread e forms the eight
+        // sums of the tile's row (a, b), from the two whole rows of fine bricks in it and a cell at each end.
+        const bool flat = L.flat;
+        const float w0 = 0.25f, w1 = 0.75f;
+        for (int B = 0; B < C.nb; ++B) {
+            if (t < E * E) {
+                const int b = t % E, a = t / E;
+                const int rowcell = (((a + 7) & 7) * 8 + ((b + 7) & 7)) * 8;
+                const int4 id = reinterpret_cast<const int4 *>(cid + 64 * B)[((a + 7) >> 3) * 4 + ((b + 7) >> 3)];
+                const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                auto row = [&](int brick, int half) {
+                    return brick >= 0 ? *reinterpret_cast<const float4 *>(&ex[brick * BRICK_CELLS + rowcell + 4 * half]) : zero;
+                };
+                float v[E];
+                v[0] = id.x >= 0 ? ex[id.x * BRICK_CELLS + rowcell + 7] : 0.0f;
+                unpack4(row(id.y, 0), v + 1);
+                unpack4(row(id.y, 1), v + 5);
+                unpack4(row(id.z, 0), v + 9);
+                unpack4(row(id.z, 1), v + 13);
+                v[17] = id.w >= 0 ? ex[id.w * BRICK_CELLS + rowcell] : 0.0f;
+                float o[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const float *u = v + 2 * k;
+                    o[k] = flat ? 0.0f * u[0] + 1.0f * u[1] + 0.0f * u[2] + 0.0f * u[3]
+                                : w0 * u[0] + w1 * u[1] + w1 * u[2] + w0 * u[3];
+                }
+                store4(t1, 8 * t, o);
+                store4(t1, 8 * t + 4, o + 4);
+            }
+            __syncthreads();
+            for (int e = t; e < E * 64; e += BOTTOM_THREADS) {
+                const int k = e & 7, j = (e >> 3) & 7, a = e >> 6;
+                const float *row = &t1[(a * E + 2 * j) * 8 + k];
+                float acc = 0.0f;
+                acc += w0 * row[0];
+                acc += w1 * row[8];
+                acc += w1 * row[16];
+                acc += w0 * row[24];
+                t2[e] = acc;
+            }
+            __syncthreads();
+            if (t < BRICK_CELLS) {
+                const float *row = &t2[(2 * (t >> 6)) * 64 + (t & 63)];
+                float acc = 0.0f;
+                acc += w0 * row[0];
+                acc += w1 * row[64];
+                acc += w1 * row[128];
+                acc += w0 * row[192];
+                rc[B * BRICK_CELLS + t] = acc;
+            }
+        }
+        __syncthreads();
+    }
+
+    // the coarsest brick: k_coarse_solve
+    {
+        const BottomLevel &L = G.lev[n - 1];
+        const bool mine = own < 2;
+        const int kqlo = t & 1, base = ((t >> 5) & 7) * 64 + ((t >> 1) & 7) * 8 + ((t >> 4) & 1) * 4 + 2 * kqlo;
+        BottomCells c[2]{};
+        int cc[2] = {-1, -1};
+        float cz[2] = {0.0f, 0.0f};
+        double mx = 0.0;
+        __syncthreads();
+        if (mine) {
+            const float *gx = cop[0], *gy = cop[1], *gz = cop[2], *dir = cop[3];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int e = base + j, ei = e >> 6, ej = (e >> 3) & 7, ek = e & 7;
+                BottomCells &o = c[j];
+                o.xm = gx[e];
+                o.ym = gy[e];
+                o.zm = gz[e];
+                o.xp = ei < 7 ? gx[e + 64] : 0.0f;
+                o.yp = ej < 7 ? gy[e + 8] : 0.0f;
+                o.zp = ek < 7 ? gz[e + 1] : 0.0f;
+                o.diag = dir[e] + ((o.xm + o.xp) + (o.ym + o.yp) + (o.zm + o.zp));
+                o.inv = dir[e] >= 0 && o.diag > 0 ? omega / o.diag : 0.0f;
+                o.rs = n == 1 ? L.rhs[e] : dir[e] >= 0 ? rc[e] : 0.0f;
+                cc[j] = code[e];
+                if (cc[j] >= 0) mx = fmax(mx, fabs((double)o.rs));
+            }
+        }
+        const unsigned long long vote = __ballot(cc[0] >= 0 || cc[1] >= 0);
+        if (mine && (t & 63) == 0) any[t >> 6] = vote != 0;
+        __syncthreads();
+        if (any[0] | any[1] | any[2] | any[3]) {
+            if (t < BRICK_CELLS) sums.clear(t);
+            const int sh = ComponentSums::shift(block_max(mx, red));
+#pragma unroll
+            for (int j = 0; j < 2; ++j) sums.add(cc[j], (double)c[j].rs, sh);
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                if (cc[j] >= 0) c[j].rs = c[j].rs - (float)sums.mean(cc[j], sh);
+        }
+        bottom_solve(c, cz, t1, sweeps, mine, base, kqlo);
+        if (mine) {
+            float *to = n > 1 ? rc : slot && !L.deepest ? L.tmp : L.z;
+            to[base] = cz[0];
+            to[base + 1] = cz[1];
+        }
+        __syncthreads();
+    }
+
+    for (int d = n - 2; d >= 0; --d) {
+        const BottomLevel &L = G.lev[d], &C = G.lev[d + 1];
+        if (d + 2 < n) {
+            load(L, C);
+            if (work) {
+                r = take(L.rhs);
+                z = take(L.z);
+            }
+            __syncthreads();
+        }
+        // k_prolong4's correction from rc
+        if (work) {
+            const int px = parity >> 2, py = (parity >> 1) & 1, pz = parity & 1;
+            const int a0 = (li >> 1) + 1, b0 = (lj >> 1) + 1;
+            const int a1 = (li & 1) ? a0 + 1 : a0 - 1, b1 = (lj & 1) ? b0 + 1 : b0 - 1;
+            // the four coarse values 2h .. 2h + 3 along z of tile row (a, b)
+            auto row = [&](int a, int b, float o[4]) {
+                const int ia = 4 * px + 7 + a, ib = 4 * py + 7 + b;
+                const int rowslot = (((ia >> 3) - px) * 2 + ((ib >> 3) - py)) * 2, rowcell = ((ia & 7) * 8 + (ib & 7)) * 8;
+                const int2 id = *reinterpret_cast<const int2 *>(&pb[own][rowslot]);  // both bricks of the row
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int ic = 4 * pz + 7 + 2 * h + u;
+                    const int b = (ic >> 3) - pz ? id.y : id.x;
+                    o[u] = b >= 0 ? rc[b * BRICK_CELLS + rowcell + (ic & 7)] : 0.0f;
+                }
+            };
+            float c00[4], c01[4], c10[4], c11[4];
+            row(a0, b0, c00);
+            row(a0, b1, c01);
+            row(a1, b0, c10);
+            row(a1, b1, c11);
+            const float nn = 0.75f, f = 0.25f;
+            const float nk = L.flat ? 1.0f : nn, fk = L.flat ? 0.0f : f;
+            float add[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int u0 = (j >> 1) + 1, u1 = (j & 1) ? u0 + 1 : u0 - 1;
+                const float v = nn * (nn * (nk * c00[u0] + fk * c00[u1]) + f * (nk * c01[u0] + fk * c01[u1])) +
+                                f * (nn * (nk * c10[u0] + fk * c10[u1]) + f * (nk * c11[u0] + fk * c11[u1]));
+                add[j] = (unk >> j) & 1 ? v : 0.0f;
+            }
+            const SgsRow a = sgs_group(add, c1);
+            z.p0 += a.p0;
+            z.p1 += a.p1;
+            z.q0 += a.q0;
+            z.q1 += a.q1;
+        }
+        publish();
+        for (int s = 0; s < post; ++s) smooth();
+        if (work) {
+            give(d > 0 ? rc : slot && !L.deepest ? L.tmp : L.z, z);
+        }
+        __syncthreads();
     }
 }
 

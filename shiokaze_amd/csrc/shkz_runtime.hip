@@ -487,7 +487,7 @@ struct shkz_ctx {
     struct Pinned {
         void *p = nullptr;
         size_t cap = 0;
-    } pin_flags, pin_meta0, pin_meta, pin_links, pin_counts;
+    } pin_flags, pin_meta0, pin_meta, pin_links, pin_counts, pin_bottom;
     // timing
     bool timing = false;
     std::vector<std::string> kernel_names;
@@ -508,6 +508,9 @@ struct shkz_ctx {
     // first finest-level sweep fused into the residual update (SHKZ_NO_FUSE=1: separate kernels;
     // the results are the same)
     bool fuse_krylov = true;
+    // each grid's last levels in one workgroup (SHKZ_NO_BOTTOM=1: one launch per level and step, as on
+    // the levels above them; the results are the same)
+    bool use_bottom = true;
     // coarse levels of at most this many stored bricks smooth with multi-sweep launches unless the
     // autotuner picks another limit (SHKZ_MULTI_MAX_BRICKS overrides the default; the results do
     // not depend on it)
@@ -633,6 +636,11 @@ struct Problem {
     double omega = 0.9;
     int multi_max_bricks = 1024;  // coarse levels up to this size smooth with multi-sweep launches
     double eta = 0.0;  // mixed precision: relative defect reduction asked of each inner solve (0: to the tolerance)
+    // mixed precision: the grids' bottoms (device), and the first level every grid's bottom covers
+    const BottomGrid *bottom = nullptr;
+    int bottom_level = 0;
+    // the brick-local V-cycle leaves the bottoms to k_bottom
+    bool with_bottom() const { return bottom && smoother == SHKZ_SMOOTH_BRICK; }
 };
 
 template <class T>
@@ -777,6 +785,9 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
     std::vector<T *> zcur(nl), zoth(nl);
     const T om = (T)P.omega;
     const double es = (double)sizeof(T);
+    const bool bottom = brick_smoother && P.with_bottom();
+    // which of a coarse level's two vectors holds its smoothed z
+    const int bottom_slot = final_slot(P.pre_c, P.post_c, false, false, true);
     // coarse levels small enough smooth with one multi-sweep launch per smoothing step (Jacobi);
     // with the brick-local smoother every level uses it, whatever its size
     std::vector<char> mpre(nl, 0), mpost(nl, 0);
@@ -797,7 +808,17 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
         const bool f = l == 0;
         const int pre = f ? P.pre : P.pre_c, post = f ? P.post : P.post_c;
         const bool last = l == nl - 1;
-        if (L.any_coarsest) {
+        if (bottom && l == P.bottom_level) {
+            // every grid's remaining levels, in one launch
+            if constexpr (sizeof(T) == 4) {
+                const double bytes = 9 * es * (double)L.unknowns;
+                K.go("bottom", -1, 0, bytes, dim3((unsigned)P.ngrids), dim3(BOTTOM_THREADS), k_bottom, P.bottom, P.pre_c,
+                     P.post_c, P.coarse_sweeps, om, bottom_slot, Q);
+            }
+            zcur[l] = bottom_slot && !last ? tmp : z;
+            break;
+        }
+        if (L.any_coarsest && !(bottom && !f)) {
             // grids ending here: their z goes where the other grids' smoothed z ends up
             // (the brick-local smoother swaps as the finest level's Jacobi does on every level)
             T *dst = (last || final_slot(pre, post, mpre[l], mpost[l], f || brick_smoother) == 0) ? z : tmp;
@@ -894,7 +915,7 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
         zcur[l] = cur;
         zoth[l] = oth;
     }
-    for (int l = nl - 2; l >= 0; --l) {
+    for (int l = (bottom ? P.bottom_level : nl - 1) - 1; l >= 0; --l) {
         LevelHost &L = C->levels[l];
         LevelHost &Lc = C->levels[l + 1];
         const T *rhs = l == 0 ? rhs0 : (const T *)L.rhs;
@@ -1010,6 +1031,8 @@ static std::string graph_key(shkz_ctx *C, const Problem &P, const void *const *v
                   sizeof(T), precond ? 1 : 0, P.ngrids, P.nlev, P.pre, P.post, P.pre_c, P.post_c, P.coarse_sweeps,
                   P.multi_max_bricks, P.smoother, P.local_k, P.omega, (void *)P.red.partials);
     k += buf;
+    std::snprintf(buf, sizeof(buf), "bt%p %d|", (const void *)P.bottom, P.bottom_level);
+    k += buf;
     for (int i = 0; i < nvec; ++i) {
         std::snprintf(buf, sizeof(buf), "%p,", vecs[i]);
         k += buf;
@@ -1051,7 +1074,7 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
     const dim3 g(nb), b(BLOCK);
     const OpDesc<T> A = op_of<T>(L0);
     const double es = (double)sizeof(T);
-    const Gate Q{ctl, S};
+    const Gate Q{ctl, S, BM_COARSEST | (sizeof(T) == 4 && P.with_bottom() ? BM_BOTTOM | BM_BELOW : 0)};
     // FP32 (the inner solve of the mixed-precision mode): the iterate is the FP64 pressure and the
     // operator apply uses the FP64 operator in FP64 arithmetic (k_apply_dot4, k_cg_update4)
     double *const x64 = P.x64;
@@ -2010,6 +2033,49 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
     int max_bricks = 8;
     for (int l = 1; l < P.nlev; ++l) finish_level(l);
     for (int l = 0; l < P.nlev; ++l) max_bricks = std::max(max_bricks, (int)brick_grid(C->levels[l].nbricks));
+    for (int l = 1; l < P.nlev; ++l) {
+        LevelHost &L = C->levels[l];
+        const size_t n = (size_t)std::max(L.nbricks, 1) * BRICK_CELLS;
+        const std::string sfx = std::to_string(l);
+        void *pp = nullptr;
+        SHKZ_TRY(AR.get("dir_l" + sfx, n * es, &pp));
+        L.dir = pp;
+        SHKZ_TRY(AR.get("gx_l" + sfx, n * es, &pp));
+        L.gx = pp;
+        SHKZ_TRY(AR.get("gy_l" + sfx, n * es, &pp));
+        L.gy = pp;
+        SHKZ_TRY(AR.get("gz_l" + sfx, n * es, &pp));
+        L.gz = pp;
+        SHKZ_TRY(AR.get("idiag_l" + sfx, n * es, &pp));
+        L.idiag = pp;
+        SHKZ_TRY(AR.get("rhs_l" + sfx, n * es, &pp));
+        L.rhs = pp;
+        SHKZ_TRY(AR.get("z_l" + sfx, n * es, &pp));
+        L.z = pp;
+        SHKZ_TRY(AR.get("tmp_l" + sfx, n * es, &pp));
+        L.tmp = pp;
+        SHKZ_TRY(AR.get("res_l" + sfx, n * es, &pp));
+        L.res = pp;
+    }
+    // the grids' bottoms: in mixed precision, each grid's levels of at most BOTTOM_BRICKS bricks (its
+    // last BOTTOM_LEVELS at most), which the brick-local V-cycle runs in one workgroup per grid
+    std::vector<int> bottom_of(ngrids, P.nlev), depth_of(ngrids, 1);  // first and one past the last level
+    const bool bottoms = P.mixed && P.nlev > 1 && C->use_bottom;
+    if (bottoms) {
+        P.bottom_level = 1;
+        for (int g = 0; g < ngrids; ++g) {
+            auto bricks = [&](int l) { return C->levels[l].gl[g].brick_end - C->levels[l].gl[g].brick_start; };
+            while (depth_of[g] < P.nlev && bricks(depth_of[g]) > 0) ++depth_of[g];
+            if (depth_of[g] == 1) continue;  // one brick, or no unknowns
+            int l = depth_of[g] - 1;
+            while (l > 1 && depth_of[g] - l < BOTTOM_LEVELS && bricks(l - 1) <= BOTTOM_BRICKS) --l;
+            bottom_of[g] = l;
+            P.bottom_level = std::max(P.bottom_level, l);
+            for (; l < depth_of[g]; ++l)
+                for (int b = C->levels[l].gl[g].brick_start; b < C->levels[l].gl[g].brick_end; ++b)
+                    C->levels[l].meta[b].flags |= l == bottom_of[g] ? BM_BOTTOM : BM_BOTTOM | BM_BELOW;
+        }
+    }
     // levels >= 1: their base tables
     SHKZ_TRY(upload_tables(1, P.nlev, false, "meta", C->pin_meta, true));
     if (C->host_links) {
@@ -2059,6 +2125,47 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
         for (int l = 0; l < P.nlev; ++l) std::fprintf(stderr, " %d%s", C->levels[l].nbricks, C->levels[l].any_coarsest ? "*" : "");
         std::fprintf(stderr, " bricks\n");
     }
+    if (multigrid)
+        for (int l = 0; l < P.nlev; ++l) {
+            LevelHost &L = C->levels[l];
+            L.ccode = nullptr;
+            if (L.any_coarsest)
+                SHKZ_TRY(arena_get(AR, "ccode_l" + std::to_string(l), (size_t)L.nbricks * BRICK_CELLS, &L.ccode));
+        }
+    if (bottoms) {
+        BottomGrid *db = nullptr;
+        SHKZ_TRY(arena_get(AR, "bottom", (size_t)ngrids, &db));
+        void *hb = nullptr;
+        SHKZ_TRY(ensure_pinned(C->pin_bottom, (size_t)ngrids * sizeof(BottomGrid), &hb));
+        for (int g = 0; g < ngrids; ++g) {
+            BottomGrid B{};
+            for (int l = bottom_of[g]; l < depth_of[g]; ++l) {
+                const LevelHost &L = C->levels[l];
+                const size_t first = (size_t)L.gl[g].brick_start, c = first * BRICK_CELLS;
+                BottomLevel &o = B.lev[B.n++];
+                o.dir = (const float *)L.dir + c;
+                o.gx = (const float *)L.gx + c;
+                o.gy = (const float *)L.gy + c;
+                o.gz = (const float *)L.gz + c;
+                o.idiag = (const float *)L.idiag + c;
+                o.rhs = (float *)L.rhs + c;
+                o.z = (float *)L.z + c;
+                o.tmp = (float *)L.tmp + c;
+                o.meta = L.desc.meta + first;
+                o.bxyz = L.desc.bxyz + 3 * first;
+                o.child64 = L.desc.child64 + 64 * first;
+                o.parent8 = L.desc.parent8 ? L.desc.parent8 + 8 * first : nullptr;
+                o.brick_start = (int)first;
+                o.nb = L.gl[g].brick_end - L.gl[g].brick_start;
+                o.deepest = l == P.nlev - 1;
+                o.flat = flat ? 1 : 0;
+                B.code = L.ccode ? L.ccode + c : nullptr;
+            }
+            std::memcpy((BottomGrid *)hb + g, &B, sizeof(B));
+        }
+        SHKZ_HIP(hipMemcpyAsync(db, hb, (size_t)ngrids * sizeof(BottomGrid), hipMemcpyHostToDevice, s));
+        P.bottom = db;
+    }
     // reduction scratch, scalars, control blocks
     SHKZ_TRY(arena_get(AR, "partials", (size_t)2 * max_bricks, &P.red.partials));
     SolveScalars *Sbuf = nullptr;
@@ -2068,30 +2175,6 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
     P.S_fin = Sbuf + 2 * ngrids;
     SHKZ_TRY(arena_get(AR, "ctl", 2, &P.ctl));
 
-    for (int l = 1; l < P.nlev; ++l) {
-        LevelHost &L = C->levels[l];
-        const size_t n = (size_t)std::max(L.nbricks, 1) * BRICK_CELLS;
-        const std::string sfx = std::to_string(l);
-        void *pp = nullptr;
-        SHKZ_TRY(AR.get("dir_l" + sfx, n * es, &pp));
-        L.dir = pp;
-        SHKZ_TRY(AR.get("gx_l" + sfx, n * es, &pp));
-        L.gx = pp;
-        SHKZ_TRY(AR.get("gy_l" + sfx, n * es, &pp));
-        L.gy = pp;
-        SHKZ_TRY(AR.get("gz_l" + sfx, n * es, &pp));
-        L.gz = pp;
-        SHKZ_TRY(AR.get("idiag_l" + sfx, n * es, &pp));
-        L.idiag = pp;
-        SHKZ_TRY(AR.get("rhs_l" + sfx, n * es, &pp));
-        L.rhs = pp;
-        SHKZ_TRY(AR.get("z_l" + sfx, n * es, &pp));
-        L.z = pp;
-        SHKZ_TRY(AR.get("tmp_l" + sfx, n * es, &pp));
-        L.tmp = pp;
-        SHKZ_TRY(AR.get("res_l" + sfx, n * es, &pp));
-        L.res = pp;
-    }
     {
         void *pp = nullptr;
         SHKZ_TRY(AR.get("res_l0", n0 * es, &pp));
@@ -2128,9 +2211,7 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
     if (multigrid) {
         for (int l = 0; l < P.nlev; ++l) {
             LevelHost &L = C->levels[l];
-            L.ccode = nullptr;
             if (!L.any_coarsest) continue;
-            SHKZ_TRY(arena_get(AR, "ccode_l" + std::to_string(l), (size_t)L.nbricks * BRICK_CELLS, &L.ccode));
             if (P.fp64_levels)
                 K.go("coarse_components", -1, 0, 0, dim3((unsigned)P.ngrids), dim3(BRICK_CELLS),
                      k_coarse_components<double>, L.desc, op_of<double>(L), L.ccode);
@@ -2807,6 +2888,8 @@ int shkz_create(int device, uint64_t hbm_budget_bytes, shkz_ctx **out) {
     C->keep_direction = kd && kd[0] == '1';
     const char *nf = std::getenv("SHKZ_NO_FUSE");
     C->fuse_krylov = !(nf && nf[0] == '1');
+    const char *nbt = std::getenv("SHKZ_NO_BOTTOM");
+    C->use_bottom = !(nbt && nbt[0] == '1');
     C->under_profiler = std::getenv("ROCP_TOOL_LIBRARIES") || std::getenv("ROCPROF_OUTPUT_PATH");
     const char *mb = std::getenv("SHKZ_MULTI_MAX_BRICKS");
     if (mb && mb[0]) C->multi_max_bricks = std::atoi(mb);
@@ -2833,7 +2916,7 @@ void shkz_destroy(shkz_ctx *C) {
     C->own_scenes.clear();
     if (C->host_scalars) (void)hipHostFree(C->host_scalars);
     if (C->host_ctl) (void)hipHostFree(C->host_ctl);
-    for (shkz_ctx::Pinned *b : {&C->pin_flags, &C->pin_meta0, &C->pin_meta, &C->pin_links, &C->pin_counts})
+    for (shkz_ctx::Pinned *b : {&C->pin_flags, &C->pin_meta0, &C->pin_meta, &C->pin_links, &C->pin_counts, &C->pin_bottom})
         if (b->p) (void)hipHostFree(b->p);
     delete C;
 }
