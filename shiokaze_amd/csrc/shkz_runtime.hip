@@ -20,6 +20,7 @@
 #include "shkz_advect.hpp"
 #include "shkz_serve.hpp"
 #include "shkz_error.hpp"
+#include "shkz_graph.hpp"
 
 #include <hip/hip_ext.h>
 
@@ -542,7 +543,12 @@ namespace shkz {
 struct Launcher {
     shkz_ctx *C;
     hipStream_t s;
-    bool capturing = false;
+    // a graph under construction: launches become its nodes, each after the one before.  The nodes are
+    // added one by one rather than captured from the stream, which is a state of the process: while one
+    // thread captured, a synchronous copy of another (a server's client) could fail (hipError 906).
+    hipGraph_t graph = nullptr;
+    hipGraphNode_t last = nullptr;
+    hipError_t graph_error = hipSuccess;
 
     int kernel_id(const char *name) {
         auto it = C->kernel_ids.find(name);
@@ -567,11 +573,15 @@ struct Launcher {
     // (hipExtLaunchKernelGGL), so the elapsed time is the kernel's own execution, as a kernel trace
     // reports it, without the cost of separate event packets.  The byte model (per unknown of
     // `level`, plus fixed) feeds the per-kernel achieved-bandwidth statistics.
-    template <class K, class... Args>
-    void go(const char *name, int level, double bytes_per_unknown, double bytes_fixed, dim3 grid, dim3 block, K kernel,
-            Args... args) {
+    template <class... P, class... Args>
+    void go(const char *name, int level, double bytes_per_unknown, double bytes_fixed, dim3 grid, dim3 block,
+            void (*kernel)(P...), Args... args) {
         if (grid.x == 0) return;
-        if (C->timing && !capturing) {
+        if (graph) {
+            if (graph_error == hipSuccess) graph_error = add_kernel_node(graph, &last, grid, block, kernel, args...);
+            return;
+        }
+        if (C->timing) {
             hipEvent_t e0 = event(), e1 = event();
             if (e0 && e1) {
                 hipExtLaunchKernelGGL(kernel, grid, block, 0, s, e0, e1, 0, args...);
@@ -1054,8 +1064,8 @@ static std::string graph_key(shkz_ctx *C, const Problem &P, const void *const *v
 
 // Krylov loop on level 0 for every grid of the batch: T = element type; precond = V-cycle or
 // identity (plain CG).  Expects r (residual) and per-grid S with tol/maxit/iter set and the control
-// block counting the grids already done.  x is updated in place.  One iteration is captured once
-// into a hipGraph and replayed; every kernel returns at once when all grids are done and skips the
+// block counting the grids already done.  x is updated in place.  One iteration is built once as a
+// hipGraph and replayed; every kernel returns at once when all grids are done and skips the
 // bricks of a grid that is done, so a chunk of replays may overshoot by a few no-op iterations
 // without changing any result.  `last` receives the final per-grid scalars.
 //
@@ -1175,7 +1185,7 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
         }
     };
     // the iteration (fused: each of the two half-iterations, which alternate the direction
-    // buffers) captured once into a hipGraph and replayed
+    // buffers) built once as a hipGraph and replayed
     auto graph_for = [&](const std::string &key, auto &&body, hipGraphExec_t *out) -> int {
         for (auto &g : C->graphs)
             if (g.exec && g.key == key) {
@@ -1193,16 +1203,16 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
             SHKZ_HIP(hipGraphExecDestroy(C->graphs[lru].exec));
             C->graphs.erase(C->graphs.begin() + (long)lru);
         }
-        hipGraph_t graph = nullptr;
-        SHKZ_HIP(hipStreamBeginCapture(K.s, hipStreamCaptureModeThreadLocal));
-        K.capturing = true;
+        SHKZ_HIP(hipGraphCreate(&K.graph, 0));
+        K.last = nullptr;
+        K.graph_error = hipSuccess;
         body();
-        K.capturing = false;
-        SHKZ_HIP(hipStreamEndCapture(K.s, &graph));
         hipGraphExec_t made = nullptr;
-        hipError_t e = hipGraphInstantiateWithFlags(&made, graph, 0);
-        (void)hipGraphDestroy(graph);
-        if (e != hipSuccess) return fail(SHKZ_ERR_DEVICE, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
+        hipError_t e = K.graph_error;
+        if (e == hipSuccess) e = hipGraphInstantiateWithFlags(&made, K.graph, 0);
+        (void)hipGraphDestroy(K.graph);
+        K.graph = nullptr;
+        if (e != hipSuccess) return fail(SHKZ_ERR_DEVICE, "building an iteration's graph failed: %s", hipGetErrorString(e));
         C->graphs.push_back(shkz_ctx::GraphSlot{key, made, ++C->graph_clock});
         *out = made;
         return SHKZ_OK;
