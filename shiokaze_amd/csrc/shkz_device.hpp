@@ -113,7 +113,8 @@ struct OpDesc {
 // Scalars of one grid's Krylov solve, resident on the device so that no iteration waits on the
 // host.
 struct SolveScalars {
-    double rz;        // r.z of the current iteration
+    double rz[2];     // r.z of the current iteration: [0], or, where the kernels that use r.z form it
+                      // themselves (fold_partials), alternately [0] and [1]
     double pq;        // p.Ap
     double alpha, beta;
     double rinf;      // ||r||_inf after the last update

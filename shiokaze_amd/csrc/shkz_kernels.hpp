@@ -684,6 +684,8 @@ __global__ __launch_bounds__(BLOCK) void k_update_p(LevelDesc L, const T *__rest
     p[c] = first ? zv : zv + (T)Sg.beta * pv;
 }
 
+constexpr int ROW4_GROUP = BRICK_CELLS / 4;  // threads of a row-4 workgroup of one brick
+
 enum FinOp {
     FIN_PQ = 0,           // alpha = rz / pq
     FIN_UPDATE = 1,       // rinf, rl2, iteration count, convergence test
@@ -730,6 +732,139 @@ __device__ __forceinline__ void mark_done(SolveScalars &S, BatchCtl *ctl) {
         if (n >= ctl->ngrids) ctl->all_done = 1;
     }
 }
+
+// The convergence test of pcg_solver.h:278-285 on a grid's updated residual: a = ||r||_inf, b = r.r;
+// s0: the scalars before the update.
+__device__ __forceinline__ void finish_update(SolveScalars &S, const SolveScalars &s0, double a, double b, BatchCtl *ctl,
+                                              bool cg) {
+    const double rl2 = sqrt(b);
+    S.rinf = a;
+    S.rl2 = rl2;
+    const int it = s0.iter + 1;
+    S.iter = it;
+    const double cur = s0.norm == 0 ? a : rl2;
+    if (cg) {
+        S.beta = b / s0.rz[0];
+        S.rz[0] = b;
+    }
+    // an inner solve whose FP32 residual stops reaching new minima hands back to the FP64
+    // defect correction (a consistent singular system, for one, keeps a null-space component
+    // of the FP32 rounding that no iteration removes)
+    bool stalled = false;
+    if (s0.stall_limit > 0) {
+        if (cur < s0.rmin) {
+            S.rmin = cur;
+            S.stall = 0;
+        } else {
+            const int st = s0.stall + 1;
+            S.stall = st;
+            stalled = st >= s0.stall_limit;
+        }
+    }
+    if (!(b == b)) {
+        S.status = 1;
+        mark_done(S, ctl);
+    } else if (cur <= s0.tol) {
+        S.converged = 1;
+        mark_done(S, ctl);
+    } else if (it >= s0.maxit || stalled) {
+        mark_done(S, ctl);
+    }
+}
+
+// The sums of a grid's partials are those of 1024 threads (k_finalize): thread t adds the partials t,
+// t + 1024, ... of the grid, 64 threads a wavefront's butterfly, and the 16 wavefronts' sums are added
+// in order.  The kernels below take them in smaller workgroups, with the same bits.
+constexpr int FIN_THREADS = 1024;
+
+// k_finalize's FIN_UPDATE of grid g in a 512-thread workgroup: each thread stands for two.
+struct FinUpdate {
+    const double *partials;  // nullptr: nothing to do
+    SolveScalars *S;
+    BatchCtl *ctl;
+};
+__device__ __forceinline__ void finalize_update(const FinUpdate &F, const LevelDesc &L0, int g) {
+    __shared__ double lds[2][FIN_THREADS / 64];
+    SolveScalars &S = F.S[g];
+    const SolveScalars s0 = S;
+    const bool stop = s0.done || F.ctl->all_done;
+    int bs = 0, be = L0.nbricks;
+    if (L0.ngrids > 1) {
+        bs = L0.gl[g].brick_start;
+        be = L0.gl[g].brick_end;
+    }
+    const double2 *pp = reinterpret_cast<const double2 *>(F.partials);
+    double a[2] = {0.0, 0.0}, b[2] = {0.0, 0.0};
+    constexpr int U = 6;  // 12 loads in flight per thread (a 256^3 grid of 10,000 bricks takes 20)
+    for (int i = bs + (int)threadIdx.x; i < be; i += U * FIN_THREADS) {
+        double2 v[2][U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int j = i + u * FIN_THREADS + k * (FIN_THREADS / 2);
+                v[k][u] = j < be ? pp[j] : make_double2(0.0, 0.0);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                a[k] = fmax(a[k], v[k][u].x);
+                b[k] += v[k][u].y;
+            }
+    }
+    if (stop) return;
+    const int w = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const double wa = wave_max(a[k]), wb = wave_sum(b[k]);
+        if ((threadIdx.x & 63) == 0) {
+            lds[0][w + k * (FIN_THREADS / 128)] = wa;
+            lds[1][w + k * (FIN_THREADS / 128)] = wb;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    double sa = 0.0, sb = 0.0;
+    for (int i = 0; i < FIN_THREADS / 64; ++i) {
+        sa = fmax(sa, lds[0][i]);
+        sb += lds[1][i];
+    }
+    finish_update(S, s0, sa, sb, F.ctl, false);
+}
+
+// The first partials of the n <= FOLD_BRICKS bricks of a single grid, summed by every 128-thread
+// workgroup of the kernel that uses the sum, so that no finalize launch (3 to 4 us, most of it its
+// boundary and one trip to memory) stands between the producer and it.  load() issues the loads,
+// sum() adds; all threads call both.  lds: 16 doubles.  The limit keeps what all workgroups read
+// together (8 n^2 bytes) well under the time of a launch: 8 MB from the L2s at 1024.
+constexpr int FOLD_BRICKS = 1024;
+struct FoldPartials {
+    double v[FOLD_BRICKS / ROW4_GROUP];
+    int n;
+    __device__ __forceinline__ void load(const double *__restrict__ partials, int nb) {
+        n = nb;
+#pragma unroll
+        for (int k = 0; k < FOLD_BRICKS / ROW4_GROUP; ++k) {
+            const int i = k * ROW4_GROUP + (int)threadIdx.x;
+            v[k] = i < nb ? partials[2 * i] : 0.0;
+        }
+    }
+    __device__ __forceinline__ double sum(double *lds) const {
+        const int w = threadIdx.x >> 6;
+#pragma unroll
+        for (int k = 0; k < FOLD_BRICKS / ROW4_GROUP; ++k) {
+            if (k * ROW4_GROUP >= n) break;
+            const double s = wave_sum(v[k]);
+            if ((threadIdx.x & 63) == 0) lds[2 * k + w] = s;
+        }
+        __syncthreads();
+        double total = 0.0;
+        const int waves = 2 * ((n + ROW4_GROUP - 1) / ROW4_GROUP);
+        for (int i = 0; i < waves; ++i) total += lds[i];
+        return total;
+    }
+};
 
 // One block per grid combines the partials of the grid's bricks in brick order and updates the
 // grid's scalars.  Grids that finished are left alone (their kernels stored no partials).
@@ -780,7 +915,7 @@ __global__ __launch_bounds__(1024) void k_finalize(const double *__restrict__ pa
     switch (op) {
     case FIN_PQ: {
         S.pq = a;
-        const double al = s0.rz / a;
+        const double al = s0.rz[0] / a;
         S.alpha = al;
         if (!(al == al) || al - al != 0.0) {
             S.status = 1;
@@ -789,46 +924,13 @@ __global__ __launch_bounds__(1024) void k_finalize(const double *__restrict__ pa
         break;
     }
     case FIN_UPDATE:
-    case FIN_UPDATE_CG: {
-        const double rl2 = sqrt(b);
-        S.rinf = a;
-        S.rl2 = rl2;
-        const int it = s0.iter + 1;
-        S.iter = it;
-        const double cur = s0.norm == 0 ? a : rl2;
-        if (op == FIN_UPDATE_CG) {
-            S.beta = b / s0.rz;
-            S.rz = b;
-        }
-        // an inner solve whose FP32 residual stops reaching new minima hands back to the FP64
-        // defect correction (a consistent singular system, for one, keeps a null-space component
-        // of the FP32 rounding that no iteration removes)
-        bool stalled = false;
-        if (s0.stall_limit > 0) {
-            if (cur < s0.rmin) {
-                S.rmin = cur;
-                S.stall = 0;
-            } else {
-                const int st = s0.stall + 1;
-                S.stall = st;
-                stalled = st >= s0.stall_limit;
-            }
-        }
-        if (!(b == b)) {
-            S.status = 1;
-            mark_done(S, ctl);
-        } else if (cur <= s0.tol) {
-            S.converged = 1;
-            mark_done(S, ctl);
-        } else if (it >= s0.maxit || stalled) {
-            mark_done(S, ctl);
-        }
+    case FIN_UPDATE_CG:
+        finish_update(S, s0, a, b, ctl, op == FIN_UPDATE_CG);
         break;
-    }
     case FIN_RZ_FIRST:
     case FIN_RZ: {
-        S.beta = op == FIN_RZ_FIRST ? 0.0 : a / s0.rz;
-        S.rz = a;
+        S.beta = op == FIN_RZ_FIRST ? 0.0 : a / s0.rz[0];
+        S.rz[0] = a;
         if (!(a == a)) {
             S.status = 1;
             mark_done(S, ctl);
@@ -1027,7 +1129,7 @@ __device__ __forceinline__ void jacobi_brick(const LevelDesc &L, const OpDesc<T>
 // h = q & 1; the two lanes of a row are neighbours in the wavefront and swap their edge values, so
 // only the row's two end cells read a value across the brick's z faces.  A quarter of the load
 // instructions of the one-cell form, and 16-byte accesses.
-constexpr int ROW4_THREADS = BRICK_CELLS / 4;
+constexpr int ROW4_THREADS = ROW4_GROUP;
 
 __device__ __forceinline__ float4 ld4(const float *__restrict__ a, long i) {
     return *reinterpret_cast<const float4 *>(a + i);
@@ -1603,9 +1705,9 @@ __device__ __forceinline__ void apply_row4(const LevelDesc &L, const OpDesc<T> &
 // flag fixes BPB at compile time (blockDim.x is a 16-bit hidden kernel argument that hipcc reads
 // with a vector load, one more memory round trip at the start of every wave).
 template <int FINEST>
-__device__ __forceinline__ void row4_slot(const LevelDesc &L, int &br, int &q) {
+__device__ __forceinline__ void row4_slot(const LevelDesc &L, int &br, int &q, int skip = 0) {
     constexpr int BPB = FINEST ? BLOCK / ROW4_THREADS : 1;
-    br = BPB * xcd_brick(blockIdx.x, gridDim.x) + (int)(threadIdx.x / ROW4_THREADS);
+    br = BPB * xcd_brick(blockIdx.x - skip, gridDim.x - skip) + (int)(threadIdx.x / ROW4_THREADS);
     q = threadIdx.x % ROW4_THREADS;
 }
 
@@ -1624,12 +1726,25 @@ __device__ __forceinline__ void row4_reduce2(double &a, double &b, double *lds) 
     b = lds[2] + lds[3];
 }
 
-// res = rhs - A z (k_residual on rows).
-template <int FINEST>
+// res = rhs - A z (k_residual on rows).  FIN (finest level): the first workgroups, one per grid (rounded
+// up to 8, which keeps the bricks' XCDs), run the convergence test of the residual update before this
+// kernel instead of a launch of their own (3 to 6 us).  Nothing in the V-cycle waits for its outcome: a
+// grid that it finds done only loses what this kernel and its neighbours do for it.
+template <int FINEST, int FIN = 0>
 __global__ __launch_bounds__(BLOCK) void k_residual4(LevelDesc L, OpDesc<float> A, const float *__restrict__ rhs,
-                                                     const float *__restrict__ z, float *__restrict__ res, Gate Q) {
+                                                     const float *__restrict__ z, float *__restrict__ res, Gate Q,
+                                                     FinUpdate F) {
     int br, q;
-    row4_slot<FINEST>(L, br, q);
+    if (FIN) {
+        const int front = (L.ngrids + 7) & ~7;
+        if ((int)blockIdx.x < front) {
+            if ((int)blockIdx.x < L.ngrids) finalize_update(F, L, blockIdx.x);
+            return;
+        }
+        row4_slot<FINEST>(L, br, q, front);
+    } else {
+        row4_slot<FINEST>(L, br, q);
+    }
     if (br >= L.nbricks) return;
     const BrickMeta m = L.meta[br];
     if (all_done(Q) || skip_smooth(Q, L, m)) return;
@@ -1739,22 +1854,45 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_apply_dot4(LevelDesc L, OpDesc
 // and of their neighbours is formed on the fly from z and the previous direction (the same FP32
 // arithmetic), written to pnew (a different buffer than pold: other workgroups still read pold),
 // and q = A pnew with the pnew.q partials.
+// FOLD (a single grid of at most FOLD_BRICKS bricks): beta = r.z / (the r.z before, S->rz[slot]) is
+// formed here from the partials of r.z (rz), as FIN_RZ does; the workgroup of brick 0 records it, r.z in
+// S->rz[slot ^ 1].
+template <int FOLD>
 __global__ __launch_bounds__(ROW4_THREADS) void k_apply_dot4p(LevelDesc L, OpDesc<double> A,
                                                               const float *__restrict__ z,
                                                               const float *__restrict__ pold,
                                                               float *__restrict__ pnew, float *__restrict__ qv,
-                                                              const SolveScalars *S, const BatchCtl *ctl, RedBuf R) {
-    __shared__ double lds[4];
+                                                              SolveScalars *S, BatchCtl *ctl, RedBuf R,
+                                                              const double *__restrict__ rz, int slot) {
+    __shared__ double lds[FOLD ? 16 : 4];
     const int br = brick_or_idle(L);
     if (br < 0) return;
     const BrickMeta m = L.meta[br];
     const int g = L.ngrids > 1 ? m.grid : 0;
     if (L.ngrids > 1 && (ctl->all_done || S[g].done)) return;
     const Row4Nbrs N = row4_nbrs(m, br, threadIdx.x);
+    FoldPartials P;
+    if (FOLD) P.load(rz, L.nbricks);
     const Row4Vals<float> zv = row4_vals(z, N);
     const Row4Vals<float> po = row4_vals(pold, N);
     if (ctl->all_done) return;
-    const float beta = (float)S[g].beta;
+    float beta;
+    if (FOLD) {
+        const double now = P.sum(lds), b64 = now / S->rz[slot];
+        if (br == 0 && threadIdx.x == 0) {
+            S->beta = b64;
+            S->rz[slot ^ 1] = now;
+            if (!(now == now)) {
+                S->status = 1;
+                mark_done(*S, ctl);
+            }
+        }
+        if (!(now == now)) return;
+        beta = (float)b64;
+        __syncthreads();  // lds is used again
+    } else {
+        beta = (float)S[g].beta;
+    }
     Row4Vals<float> v;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1787,20 +1925,25 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_apply_dot4p(LevelDesc L, OpDes
 // (not those of grids ending on this level), with the same arithmetic: 1 = a damped Jacobi sweep
 // (k_smooth_first4<1>), z = omega * idiag * r; 2 = the brick-local smoother (k_pre_local4<K>),
 // whose brick is the workgroup's.  A grid that this update finds converged gets a z it never uses.
-template <int ZFIRST, int K = LOCAL_SGS_SWEEPS>
+// FOLD (a single grid of at most FOLD_BRICKS bricks): alpha = S->rz[slot] / (p.q) is formed here from the
+// partials of p.q (pq), as FIN_PQ does; the workgroup of brick 0 records it.
+template <int ZFIRST, int K = LOCAL_SGS_SWEEPS, int FOLD = 0>
 __global__ __launch_bounds__(ROW4_THREADS) void k_cg_update4(LevelDesc L, double *__restrict__ x,
                                                              float *__restrict__ r, const float *__restrict__ p,
-                                                             const float *__restrict__ qv, const SolveScalars *S,
-                                                             const BatchCtl *ctl, RedBuf R,
+                                                             const float *__restrict__ qv, SolveScalars *S,
+                                                             BatchCtl *ctl, RedBuf R,
                                                              const float *__restrict__ idiag, float *__restrict__ z,
-                                                             float omega, OpDesc<float> A32) {
-    __shared__ double lds[4];
+                                                             float omega, OpDesc<float> A32,
+                                                             const double *__restrict__ pq, int slot) {
+    __shared__ double lds[FOLD ? 16 : 4];
     const int br = brick_or_idle(L);
     if (br < 0) return;
     const long c = (long)br * BRICK_CELLS + 4 * threadIdx.x;
     const BrickMeta m = L.meta[br];
     const int g = L.ngrids > 1 ? m.grid : 0;
     if (L.ngrids > 1 && (ctl->all_done || S[g].done)) return;
+    FoldPartials P;
+    if (FOLD) P.load(pq, L.nbricks);
     double xv[4];
     float pv[4], rv[4], qq[4], id[4];
     load4(x, c, xv);
@@ -1821,7 +1964,24 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_cg_update4(LevelDesc L, double
     }
     const SolveScalars &Sg = S[g];
     if (ctl->all_done || Sg.done) return;
-    const double alpha = Sg.alpha;
+    double alpha;
+    if (FOLD) {
+        const double now = P.sum(lds);
+        alpha = S->rz[slot] / now;
+        const bool bad = !(alpha == alpha) || alpha - alpha != 0.0;
+        if (br == 0 && threadIdx.x == 0) {
+            S->pq = now;
+            S->alpha = alpha;
+            if (bad) {
+                S->status = 1;
+                mark_done(*S, ctl);
+            }
+        }
+        if (bad) return;
+        __syncthreads();  // lds is used again
+    } else {
+        alpha = Sg.alpha;
+    }
     const float alpha32 = (float)alpha;
     double mx = 0.0, sq = 0.0;
 #pragma unroll

@@ -639,7 +639,7 @@ struct Problem {
     // per-grid scalars: outer (FP64 defect / FP64 solve), inner (FP32 solve), final check
     SolveScalars *S_out = nullptr, *S_in = nullptr, *S_fin = nullptr;
     BatchCtl *ctl = nullptr;  // [0] outer / FP64 solve, [1] inner solve
-    RedBuf red{};
+    RedBuf red{}, red2{};  // red2: the p.q partials where their reader writes partials itself
     int pre = 4, post = 4, pre_c = 4, post_c = 4, coarse_sweeps = 48;
     int smoother = SHKZ_SMOOTH_JACOBI;  // finest level (SHKZ_SMOOTH_BRICK only with an FP32 V-cycle)
     int local_k = LOCAL_SGS_SWEEPS;      // brick-local smoother: sweeps per finest-level application (2, 3)
@@ -786,10 +786,11 @@ static void jacobi_sweep(shkz_ctx *C, Launcher &K, int l, bool dot, const LevelD
 // z.  Each grid descends to its own coarsest level (one brick), solved there by k_coarse_solve;
 // the smoothing kernels skip the bricks of grids that end on their level.  With dot_partials, the
 // last post-smoothing sweep on the finest level (or the coarse solve of a one-brick grid) also
-// stores r.z partials in P.red.
+// stores r.z partials in P.red.  fin (brick-local smoother, more than one level): the convergence test
+// of the residual update before the cycle, run beside the finest level's residual.
 template <class T>
 static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *tmp0, Gate Q, bool dot_partials,
-                 bool first_done = false) {
+                 bool first_done = false, FinUpdate fin = FinUpdate{nullptr, nullptr, nullptr}) {
     const int nl = P.nlev;
     const bool brick_smoother = sizeof(T) == 4 && P.smoother == SHKZ_SMOOTH_BRICK;
     std::vector<T *> zcur(nl), zoth(nl);
@@ -900,10 +901,14 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
             }
         }
         if (!res_done) {
-            if constexpr (sizeof(T) == 4)
-                K.go(f ? "residual_L0" : "residual_Lc", l, 7 * es, -usave(C, l, 4 * es), row4_launch(L.nbricks, f).grid,
-                     row4_launch(L.nbricks, f).block, f ? k_residual4<1> : k_residual4<0>, L.desc, A, rhs,
-                     (const T *)cur, (T *)L.res, Q);
+            if constexpr (sizeof(T) == 4) {
+                Row4Launch R4 = row4_launch(L.nbricks, f);
+                const bool with_fin = f && fin.partials;
+                if (with_fin) R4.grid.x += (unsigned)((P.ngrids + 7) & ~7);
+                K.go(f ? "residual_L0" : "residual_Lc", l, 7 * es, -usave(C, l, 4 * es), R4.grid, R4.block,
+                     with_fin ? k_residual4<1, 1> : f ? k_residual4<1> : k_residual4<0>, L.desc, A, rhs,
+                     (const T *)cur, (T *)L.res, Q, fin);
+            }
             else
                 K.go(f ? "residual_L0" : "residual_Lc", l, 7 * es, -usave(C, l, 4 * es), g, b,
                      f ? k_residual<T, 1> : k_residual<T, 0>, L.desc, A, rhs, (const T *)cur, (T *)L.res, Q);
@@ -1115,47 +1120,56 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
     // sweep (k_cg_update4z); the direction alternates between two buffers, so one captured graph
     // holds two iterations.  Same kernels' arithmetic, same results as the separate kernels.
     const bool fused = sizeof(T) == 4 && precond && !keep_dir && C->fuse_krylov && P.kp2;
+    const bool brick = P.smoother == SHKZ_SMOOTH_BRICK;
+    // alpha and beta formed by the kernels that use them (single grids up to FOLD_BRICKS bricks), p.q
+    // partials apart from the others
+    const bool fold = fused && brick && P.ngrids == 1 && L0.nbricks <= FOLD_BRICKS && P.nlev > 1 && fused_dot;
+    const RedBuf pq = fold ? P.red2 : P.red;
     T *const p2 = (T *)P.kp2;
-    auto half = [&](T *pc, T *pn) {
+    // slot: which of S->rz holds the r.z of pc
+    auto half = [&](T *pc, T *pn, int slot) {
         if constexpr (sizeof(T) == 4) {
             const bool zfirst = P.nlev > 1;
             const LevelHost &F0 = C->levels[0];
             const OpDesc<float> A32 = op_of<float>(F0);
-            if (zfirst && P.smoother == SHKZ_SMOOTH_BRICK)
+            if (zfirst && brick)
                 K.go("cg_update_z", 0, 52, -usave(C, 0, 16), g, dim3(ROW4_THREADS),
-                     P.local_k == 3 ? k_cg_update4<2, 3> : k_cg_update4<2, 2>, L0.desc, x64, r,
-                     (const T *)pc, (const T *)q, (const SolveScalars *)S, (const BatchCtl *)ctl, P.red,
-                     (const T *)F0.idiag, z, (T)P.omega, A32);
+                     fold ? (P.local_k == 3 ? k_cg_update4<2, 3, 1> : k_cg_update4<2, 2, 1>)
+                          : (P.local_k == 3 ? k_cg_update4<2, 3> : k_cg_update4<2, 2>),
+                     L0.desc, x64, r, (const T *)pc, (const T *)q, S, ctl, P.red, (const T *)F0.idiag, z, (T)P.omega, A32,
+                     (const double *)pq.partials, slot);
             else if (zfirst)
                 K.go("cg_update_z", 0, 40, -usave(C, 0, 4), g, dim3(ROW4_THREADS), k_cg_update4<1>, L0.desc, x64, r,
-                     (const T *)pc, (const T *)q, (const SolveScalars *)S, (const BatchCtl *)ctl, P.red,
-                     (const T *)F0.idiag, z, (T)P.omega, A32);
+                     (const T *)pc, (const T *)q, S, ctl, P.red, (const T *)F0.idiag, z, (T)P.omega, A32,
+                     (const double *)nullptr, 0);
             else
                 K.go("cg_update", 0, 32, 0, g, dim3(ROW4_THREADS), k_cg_update4<0>, L0.desc, x64, r, (const T *)pc,
-                     (const T *)q, (const SolveScalars *)S, (const BatchCtl *)ctl, P.red, (const T *)nullptr,
-                     (T *)nullptr, (T)0, A32);
-            finalize(K, P, L0.desc, S, ctl, FIN_UPDATE);
-            const T *zz = vcycle<T>(C, K, P, r, z, tmp, Q, fused_dot, zfirst);
+                     (const T *)q, S, ctl, P.red, (const T *)nullptr, (T *)nullptr, (T)0, A32, (const double *)nullptr, 0);
+            // (a one-brick grid's r.z partials come from its coarse solve, before the residual)
+            const bool with_residual = zfirst && brick && !L0.any_coarsest;
+            if (!with_residual) finalize(K, P, L0.desc, S, ctl, FIN_UPDATE);
+            const T *zz = vcycle<T>(C, K, P, r, z, tmp, Q, fused_dot, zfirst,
+                                    with_residual ? FinUpdate{P.red.partials, S, ctl} : FinUpdate{nullptr, nullptr, nullptr});
             if (!fused_dot)
                 K.go("dot_rz", 0, 2 * es, 0, g, b, k_dot_rz<T>, L0.desc, (const T *)r, zz, (const SolveScalars *)S,
                      (const BatchCtl *)ctl, P.red);
-            finalize(K, P, L0.desc, S, ctl, FIN_RZ);
-            K.go("apply_dot_p", 0, 48, -usave(C, 0, 32), g, dim3(ROW4_THREADS), k_apply_dot4p, L0.desc, A64, zz,
-                 (const T *)pc, pn, q, (const SolveScalars *)S, (const BatchCtl *)ctl, P.red);
-            finalize(K, P, L0.desc, S, ctl, FIN_PQ);
+            if (!fold) finalize(K, P, L0.desc, S, ctl, FIN_RZ);
+            K.go("apply_dot_p", 0, 48, -usave(C, 0, 32), g, dim3(ROW4_THREADS), fold ? k_apply_dot4p<1> : k_apply_dot4p<0>,
+                 L0.desc, A64, zz, (const T *)pc, pn, q, S, ctl, pq, (const double *)P.red.partials, slot);
+            if (!fold) finalize(K, P, L0.desc, S, ctl, FIN_PQ);
         }
     };
     if (fused) {
         // the first direction's operator apply (the loop starts with the residual update)
         if constexpr (sizeof(T) == 4)
             K.go("apply_dot", 0, 40, -usave(C, 0, 32), g, dim3(ROW4_THREADS), k_apply_dot4, L0.desc, A64, (const T *)p,
-                 q, (const SolveScalars *)S, (const BatchCtl *)ctl, P.red);
-        finalize(K, P, L0.desc, S, ctl, FIN_PQ);
+                 q, (const SolveScalars *)S, (const BatchCtl *)ctl, pq);
+        if (!fold) finalize(K, P, L0.desc, S, ctl, FIN_PQ);
     }
     auto iteration = [&]() {
         if (fused) {
-            half(p, p2);
-            half(p2, p);
+            half(p, p2, 0);
+            half(p2, p, 1);
             return;
         }
         if constexpr (sizeof(T) == 4)
@@ -1167,8 +1181,8 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
         finalize(K, P, L0.desc, S, ctl, FIN_PQ);
         if constexpr (sizeof(T) == 4)
             K.go("cg_update", 0, 32, 0, g, dim3(ROW4_THREADS), k_cg_update4<0>, L0.desc, x64, r, (const T *)p,
-                 (const T *)q, (const SolveScalars *)S, (const BatchCtl *)ctl, P.red, (const T *)nullptr, (T *)nullptr,
-                 (T)0, op_of<float>(L0));
+                 (const T *)q, S, ctl, P.red, (const T *)nullptr, (T *)nullptr, (T)0, op_of<float>(L0),
+                 (const double *)nullptr, 0);
         else
             K.go("cg_update", 0, 6 * es, 0, g, b, k_cg_update<T>, L0.desc, x, r, (const T *)p, (const T *)q,
                  (const SolveScalars *)S, (const BatchCtl *)ctl, P.red);
@@ -1226,8 +1240,8 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
         if (fused) {
             // one graph per half-iteration (the second one a later find cannot evict: the first
             // was used last but one), so that a solve replays exactly the iterations it asks for
-            SHKZ_TRY(graph_for(key + "A", [&]() { half(p, p2); }, &exec));
-            SHKZ_TRY(graph_for(key + "B", [&]() { half(p2, p); }, &exec2));
+            SHKZ_TRY(graph_for(key + "A", [&]() { half(p, p2, 0); }, &exec));
+            SHKZ_TRY(graph_for(key + "B", [&]() { half(p2, p, 1); }, &exec2));
         } else {
             SHKZ_TRY(graph_for(key, iteration, &exec));
         }
@@ -1243,8 +1257,8 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
                 continue;
             }
             if (exec) SHKZ_HIP(hipGraphLaunch(phase ? exec2 : exec, K.s));
-            else if (phase) half(p2, p);
-            else half(p, p2);
+            else if (phase) half(p2, p, 1);
+            else half(p, p2, 0);
             phase ^= 1;
         }
         SHKZ_TRY(read_scalars(C, K.s, S, P.ngrids, last, ctl, &hc, S2, last2));
@@ -2177,7 +2191,8 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
         P.bottom = db;
     }
     // reduction scratch, scalars, control blocks
-    SHKZ_TRY(arena_get(AR, "partials", (size_t)2 * max_bricks, &P.red.partials));
+    SHKZ_TRY(arena_get(AR, "partials", (size_t)4 * max_bricks, &P.red.partials));
+    P.red2.partials = P.red.partials + (size_t)2 * max_bricks;
     SolveScalars *Sbuf = nullptr;
     SHKZ_TRY(arena_get(AR, "scalars", (size_t)3 * ngrids, &Sbuf));
     P.S_out = Sbuf;
