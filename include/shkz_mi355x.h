@@ -387,7 +387,7 @@ int shkz_linsolve_csr(shkz_linsolver *solver, int64_t n, const int64_t *rowptr, 
  * are not read back to be checked).  Same iteration, kernels and launch shapes as
  * shkz_linsolve_csr, so the same result, launched directly on `stream` (no graph).
  * The working vectors live in one fixed device array inside the library, sized for at most
- * SHKZ_LS_NOALLOC_MAX_ROWS rows (about 10.6 MB; each GPU the library runs on holds its own copy
+ * SHKZ_LS_NOALLOC_MAX_ROWS rows (about 11.2 MB; each GPU the library runs on holds its own copy
  * until the process ends); larger systems fail with SHKZ_ERR_INVALID.  No call allocates or frees
  * device memory.  Every call on one GPU shares that GPU's array: calls that overlap on one GPU
  * (from any solver object or thread) race and must be serialised by the caller.  Each call

@@ -11,11 +11,13 @@
 //
 // Layout: CSR with 32-bit column indices on the device.  SpMV gives each row 8 lanes of a
 // 64-wide wavefront (rows of a few to a few dozen entries, the shape of the Poisson systems the
-// reference assembles) and reduces them with lane shuffles.  Dot products and norms are
+// reference assembles) and reduces them across the lanes.  Dot products and norms are
 // deterministic two-pass reductions (per-block partials, summed in block order by one block).
-// One iteration is captured once into a hipGraph and replayed; the scalars stay on the device.
+// Iterations are replayed from hipGraphs; the scalars stay on the device.
 #include "../../include/shkz_mi355x.h"
+#include "shkz_device.hpp"
 #include "shkz_error.hpp"
+#include "shkz_graph.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -37,23 +39,12 @@ struct LsScalars {
     int32_t iter, maxit, done, converged, status, pad;
 };
 
-__device__ __forceinline__ double ls_wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-__device__ __forceinline__ double ls_wave_max(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 // Block reduction of (a: max or sum, b: sum) into partials[2*block].
 template <bool AMAX>
 __device__ __forceinline__ void ls_block_partials(double a, double b, double *partials) {
     __shared__ double lds[2][LS_BLOCK / 64];
-    a = AMAX ? ls_wave_max(a) : ls_wave_sum(a);
-    b = ls_wave_sum(b);
+    a = AMAX ? shkz::wave_max(a) : shkz::wave_sum(a);
+    b = shkz::wave_sum(b);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0) {
         lds[0][wid] = a;
@@ -99,6 +90,15 @@ __global__ void k_ls_init(int n, const double *__restrict__ b, double *__restric
     ls_block_partials<true>(mx, rz, partials);
 }
 
+// Sum over a row's 8 lanes in the first of them (lanes i, i + 4, then i, i + 2, then i, i + 1), by DPP
+// row shifts.
+__device__ __forceinline__ double ls_row_sum(double acc) {
+    acc += shkz::dpp_move<0x104>(acc);
+    acc += shkz::dpp_move<0x102>(acc);
+    acc += shkz::dpp_move<0x101>(acc);
+    return acc;
+}
+
 // q = A p, partial p.q
 __global__ void k_ls_spmv_dot(int n, const int *__restrict__ rowptr, const int *__restrict__ col,
                               const double *__restrict__ val, const double *__restrict__ p, double *__restrict__ q,
@@ -111,8 +111,7 @@ __global__ void k_ls_spmv_dot(int n, const int *__restrict__ rowptr, const int *
         const int e1 = rowptr[row + 1];
         for (int e = rowptr[row] + lane; e < e1; e += LS_LANES) acc += val[e] * p[col[e]];
     }
-#pragma unroll
-    for (int off = LS_LANES / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    acc = ls_row_sum(acc);
     double part = 0.0;
     if (row < n && lane == 0) {
         q[row] = acc;
@@ -150,6 +149,149 @@ __global__ void k_ls_direction(int n, const double *__restrict__ z, double *__re
     p[i] = first ? z[i] : z[i] + S->beta * p[i];
 }
 
+// The scalars after an update of the residual (a = ||r||_inf, b = r.z), as the reference's loop sets
+// them between its BLAS calls (pcg_solver.h:276-290).
+__device__ __forceinline__ void ls_after_update(LsScalars &s, double a, double b) {
+    s.rinf = a;
+    s.iter += 1;
+    if (!(a == a) || !(b == b)) {
+        s.status = 1;
+        s.done = 1;
+    } else if (a <= s.tol) {
+        s.converged = 1;
+        s.done = 1;
+    } else if (s.iter >= s.maxit) {
+        s.done = 1;
+    } else {
+        s.beta = b / s.rz;
+        s.rz = b;
+    }
+}
+
+// ---- Small systems (at most LS_FOLD_ROWS rows): an iteration in two launches instead of five, each a
+// launch's boundary and a trip or two to memory (2.3 to 3.8 us) for under 1 us of work.  Every
+// workgroup of the kernel that needs a scalar forms it from the block partials itself, with
+// k_ls_finalize's sums in its order, so both forms give the same bits.  The record S alternates between
+// two slots (all workgroups read one, the first writes the other), the direction between two buffers
+// (its neighbours' new values are formed from the old ones on the fly), and the two kinds of partials
+// have a buffer each.  The limit keeps what the workgroups of the update read together, 16 n^2 / 8192
+// bytes of partials, at 8 MB or 2 us from the L2s; a larger system gains less and less of its time.
+constexpr int LS_FOLD_ROWS = 1 << 16;
+
+// Sums (or max and sum) of nb partials as k_ls_finalize's 1024 threads form them, in LS_BLOCK threads:
+// thread t stands for t, t + 256, t + 512 and t + 768.  Valid in every thread.
+template <bool AMAX>
+__device__ __forceinline__ void ls_fold(const double *__restrict__ partials, int nb, double &a, double &b) {
+    __shared__ double lds[2][16];
+    constexpr int KV = 1024 / LS_BLOCK;
+    const double2 *pp = reinterpret_cast<const double2 *>(partials);
+    double va[KV], vb[KV];
+#pragma unroll
+    for (int k = 0; k < KV; ++k) {
+        va[k] = vb[k] = 0.0;
+        for (int i = (int)threadIdx.x + k * LS_BLOCK; i < nb; i += 1024) {
+            const double2 v = pp[i];
+            va[k] = AMAX ? fmax(va[k], v.x) : va[k] + v.x;
+            if (AMAX) vb[k] += v.y;
+        }
+    }
+    const int w = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < KV; ++k) {
+        if (k * LS_BLOCK >= nb) break;
+        const double wa = AMAX ? shkz::wave_max(va[k]) : shkz::wave_sum(va[k]), wb = AMAX ? shkz::wave_sum(vb[k]) : 0.0;
+        if ((threadIdx.x & 63) == 0) {
+            lds[0][w + k * (LS_BLOCK / 64)] = wa;
+            lds[1][w + k * (LS_BLOCK / 64)] = wb;
+        }
+    }
+    __syncthreads();
+    a = b = 0.0;
+    const int waves = LS_BLOCK / 64 * min(KV, (nb + LS_BLOCK - 1) / LS_BLOCK);
+    for (int i = 0; i < waves; ++i) {
+        a = AMAX ? fmax(a, lds[0][i]) : a + lds[0][i];
+        b += lds[1][i];
+    }
+}
+
+// k_ls_finalize's LS_FIN_UPDATE, k_ls_direction and k_ls_spmv_dot: pnew = z + beta pold, q = A pnew,
+// partials of pnew.q.  S0: the record before the update, S1: after it.  FIRST: pnew = z, no update.
+template <bool FIRST>
+__global__ __launch_bounds__(LS_BLOCK) void k_ls_direction_spmv(int n, const int *__restrict__ rowptr,
+                                                                const int *__restrict__ col,
+                                                                const double *__restrict__ val,
+                                                                const double *__restrict__ z,
+                                                                const double *__restrict__ pold,
+                                                                double *__restrict__ pnew, double *__restrict__ q,
+                                                                const LsScalars *S0, LsScalars *S1,
+                                                                const double *__restrict__ upd, int nb_upd,
+                                                                double *__restrict__ pq) {
+    LsScalars s = *S0;
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    if (s.done) {
+        if (!FIRST && first) *S1 = s;
+        return;
+    }
+    const int row = blockIdx.x * LS_ROWS + (threadIdx.x / LS_LANES);
+    const int lane = threadIdx.x % LS_LANES;
+    const int e0 = row < n ? rowptr[row] : 0, e1 = row < n ? rowptr[row + 1] : 0;
+    if (!FIRST) {
+        double a, b;
+        ls_fold<true>(upd, nb_upd, a, b);
+        ls_after_update(s, a, b);
+        if (first) *S1 = s;
+        if (s.done) return;
+    }
+    const double beta = s.beta;
+    double acc = 0.0;
+    for (int e = e0 + lane; e < e1; e += LS_LANES) {
+        const int c = col[e];
+        acc += val[e] * (FIRST ? z[c] : z[c] + beta * pold[c]);
+    }
+    acc = ls_row_sum(acc);
+    double part = 0.0;
+    if (row < n && lane == 0) {
+        const double p = FIRST ? z[row] : z[row] + beta * pold[row];
+        pnew[row] = p;
+        q[row] = acc;
+        part = p * acc;
+    }
+    ls_block_partials<false>(part, 0.0, pq);
+}
+
+// k_ls_finalize's LS_FIN_PQ and k_ls_update.
+__global__ __launch_bounds__(LS_BLOCK) void k_ls_update_folded(int n, double *__restrict__ x, double *__restrict__ r,
+                                                               double *__restrict__ z, const double *__restrict__ p,
+                                                               const double *__restrict__ q,
+                                                               const double *__restrict__ idiag, const LsScalars *S,
+                                                               const double *__restrict__ pq, int nb_pq,
+                                                               double *__restrict__ upd) {
+    if (S->done) return;
+    const int i = blockIdx.x * LS_BLOCK + threadIdx.x;
+    double xv = 0.0, pv = 0.0, qv = 0.0, r0 = 0.0, d = 0.0;
+    if (i < n) {
+        xv = x[i];
+        pv = p[i];
+        qv = q[i];
+        r0 = r[i];
+        if (idiag) d = idiag[i];
+    }
+    double sum, unused;
+    ls_fold<false>(pq, nb_pq, sum, unused);
+    const double a = S->rz / sum;
+    double mx = 0.0, rz = 0.0;
+    if (i < n) {
+        x[i] = xv + a * pv;
+        const double rv = r0 - a * qv;
+        r[i] = rv;
+        const double zi = idiag ? d * rv : rv;
+        if (idiag) z[i] = zi;
+        mx = fabs(rv);
+        rz = rv * zi;
+    }
+    ls_block_partials<true>(mx, rz, upd);
+}
+
 enum { LS_FIN_INIT = 0, LS_FIN_PQ = 1, LS_FIN_UPDATE = 2 };
 
 // One block combines the partials of nb blocks in block order and updates the scalars, as the
@@ -164,8 +306,8 @@ __global__ __launch_bounds__(1024) void k_ls_finalize(const double *__restrict__
         a = amax ? fmax(a, partials[2 * i]) : a + partials[2 * i];
         b += partials[2 * i + 1];
     }
-    a = amax ? ls_wave_max(a) : ls_wave_sum(a);
-    b = ls_wave_sum(b);
+    a = amax ? shkz::wave_max(a) : shkz::wave_sum(a);
+    b = shkz::wave_sum(b);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0) {
         lds[0][wid] = a;
@@ -202,20 +344,7 @@ __global__ __launch_bounds__(1024) void k_ls_finalize(const double *__restrict__
     } else if (op == LS_FIN_PQ) {
         s.alpha = s.rz / a;
     } else {
-        s.rinf = a;
-        s.iter += 1;
-        if (!(a == a) || !(b == b)) {
-            s.status = 1;
-            s.done = 1;
-        } else if (a <= s.tol) {
-            s.converged = 1;
-            s.done = 1;
-        } else if (s.iter >= s.maxit) {
-            s.done = 1;
-        } else {
-            s.beta = b / s.rz;
-            s.rz = b;
-        }
+        ls_after_update(s, a, b);
     }
 }
 
@@ -235,9 +364,9 @@ struct shkz_linsolver {
     struct Buf {
         void *p = nullptr;
         size_t cap = 0;
-    } rowptr, col, val, b, x, r, z, p, q, idiag, partials, scalars;
+    } rowptr, col, val, b, x, r, z, p, p2, q, idiag, partials, partials2, scalars;
     LsScalars *host_s = nullptr;
-    hipGraphExec_t exec = nullptr;
+    hipGraphExec_t exec = nullptr, exec_many = nullptr;  // the shortest replay and a longer one
     std::vector<const void *> exec_key;
     int exec_n = -1, exec_prec = -1;
 };
@@ -277,13 +406,15 @@ struct LsArrays {
     const int *rowptr, *col;
     const double *val, *b;
     double *x, *r, *z, *p, *q, *idiag, *partials;
-    LsScalars *S;
+    double *p2, *partials2;  // small systems (LS_FOLD_ROWS): the other direction and the p.q partials
+    LsScalars *S;            // two records
 };
 
-// The solve on device arrays (b filled); x receives the result.  With `graph`, one iteration is
-// captured once into a hipGraph kept by the solver and replayed; without, the same kernels are
-// launched directly (same launch shapes, so the same results).  Scalars come back through the
-// solver's pinned buffer.
+// The solve on device arrays (b filled); x receives the result.  With `graph`, the iterations are
+// replayed from two hipGraphs kept by the solver (the shortest step and several of them in one launch:
+// a launch costs the host about as much as an iteration takes); without, the same kernels are launched
+// directly (same launch shapes, so the same results).  Scalars come back through the solver's pinned
+// buffer.
 int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, const shkz_linsolve_params *prm,
                     shkz_linsolve_result *res, bool graph) {
     const int *rp = D.rowptr, *cl = D.col;
@@ -295,32 +426,59 @@ int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, 
     double *zz = jacobi ? z : r;  // without a preconditioner z is r itself
     const unsigned nb_v = blocks_of(n, LS_BLOCK), nb_m = blocks_of(n, LS_ROWS);
     const int maxit = prm->max_iterations > 0 ? prm->max_iterations : 30000;
-    if (jacobi) k_ls_idiag<<<nb_v, LS_BLOCK, 0, s>>>(n, rp, cl, vl, id);
-    k_ls_init<<<nb_v, LS_BLOCK, 0, s>>>(n, b, x, r, z, M, part);
-    k_ls_finalize<<<1, 1024, 0, s>>>(part, (int)nb_v, S, LS_FIN_INIT, prm->residual, maxit);
-    k_ls_direction<<<nb_v, LS_BLOCK, 0, s>>>(n, zz, p, S, 1);
-    auto iteration = [&]() {
-        k_ls_spmv_dot<<<nb_m, LS_BLOCK, 0, s>>>(n, rp, cl, vl, p, q, S, part);
-        k_ls_finalize<<<1, 1024, 0, s>>>(part, (int)nb_m, S, LS_FIN_PQ, 0.0, 0);
-        k_ls_update<<<nb_v, LS_BLOCK, 0, s>>>(n, x, r, z, p, q, M, S, part);
-        k_ls_finalize<<<1, 1024, 0, s>>>(part, (int)nb_v, S, LS_FIN_UPDATE, 0.0, 0);
-        k_ls_direction<<<nb_v, LS_BLOCK, 0, s>>>(n, zz, p, S, 0);
+    const bool fold = n <= LS_FOLD_ROWS;
+    // a launch on the stream, or a node of the graph under construction
+    hipGraph_t building = nullptr;
+    hipGraphNode_t last = nullptr;
+    hipError_t err = hipSuccess;
+    auto go = [&](unsigned blocks, unsigned threads, auto kernel, auto... args) {
+        if (!building) kernel<<<blocks, threads, 0, s>>>(args...);
+        else if (err == hipSuccess) err = shkz::add_kernel_node(building, &last, dim3(blocks), dim3(threads), kernel, args...);
     };
+    if (jacobi) go(nb_v, LS_BLOCK, k_ls_idiag, n, rp, cl, vl, id);
+    go(nb_v, LS_BLOCK, k_ls_init, n, b, x, r, z, M, part);
+    go(1, 1024, k_ls_finalize, part, (int)nb_v, S, (int)LS_FIN_INIT, prm->residual, maxit);
+    if (fold)
+        go(nb_m, LS_BLOCK, k_ls_direction_spmv<true>, n, rp, cl, vl, zz, p, p, q, S, S, part, (int)nb_v, D.partials2);
+    else
+        go(nb_v, LS_BLOCK, k_ls_direction, n, zz, p, S, 1);
+    // one step: an iteration, or with the scalars folded two, which alternate the records and directions
+    auto step = [&]() {
+        if (fold) {
+            for (int k = 0; k < 2; ++k) {
+                double *const pc = k ? D.p2 : p, *const pn = k ? p : D.p2;
+                go(nb_v, LS_BLOCK, k_ls_update_folded, n, x, r, z, pc, q, M, S + k, D.partials2, (int)nb_m, part);
+                go(nb_m, LS_BLOCK, k_ls_direction_spmv<false>, n, rp, cl, vl, zz, pc, pn, q, S + k, S + (k ^ 1), part,
+                   (int)nb_v, D.partials2);
+            }
+            return;
+        }
+        go(nb_m, LS_BLOCK, k_ls_spmv_dot, n, rp, cl, vl, p, q, S, part);
+        go(1, 1024, k_ls_finalize, part, (int)nb_m, S, (int)LS_FIN_PQ, 0.0, 0);
+        go(nb_v, LS_BLOCK, k_ls_update, n, x, r, z, p, q, M, S, part);
+        go(1, 1024, k_ls_finalize, part, (int)nb_v, S, (int)LS_FIN_UPDATE, 0.0, 0);
+        go(nb_v, LS_BLOCK, k_ls_direction, n, zz, p, S, 0);
+    };
+    const int per_step = fold ? 2 : 1, many = 8;  // iterations of a step, steps of the longer graph
     if (graph) {
-        // one captured iteration, reused while the arrays and sizes stay the same
-        std::vector<const void *> key = {rp, cl, vl, x, r, z, p, q, id, part, S};
+        // reused while the arrays and sizes stay the same
+        std::vector<const void *> key = {rp, cl, vl, x, r, z, p, q, id, part, S, D.p2, D.partials2};
         if (!L->exec || L->exec_key != key || L->exec_n != n || L->exec_prec != (int)jacobi) {
-            if (L->exec) (void)hipGraphExecDestroy(L->exec);
-            L->exec = nullptr;
-            hipGraph_t g = nullptr;
-            LS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            iteration();
-            LS_HIP(hipStreamEndCapture(s, &g));
-            const hipError_t e = hipGraphInstantiate(&L->exec, g, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(g);
-            if (e != hipSuccess) {
-                L->exec = nullptr;
-                return shkz_fail(SHKZ_ERR_DEVICE, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
+            for (hipGraphExec_t *e : {&L->exec, &L->exec_many}) {
+                if (*e) (void)hipGraphExecDestroy(*e);
+                *e = nullptr;
+            }
+            for (int k = 0; k < 2; ++k) {
+                LS_HIP(hipGraphCreate(&building, 0));
+                last = nullptr;
+                for (int i = 0; i < (k ? many : 1); ++i) step();
+                hipGraphExec_t made = nullptr;
+                if (err == hipSuccess) err = hipGraphInstantiateWithFlags(&made, building, 0);
+                (void)hipGraphDestroy(building);
+                building = nullptr;
+                if (err != hipSuccess)
+                    return shkz_fail(SHKZ_ERR_DEVICE, "building an iteration's graph failed: %s", hipGetErrorString(err));
+                (k ? L->exec_many : L->exec) = made;
             }
             L->exec_key = key;
             L->exec_n = n;
@@ -341,9 +499,11 @@ int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, 
             if (rate > 0 && rate < 1) next = (int)std::ceil(std::log(h.tol / h.rinf) / std::log(rate));
         }
         chunk = std::max(1, std::min({next, h.maxit - h.iter, 256}));
-        for (int it = 0; it < chunk; ++it) {
+        int steps = (chunk + per_step - 1) / per_step;
+        for (; graph && steps >= many; steps -= many) LS_HIP(hipGraphLaunch(L->exec_many, s));
+        for (; steps > 0; --steps) {
             if (graph) LS_HIP(hipGraphLaunch(L->exec, s));
-            else iteration();
+            else step();
         }
     }
     LS_HIP(hipGetLastError());
@@ -357,12 +517,13 @@ int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, 
 
 // Scratch of the allocation-free entry point: a fixed device array (each GPU the library runs on
 // holds its own copy until the process ends).  Layout in doubles: r, z, p, q, idiag (each
-// SHKZ_LS_NOALLOC_MAX_ROWS), the block partials (two per SpMV block of the largest system), then
-// the scalar record.
+// SHKZ_LS_NOALLOC_MAX_ROWS), the block partials (two per SpMV block of the largest system), the second
+// direction and p.q partials of the small systems, then the two scalar records.
 constexpr size_t NA_ROWS = SHKZ_LS_NOALLOC_MAX_ROWS;
 constexpr size_t NA_PARTIALS = 2 * ((NA_ROWS + LS_ROWS - 1) / LS_ROWS);
-constexpr size_t NA_SCALARS = (sizeof(LsScalars) + sizeof(double) - 1) / sizeof(double);
-constexpr size_t NA_DOUBLES = 5 * NA_ROWS + NA_PARTIALS + NA_SCALARS;
+constexpr size_t NA_PARTIALS2 = 2 * ((LS_FOLD_ROWS + LS_ROWS - 1) / LS_ROWS);
+constexpr size_t NA_SCALARS = 2 * ((sizeof(LsScalars) + sizeof(double) - 1) / sizeof(double));
+constexpr size_t NA_DOUBLES = 5 * NA_ROWS + NA_PARTIALS + LS_FOLD_ROWS + NA_PARTIALS2 + NA_SCALARS;
 static_assert(NA_ROWS % LS_ROWS == 0 && LS_BLOCK % LS_ROWS == 0, "partials cover both kernels' blocks");
 static __device__ __align__(256) double scratch[NA_DOUBLES];
 
@@ -431,8 +592,9 @@ void shkz_linsolver_destroy(shkz_linsolver *L) {
     (void)hipSetDevice(L->device);
     (void)hipStreamSynchronize(L->stream);
     if (L->exec) (void)hipGraphExecDestroy(L->exec);
-    for (shkz_linsolver::Buf *b : {&L->rowptr, &L->col, &L->val, &L->b, &L->x, &L->r, &L->z, &L->p, &L->q, &L->idiag,
-                                   &L->partials, &L->scalars})
+    if (L->exec_many) (void)hipGraphExecDestroy(L->exec_many);
+    for (shkz_linsolver::Buf *b : {&L->rowptr, &L->col, &L->val, &L->b, &L->x, &L->r, &L->z, &L->p, &L->p2, &L->q,
+                                   &L->idiag, &L->partials, &L->partials2, &L->scalars})
         if (b->p) (void)hipFree(b->p);
     if (L->host_s) (void)hipHostFree(L->host_s);
     (void)hipStreamDestroy(L->stream);
@@ -479,7 +641,11 @@ int shkz_linsolve_csr(shkz_linsolver *L, int64_t n, const int64_t *rowptr, const
     for (shkz_linsolver::Buf *bb : {&L->b, &L->x, &L->r, &L->z, &L->p, &L->q, &L->idiag})
         LS_TRY(ls_get(*bb, n * sizeof(double), &pp));
     LS_TRY(ls_get(L->partials, 2 * sizeof(double) * std::max(blocks_of(n, LS_BLOCK), blocks_of(n, LS_ROWS)), &pp));
-    LS_TRY(ls_get(L->scalars, sizeof(LsScalars), &pp));
+    if (n <= LS_FOLD_ROWS) {
+        LS_TRY(ls_get(L->p2, n * sizeof(double), &pp));
+        LS_TRY(ls_get(L->partials2, 2 * sizeof(double) * blocks_of(n, LS_ROWS), &pp));
+    }
+    LS_TRY(ls_get(L->scalars, 2 * sizeof(LsScalars), &pp));
     LS_HIP(hipMemcpyAsync(L->rowptr.p, rp32.data(), (n + 1) * sizeof(int), hipMemcpyHostToDevice, L->stream));
     if (nnz) {
         LS_HIP(hipMemcpyAsync(L->col.p, col32.data(), nnz * sizeof(int), hipMemcpyHostToDevice, L->stream));
@@ -490,7 +656,8 @@ int shkz_linsolve_csr(shkz_linsolver *L, int64_t n, const int64_t *rowptr, const
     const double t1 = now_ms();
     const LsArrays D{(const int *)L->rowptr.p, (const int *)L->col.p, (const double *)L->val.p, (const double *)L->b.p,
                      (double *)L->x.p, (double *)L->r.p, (double *)L->z.p, (double *)L->p.p, (double *)L->q.p,
-                     (double *)L->idiag.p, (double *)L->partials.p, (LsScalars *)L->scalars.p};
+                     (double *)L->idiag.p, (double *)L->partials.p, (double *)L->p2.p, (double *)L->partials2.p,
+                     (LsScalars *)L->scalars.p};
     const int rc = ls_solve_device(L, L->stream, D, (int)n, prm, result, true);
     LS_HIP(hipMemcpyAsync(x, L->x.p, n * sizeof(double), hipMemcpyDeviceToHost, L->stream));
     LS_HIP(hipStreamSynchronize(L->stream));
@@ -526,7 +693,9 @@ int shkz_linsolve_csr_device_noalloc(shkz_linsolver *L, int32_t n, const int32_t
     LS_TRY(noalloc_scratch(L->device, &base));
     const hipStream_t s = (hipStream_t)stream;
     const LsArrays D{rowptr, col, val, b, x, base, base + NA_ROWS, base + 2 * NA_ROWS, base + 3 * NA_ROWS,
-                     base + 4 * NA_ROWS, base + 5 * NA_ROWS, (LsScalars *)(base + 5 * NA_ROWS + NA_PARTIALS)};
+                     base + 4 * NA_ROWS, base + 5 * NA_ROWS, base + 5 * NA_ROWS + NA_PARTIALS,
+                     base + 5 * NA_ROWS + NA_PARTIALS + LS_FOLD_ROWS,
+                     (LsScalars *)(base + 5 * NA_ROWS + NA_PARTIALS + LS_FOLD_ROWS + NA_PARTIALS2)};
     const int rc = ls_solve_device(L, s, D, (int)n, prm, result, false);
     result->t_solve = now_ms() - t0;
     return rc;

@@ -126,3 +126,27 @@ def test_pure_neumann_consistent_system(ls):
     x, r = ls.solve(A["rowptr"], A["col"], A["val"], b, residual=1e-10)
     assert r.converged
     assert np.abs(b - O.spmv(A, x)).max() <= 1e-9 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("jacobi", [False, True])
+@pytest.mark.parametrize("n", [1, 31, 33, 256, 257, 8193, 65536, 65537])
+def test_sizes_at_the_edges_of_blocks_and_of_the_folded_iteration(ls, n, jacobi):
+    """Tridiagonal systems (4 on the diagonal, -1 beside it: condition number below 3, so a relative
+    residual of 1e-12 bounds the relative error by about 3e-12) at the sizes where the last block is
+    partial or the two-launch iteration ends."""
+    from scipy.linalg import solveh_banded
+    say(f"tridiagonal n={n} jacobi={jacobi}")
+    rng = np.random.default_rng(n)
+    b = rng.normal(size=n)
+    i = np.arange(n)
+    rows = np.concatenate([i, i[1:], i[:-1]])
+    cols = np.concatenate([i, i[1:] - 1, i[:-1] + 1])
+    vals = np.concatenate([np.full(n, 4.0), np.full(2 * (n - 1), -1.0)])
+    order = np.lexsort((cols, rows))
+    rowptr = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))])
+    x, r = ls.solve(rowptr, cols[order], vals[order], b, residual=1e-12,
+                    preconditioner=S.LS_JACOBI if jacobi else S.LS_NONE)
+    assert r.converged and r.iterations <= 40
+    ab = np.vstack([np.concatenate([[0.0], np.full(n - 1, -1.0)]), np.full(n, 4.0)])
+    ref = solveh_banded(ab, b)
+    assert np.abs(x - ref).max() <= 1e-11 * np.abs(ref).max()
