@@ -2436,8 +2436,13 @@ __global__ __launch_bounds__(1024) void k_smooth_k(LevelDesc L, OpDesc<T> A, con
     using C = SmoothK<T, GH>;
     constexpr int R = C::R, NR = C::NR, CPT = C::CPT;
     using PT = ProTile<T, GH>;
+    // The cells' high couplings are other cells' low ones: exchanged through LDS, in arrays of their own
+    // (the residual reads them again) or, where those would not fit (FP64 at K = 4: 160 KB), one axis after
+    // another through the second z buffer.
+    constexpr bool STAGED = sizeof(T) * 5 * NR > 128 * 1024;
+    static_assert(!(STAGED && RES), "the residual reads the couplings from LDS");
     __shared__ T zs[2][NR];
-    __shared__ T gxs[NR], gys[NR], gzs[NR];
+    __shared__ T gxs[STAGED ? 1 : NR], gys[STAGED ? 1 : NR], gzs[STAGED ? 1 : NR];
     __shared__ T ctile[PRO ? PT::N : 1];
     __shared__ int nb27[27];
     __shared__ int pb[8];
@@ -2488,11 +2493,13 @@ __global__ __launch_bounds__(1024) void k_smooth_k(LevelDesc L, OpDesc<T> A, con
         __syncthreads();
     }
     T rid[CPT], rr[CPT];
+    T gxm[CPT], gxp[CPT], gym[CPT], gyp[CPT], gzm[CPT], gzp[CPT], zr[CPT];
 #pragma unroll
     for (int q = 0; q < CPT; ++q) {
         const int e = t + q * C::THREADS;
         rid[q] = 0;
         rr[q] = 0;
+        gxm[q] = gxp[q] = gym[q] = gyp[q] = gzm[q] = gzp[q] = zr[q] = T(0);
         if (e >= NR) continue;
         const int a = e / (R * R), b = (e / R) % R, c = e % R;
         // cube offset a is brick-local cell a - GH, in brick (-1, 0 or +1) + local (0..7)
@@ -2525,28 +2532,49 @@ __global__ __launch_bounds__(1024) void k_smooth_k(LevelDesc L, OpDesc<T> A, con
                 z0 = z0 + v;
             }
         }
-        gxs[e] = g0;
-        gys[e] = g1;
-        gzs[e] = g2;
+        gxm[q] = g0;
+        gym[q] = g1;
+        gzm[q] = g2;
+        zr[q] = z0;
         zs[0][e] = z0;
+        if constexpr (!STAGED) {
+            gxs[e] = g0;
+            gys[e] = g1;
+            gzs[e] = g2;
+        }
     }
-    __syncthreads();
     // each thread keeps its cells' six couplings and own value in registers: a sweep reads only
     // the six neighbour values from LDS
-    T gxm[CPT], gxp[CPT], gym[CPT], gyp[CPT], gzm[CPT], gzp[CPT], zr[CPT];
+    auto high = [&](const T *low, T *own, int axis) {
 #pragma unroll
-    for (int q = 0; q < CPT; ++q) {
-        const int e = t + q * C::THREADS;
-        gxm[q] = gxp[q] = gym[q] = gyp[q] = gzm[q] = gzp[q] = zr[q] = T(0);
-        if (e >= NR) continue;
-        const int a = e / (R * R), b = (e / R) % R, c = e % R;
-        gxm[q] = gxs[e];
-        gym[q] = gys[e];
-        gzm[q] = gzs[e];
-        gxp[q] = a < R - 1 ? gxs[e + R * R] : T(0);
-        gyp[q] = b < R - 1 ? gys[e + R] : T(0);
-        gzp[q] = c < R - 1 ? gzs[e + 1] : T(0);
-        zr[q] = zs[0][e];
+        for (int q = 0; q < CPT; ++q) {
+            const int e = t + q * C::THREADS;
+            if (e >= NR) continue;
+            const int a = e / (R * R), b = (e / R) % R, c = e % R;
+            if (axis == 0) own[q] = a < R - 1 ? low[e + R * R] : T(0);
+            if (axis == 1) own[q] = b < R - 1 ? low[e + R] : T(0);
+            if (axis == 2) own[q] = c < R - 1 ? low[e + 1] : T(0);
+        }
+    };
+    if constexpr (STAGED) {
+        auto stage = [&](const T *low, T *own, int axis) {
+#pragma unroll
+            for (int q = 0; q < CPT; ++q) {
+                const int e = t + q * C::THREADS;
+                if (e < NR) zs[1][e] = low[q];
+            }
+            __syncthreads();
+            high(zs[1], own, axis);
+            __syncthreads();
+        };
+        stage(gxm, gxp, 0);
+        stage(gym, gyp, 1);
+        stage(gzm, gzp, 2);
+    } else {
+        __syncthreads();
+        high(gxs, gxp, 0);
+        high(gys, gyp, 1);
+        high(gzs, gzp, 2);
     }
 #pragma unroll 1
     for (int s = 0; s < K; ++s) {

@@ -673,7 +673,17 @@ static int final_slot(int pre, int post, bool multi_pre, bool multi_post, bool f
 // Sweep counts k_smooth_k is built for (its cube of cells must fit LDS).
 template <class T>
 static bool smooth_k_supported(int k) {
-    return k >= 2 && k <= (sizeof(T) == 4 ? 5 : 3);
+    return k >= 2 && k <= (sizeof(T) == 4 ? 5 : 4);
+}
+
+// Levels that smooth with one multi-sweep launch per step: up to max_bricks stored bricks, and in FP64
+// with four sweeps (90 registers, 16 wavefronts: one workgroup per CU) no more than the CUs: on 224
+// bricks the pre-smoothing takes 10 us in one launch against 12 us sweep by sweep, the post-smoothing
+// with the prolongation 12 us against 18 us; a second round of workgroups would lose.
+template <class T>
+static bool smooth_k_level(int nbricks, int max_bricks, int k) {
+    if (sizeof(T) == 8 && k == 4) max_bricks = std::min(max_bricks, 256);
+    return nbricks <= max_bricks && smooth_k_supported<T>(k);
 }
 
 // Sweep counts k_smooth_k's residual variant is built for (one more ghost layer in LDS).
@@ -705,8 +715,8 @@ static void smooth_k(Launcher &K, int l, int k, bool from_zero, const LevelDesc 
     if (zcoarse && !from_zero) {
         if (k == 2) smooth_k_go<T, 2, 0, 0, 1>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr, zcoarse, coarse_unknowns);
         if (k == 3) smooth_k_go<T, 3, 0, 0, 1>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr, zcoarse, coarse_unknowns);
+        if (k == 4) smooth_k_go<T, 4, 0, 0, 1>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr, zcoarse, coarse_unknowns);
         if constexpr (sizeof(T) == 4) {
-            if (k == 4) smooth_k_go<T, 4, 0, 0, 1>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr, zcoarse, coarse_unknowns);
             if (k == 5) smooth_k_go<T, 5, 0, 0, 1>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr, zcoarse, coarse_unknowns);
         }
         return;
@@ -728,12 +738,13 @@ static void smooth_k(Launcher &K, int l, int k, bool from_zero, const LevelDesc 
         if (from_zero) smooth_k_go<T, 3, 1, 0>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr);
         else smooth_k_go<T, 3, 0, 0>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr);
         break;
+    case 4:
+        if (from_zero) smooth_k_go<T, 4, 1, 0>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr);
+        else smooth_k_go<T, 4, 0, 0>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr);
+        break;
     default:
         if constexpr (sizeof(T) == 4) {
-            if (k == 4) {
-                if (from_zero) smooth_k_go<T, 4, 1, 0>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr);
-                else smooth_k_go<T, 4, 0, 0>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr);
-            } else if (k == 5) {
+            if (k == 5) {
                 if (from_zero) smooth_k_go<T, 5, 1, 0>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr);
                 else smooth_k_go<T, 5, 0, 0>(K, l, g, L, A, id, rhs, zin, zout, om, Q, nullptr);
             }
@@ -803,9 +814,8 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
     // with the brick-local smoother every level uses it, whatever its size
     std::vector<char> mpre(nl, 0), mpost(nl, 0);
     for (int l = 1; l < nl && !brick_smoother; ++l) {
-        const bool small = C->levels[l].nbricks <= P.multi_max_bricks;
-        mpre[l] = small && smooth_k_supported<T>(P.pre_c);
-        mpost[l] = small && smooth_k_supported<T>(P.post_c);
+        mpre[l] = smooth_k_level<T>(C->levels[l].nbricks, P.multi_max_bricks, P.pre_c);
+        mpost[l] = smooth_k_level<T>(C->levels[l].nbricks, P.multi_max_bricks, P.post_c);
     }
     for (int l = 0; l < nl; ++l) {
         LevelHost &L = C->levels[l];

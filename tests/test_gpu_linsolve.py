@@ -148,5 +148,5 @@ def test_sizes_at_the_edges_of_blocks_and_of_the_folded_iteration(ls, n, jacobi)
                     preconditioner=S.LS_JACOBI if jacobi else S.LS_NONE)
     assert r.converged and r.iterations <= 40
     ab = np.vstack([np.concatenate([[0.0], np.full(n - 1, -1.0)]), np.full(n, 4.0)])
-    ref = solveh_banded(ab, b)
+    ref = solveh_banded(ab, b) if n > 1 else b / 4.0
     assert np.abs(x - ref).max() <= 1e-11 * np.abs(ref).max()
