@@ -1055,76 +1055,43 @@ __global__ __launch_bounds__(BLOCK) void k_smooth2(LevelDesc L, OpDesc<T> A, con
     z[c] = out;
 }
 
-// zout = (1 - omega) zin + omega idiag (rhs + offdiag(zin)).  DOT: also rhs.zout partials (the
-// finest level's last post-smoothing sweep yields r.z of the preconditioned CG for free).
-template <class T, int DOT>
-__device__ __forceinline__ void jacobi_brick(const LevelDesc &L, const OpDesc<T> &A, const T *__restrict__ idiag,
-                                             const T *__restrict__ rhs, const T *__restrict__ zin,
-                                             T *__restrict__ zout, T omega, const RedBuf &R, int br, const BrickMeta &m,
-                                             double *lds);
-
-// Persistent form: the grid holds at most PERSIST_BLOCKS workgroups, each looping over virtual
-// block ids vb = blockIdx.x + k * gridDim.x (gridDim.x a multiple of 8, so vb keeps its XCD).
-constexpr int PERSIST_BLOCKS = 1024;  // 4 resident 512-thread workgroups on each of 256 CUs
-
-template <class T, int FINEST, int DOT>
-__global__ __launch_bounds__(BLOCK) void k_jacobi(LevelDesc L, OpDesc<T> A, const T *__restrict__ idiag,
-                                                  const T *__restrict__ rhs, const T *__restrict__ zin,
-                                                  T *__restrict__ zout, T omega, Gate Q, RedBuf R, int nvirt) {
+// zout = (1 - omega) zin + omega idiag (rhs + offdiag(zin)) with the rhs.zout partial of each brick: the
+// finest level's last post-smoothing sweep of an FP64 cycle yields r.z of the preconditioned CG for free.
+// One brick per workgroup (its reduction costs two barriers per brick), one cell per thread: the
+// partial keeps the order of the sum over the brick.
+template <class T>
+__global__ __launch_bounds__(BLOCK) void k_jacobi_dot(LevelDesc L, OpDesc<T> A, const T *__restrict__ idiag,
+                                                      const T *__restrict__ rhs, const T *__restrict__ zin,
+                                                      T *__restrict__ zout, T omega, Gate Q, RedBuf R) {
     __shared__ double lds[32];
-    if (DOT) {  // one brick per workgroup (its reduction costs two barriers per brick)
-        const int br = brick_or_idle(L);
-        if (br < 0) return;
-        const BrickMeta m = L.meta[br];
-        if (all_done(Q) || skip_smooth(Q, L, m)) return;
-        jacobi_brick<T, DOT>(L, A, idiag, rhs, zin, zout, omega, R, br, m, lds);
-        return;
-    }
-    if (all_done(Q)) return;
-    for (int vb = blockIdx.x; vb < nvirt; vb += gridDim.x) {
-        const int br = xcd_brick(vb, nvirt);
-        if (br >= L.nbricks) continue;
-        const BrickMeta m = L.meta[br];
-        if (skip_smooth(Q, L, m)) continue;
-        jacobi_brick<T, DOT>(L, A, idiag, rhs, zin, zout, omega, R, br, m, lds);
-    }
-}
-
-template <class T, int DOT>
-__device__ __forceinline__ void jacobi_brick(const LevelDesc &L, const OpDesc<T> &A, const T *__restrict__ idiag,
-                                             const T *__restrict__ rhs, const T *__restrict__ zin,
-                                             T *__restrict__ zout, T omega, const RedBuf &R, int br, const BrickMeta &m,
-                                             double *lds) {
+    const int br = brick_or_idle(L);
+    if (br < 0) return;
+    const BrickMeta m = L.meta[br];
+    if (all_done(Q) || skip_smooth(Q, L, m)) return;
     const int t = threadIdx.x;
     const long c = (long)br * BRICK_CELLS + t;
-    T out = 0;
-    double part = 0.0;
+    long idx[6];
+    nb_index(nbrs_of(m, br), t, idx);
+    const T r = rhs[c];
+    T out;
+    double part;
     if (m.flags & BM_UNIFORM) {
         const UniT<T> u = uni_load<T>(L, br);
-        long idx[6];
-        nb_index(nbrs_of(m, br), t, idx);
-        const T r = rhs[c];
         out = (T(1) - omega) * zin[c] + omega * u.id * (r + offdiag_uniform(u.g, zin, idx));
-        if (DOT) part = (double)r * (double)out;
+        part = (double)r * (double)out;
     } else {
         // every load is issued before the unknown test (the values of other cells are discarded)
-        const Nbrs N = nbrs_of(m, br);
-        long idx[6];
-        nb_index(N, t, idx);
         const T id = idiag[c];
-        const T r = rhs[c];
         const T v = (T(1) - omega) * zin[c] + omega * id * (r + offdiag_sum(A, zin, c, idx));
         out = id > 0 ? v : T(0);
-        if (DOT) part = id > 0 ? (double)r * (double)v : 0.0;
+        part = id > 0 ? (double)r * (double)v : 0.0;
     }
     zout[c] = out;
-    if (DOT) {
-        part = block_sum(part, lds);
-        store_partials(R, br, part, 0.0);
-    }
+    part = block_sum(part, lds);
+    store_partials(R, br, part, 0.0);
 }
 
-// ---- FP32 sweeps on cell rows: four consecutive cells (one float4 along z) per thread, 128
+// ---- Sweeps on cell rows: four consecutive cells (one float4 along z) per thread, 128
 // threads per brick.  Lane q of a brick holds the cells (q >> 4, (q >> 1) & 7, 4h .. 4h + 3) with
 // h = q & 1; the two lanes of a row are neighbours in the wavefront and swap their edge values, so
 // only the row's two end cells read a value across the brick's z faces.  A quarter of the load
@@ -1240,47 +1207,49 @@ __device__ __forceinline__ Row4Coef<T> row4_coef(const OpDesc<T> &A, const Row4N
 
 // jacobi_brick on the lane's four cells (same per-cell arithmetic); DOT adds rhs.zout of the
 // unknowns, in cell order, to part.
-template <int DOT>
-__device__ __forceinline__ void jacobi_row4(const LevelDesc &L, const OpDesc<float> &A, const float *__restrict__ idiag,
-                                            const float *__restrict__ rhs, const float *__restrict__ zin,
-                                            float *__restrict__ zout, float omega, int br, const BrickMeta &m, int q,
+template <int DOT, class T>
+__device__ __forceinline__ void jacobi_row4(const LevelDesc &L, const OpDesc<T> &A, const T *__restrict__ idiag,
+                                            const T *__restrict__ rhs, const T *__restrict__ zin,
+                                            T *__restrict__ zout, T omega, int br, const BrickMeta &m, int q,
                                             double &part) {
     const Row4Nbrs N = row4_nbrs(m, br, q);
-    const Row4Vals<float> z = row4_vals(zin, N);
-    float r[4], out[4];
-    unpack4(ld4(rhs, N.c), r);
+    const Row4Vals<T> z = row4_vals(zin, N);
+    T r[4], out[4];
+    load4(rhs, N.c, r);
     if (m.flags & BM_UNIFORM) {
-        const UniT<float> u = uni_load<float>(L, br);
+        const UniT<T> u = uni_load<T>(L, br);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const float off = u.g * z.xm[j] + u.g * z.xp[j] + u.g * z.ym[j] + u.g * z.yp[j] + u.g * z.zm[j] +
+            const T off = u.g * z.xm[j] + u.g * z.xp[j] + u.g * z.ym[j] + u.g * z.yp[j] + u.g * z.zm[j] +
                               u.g * z.zp[j];
-            out[j] = (1.0f - omega) * z.c[j] + omega * u.id * (r[j] + off);
+            out[j] = (T(1) - omega) * z.c[j] + omega * u.id * (r[j] + off);
             if (DOT) part += (double)r[j] * (double)out[j];
         }
     } else {
-        const Row4Coef<float> g = row4_coef(A, N);
-        float id[4];
-        unpack4(ld4(idiag, N.c), id);
+        const Row4Coef<T> g = row4_coef(A, N);
+        T id[4];
+        load4(idiag, N.c, id);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const float off = g.gxm[j] * z.xm[j] + g.gxp[j] * z.xp[j] + g.gym[j] * z.ym[j] + g.gyp[j] * z.yp[j] +
+            const T off = g.gxm[j] * z.xm[j] + g.gxp[j] * z.xp[j] + g.gym[j] * z.ym[j] + g.gyp[j] * z.yp[j] +
                               g.gzm[j] * z.zm[j] + g.gzp[j] * z.zp[j];
-            const float v = (1.0f - omega) * z.c[j] + omega * id[j] * (r[j] + off);
-            out[j] = id[j] > 0 ? v : 0.0f;
+            const T v = (T(1) - omega) * z.c[j] + omega * id[j] * (r[j] + off);
+            out[j] = id[j] > 0 ? v : T(0);
             if (DOT) part += id[j] > 0 ? (double)r[j] * (double)v : 0.0;
         }
     }
-    *reinterpret_cast<float4 *>(zout + N.c) = make_float4(out[0], out[1], out[2], out[3]);
+    store4(zout, N.c, out);
 }
 
-// FP32 sweep: workgroups take blockDim.x / 128 consecutive bricks per virtual block (virtual blocks
+// Sweep: workgroups take blockDim.x / 128 consecutive bricks per virtual block (virtual blocks
 // vb = blockIdx.x + k * gridDim.x < nvirt, nvirt a multiple of 8, XCD-preserving); each wavefront
-// works alone on half a brick (no barrier).
-template <int FINEST>
-__global__ __launch_bounds__(BLOCK) void k_jacobi4(LevelDesc L, OpDesc<float> A, const float *__restrict__ idiag,
-                                                   const float *__restrict__ rhs, const float *__restrict__ zin,
-                                                   float *__restrict__ zout, float omega, Gate Q, int nvirt) {
+// works alone on half a brick (no barrier).  Bound by the latency of its loads: four cells per lane keep
+// the brick's seven reads of z in 16-byte loads with a quarter of the index work.  FP64 at 128^3: 8.5 us
+// with one cell per lane, 7.8 us here (residual 7.9 to 7.4, coarse levels 4.2 to 4.0).
+template <int FINEST, class T>
+__global__ __launch_bounds__(BLOCK) void k_jacobi4(LevelDesc L, OpDesc<T> A, const T *__restrict__ idiag,
+                                                   const T *__restrict__ rhs, const T *__restrict__ zin,
+                                                   T *__restrict__ zout, T omega, Gate Q, int nvirt) {
     if (all_done(Q)) return;
     const int bpb = blockDim.x / ROW4_THREADS, slot = threadIdx.x / ROW4_THREADS, q = threadIdx.x % ROW4_THREADS;
     for (int vb = blockIdx.x; vb < nvirt; vb += gridDim.x) {
@@ -1289,7 +1258,7 @@ __global__ __launch_bounds__(BLOCK) void k_jacobi4(LevelDesc L, OpDesc<float> A,
         const BrickMeta m = L.meta[br];
         if (skip_smooth(Q, L, m)) continue;
         double part = 0.0;
-        jacobi_row4<0>(L, A, idiag, rhs, zin, zout, omega, br, m, q, part);
+        jacobi_row4<0, T>(L, A, idiag, rhs, zin, zout, omega, br, m, q, part);
     }
 }
 
@@ -1306,7 +1275,7 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_jacobi4_dot(LevelDesc L, OpDes
     const BrickMeta m = L.meta[br];
     if (all_done(Q) || skip_smooth(Q, L, m)) return;
     double part = 0.0;
-    jacobi_row4<1>(L, A, idiag, rhs, zin, zout, omega, br, m, threadIdx.x, part);
+    jacobi_row4<1, float>(L, A, idiag, rhs, zin, zout, omega, br, m, threadIdx.x, part);
     part = wave_sum(part);
     if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = part;
     __syncthreads();
@@ -1726,13 +1695,13 @@ __device__ __forceinline__ void row4_reduce2(double &a, double &b, double *lds) 
     b = lds[2] + lds[3];
 }
 
-// res = rhs - A z (k_residual on rows).  FIN (finest level): the first workgroups, one per grid (rounded
+// res = rhs - A z.  FIN (finest level): the first workgroups, one per grid (rounded
 // up to 8, which keeps the bricks' XCDs), run the convergence test of the residual update before this
 // kernel instead of a launch of their own (3 to 6 us).  Nothing in the V-cycle waits for its outcome: a
 // grid that it finds done only loses what this kernel and its neighbours do for it.
-template <int FINEST, int FIN = 0>
-__global__ __launch_bounds__(BLOCK) void k_residual4(LevelDesc L, OpDesc<float> A, const float *__restrict__ rhs,
-                                                     const float *__restrict__ z, float *__restrict__ res, Gate Q,
+template <class T, int FINEST, int FIN = 0>
+__global__ __launch_bounds__(BLOCK) void k_residual4(LevelDesc L, OpDesc<T> A, const T *__restrict__ rhs,
+                                                     const T *__restrict__ z, T *__restrict__ res, Gate Q,
                                                      FinUpdate F) {
     int br, q;
     if (FIN) {
@@ -1749,14 +1718,14 @@ __global__ __launch_bounds__(BLOCK) void k_residual4(LevelDesc L, OpDesc<float> 
     const BrickMeta m = L.meta[br];
     if (all_done(Q) || skip_smooth(Q, L, m)) return;
     const Row4Nbrs N = row4_nbrs(m, br, q);
-    const Row4Vals<float> v = row4_vals(z, N);
-    float r[4], av[4], out[4];
+    const Row4Vals<T> v = row4_vals(z, N);
+    T r[4], av[4], out[4];
     bool unk[4];
-    unpack4(ld4(rhs, N.c), r);
+    load4(rhs, N.c, r);
     apply_row4(L, A, br, m, N, v, av, unk);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) out[j] = unk[j] ? r[j] - av[j] : 0.0f;
-    *reinterpret_cast<float4 *>(res + N.c) = make_float4(out[0], out[1], out[2], out[3]);
+    for (int j = 0; j < 4; ++j) out[j] = unk[j] ? r[j] - av[j] : T(0);
+    store4(res, N.c, out);
 }
 
 // z = omega * idiag * rhs (k_smooth_first on rows).
@@ -2080,35 +2049,6 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_inner_init4(LevelDesc L, const
     store_partials(R, br, mx, sq);
 }
 
-// res = rhs - A z
-template <class T, int FINEST>
-__global__ __launch_bounds__(BLOCK) void k_residual(LevelDesc L, OpDesc<T> A, const T *__restrict__ rhs,
-                                                    const T *__restrict__ z, T *__restrict__ res, Gate Q) {
-    const int br = brick_or_idle(L);
-    if (br < 0) return;
-    const BrickMeta m = L.meta[br];
-    if (all_done(Q) || skip_smooth(Q, L, m)) return;
-    const int t = threadIdx.x;
-    const long c = (long)br * BRICK_CELLS + t;
-    T out = 0;
-    if (m.flags & BM_UNIFORM) {
-        const UniT<T> u = uni_load<T>(L, br);
-        long idx[6];
-        nb_index(nbrs_of(m, br), t, idx);
-        out = rhs[c] - apply_row_uniform(u.g, z, c, idx, z[c]);
-    } else {
-        // every load is issued before the unknown test (the values of other cells are discarded)
-        const Nbrs N = nbrs_of(m, br);
-        long idx[6];
-        nb_index(N, t, idx);
-        const T dirc = A.dir[c];
-        T diag;
-        const T v = rhs[c] - apply_row(A, z, c, idx, dirc, z[c], diag);
-        out = dirc >= 0 ? v : T(0);
-    }
-    res[c] = out;
-}
-
 // Restriction = transpose of trilinear prolongation: coarse cell I gathers fine cells
 // 2I-1..2I+2 per axis with weights 1/4, 3/4, 3/4, 1/4.  One block per coarse brick B stages the
 // 18^3 fine residuals it needs (fine cells 16B-1 .. 16B+16 per axis, in the fine bricks 2B-1 ..
@@ -2412,7 +2352,7 @@ struct SmoothK {
 
 //
 // RES: the cube carries one more ghost layer, so that after the K sweeps the brick's neighbours are
-// exact too, and the kernel also writes the residual rhs - A z of the brick (what k_residual
+// exact too, and the kernel also writes the residual rhs - A z of the brick (what k_residual4
 // computes next, in the same arithmetic): one launch fewer per V-cycle on the level.
 //
 // PRO (post-smoothing, with zin): the level's z first receives the trilinear prolongation of the
@@ -2705,7 +2645,7 @@ struct ComponentSums {
 
 // Coarse solve of every grid whose last level L is (one brick): block g handles grid g with
 // `sweeps` damped-Jacobi sweeps from zero, in LDS.  DOT (finest level only): also the r.z partial
-// of the grid's brick, as k_jacobi<..., DOT> stores it for grids with coarser levels.  CPT cells per
+// of the grid's brick, as k_jacobi_dot stores it for grids with coarser levels.  CPT cells per
 // thread (512 / CPT threads): fewer wavefronts make each sweep's barrier cheaper; every thread keeps
 // its cells' couplings and own values in registers.
 template <class T, int DOT, int CPT = 1>

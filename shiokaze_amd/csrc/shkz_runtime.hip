@@ -766,7 +766,7 @@ static inline Row4Launch row4_launch(int nbricks, bool finest) {
 }
 
 // One damped-Jacobi sweep zout = J(zin) of level l (dot: with the rhs.zout partials of the finest
-// level's last sweep).  FP32 levels sweep four cells per thread (k_jacobi4*), FP64 levels one.
+// level's last sweep).  Four cells per thread (k_jacobi4*), one in FP64's sweep with the dot.
 template <class T>
 static void jacobi_sweep(shkz_ctx *C, Launcher &K, int l, bool dot, const LevelDesc &L, OpDesc<T> A, const T *id,
                          const T *rhs, const T *zin, T *zout, T om, Gate Q, RedBuf red) {
@@ -774,22 +774,16 @@ static void jacobi_sweep(shkz_ctx *C, Launcher &K, int l, bool dot, const LevelD
     const double es = (double)sizeof(T);
     const char *name = dot ? "jacobi_dot_L0" : f ? "jacobi_L0" : "jacobi_Lc";
     const unsigned nb = brick_grid(L.nbricks);
-    if constexpr (sizeof(T) == 4) {
-        if (dot) {
-            K.go(name, l, 7 * es, -usave(C, l, 4 * es), dim3(nb), dim3(ROW4_THREADS), k_jacobi4_dot, L, A, id, rhs, zin,
-                 zout, om, Q, red);
-        } else {
-            const Row4Launch R4 = row4_launch(L.nbricks, f);
-            K.go(name, l, 7 * es, -usave(C, l, 4 * es), R4.grid, R4.block, f ? k_jacobi4<1> : k_jacobi4<0>, L, A, id,
-                 rhs, zin, zout, om, Q, (int)R4.grid.x);
-        }
-    } else if (dot) {
-        // one brick per workgroup: the reduction of the dot variant costs two barriers per brick
-        K.go(name, l, 7 * es, -usave(C, l, 4 * es), dim3(nb), dim3(BLOCK), k_jacobi<T, 1, 1>, L, A, id, rhs, zin, zout,
-             om, Q, red, (int)nb);
+    if (!dot) {
+        const Row4Launch R4 = row4_launch(L.nbricks, f);
+        K.go(name, l, 7 * es, -usave(C, l, 4 * es), R4.grid, R4.block, f ? k_jacobi4<1, T> : k_jacobi4<0, T>, L, A, id, rhs,
+             zin, zout, om, Q, (int)R4.grid.x);
+    } else if constexpr (sizeof(T) == 4) {
+        K.go(name, l, 7 * es, -usave(C, l, 4 * es), dim3(nb), dim3(ROW4_THREADS), k_jacobi4_dot, L, A, id, rhs, zin,
+             zout, om, Q, red);
     } else {
-        K.go(name, l, 7 * es, -usave(C, l, 4 * es), dim3(std::min<unsigned>(nb, PERSIST_BLOCKS)), dim3(BLOCK),
-             f ? k_jacobi<T, 1, 0> : k_jacobi<T, 0, 0>, L, A, id, rhs, zin, zout, om, Q, red, (int)nb);
+        K.go(name, l, 7 * es, -usave(C, l, 4 * es), dim3(nb), dim3(BLOCK), k_jacobi_dot<T>, L, A, id, rhs, zin, zout, om,
+             Q, red);
     }
 }
 
@@ -825,7 +819,6 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
         const OpDesc<T> A = op_of<T>(L);
         const T *id = (const T *)L.idiag;
         const dim3 g(brick_grid(L.nbricks)), b(BLOCK);
-        const dim3 gp(std::min<unsigned>(g.x, PERSIST_BLOCKS));  // persistent kernels
         const bool f = l == 0;
         const int pre = f ? P.pre : P.pre_c, post = f ? P.post : P.post_c;
         const bool last = l == nl - 1;
@@ -911,17 +904,12 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
             }
         }
         if (!res_done) {
-            if constexpr (sizeof(T) == 4) {
-                Row4Launch R4 = row4_launch(L.nbricks, f);
-                const bool with_fin = f && fin.partials;
-                if (with_fin) R4.grid.x += (unsigned)((P.ngrids + 7) & ~7);
-                K.go(f ? "residual_L0" : "residual_Lc", l, 7 * es, -usave(C, l, 4 * es), R4.grid, R4.block,
-                     with_fin ? k_residual4<1, 1> : f ? k_residual4<1> : k_residual4<0>, L.desc, A, rhs,
-                     (const T *)cur, (T *)L.res, Q, fin);
-            }
-            else
-                K.go(f ? "residual_L0" : "residual_Lc", l, 7 * es, -usave(C, l, 4 * es), g, b,
-                     f ? k_residual<T, 1> : k_residual<T, 0>, L.desc, A, rhs, (const T *)cur, (T *)L.res, Q);
+            Row4Launch R4 = row4_launch(L.nbricks, f);
+            const bool with_fin = f && fin.partials;
+            if (with_fin) R4.grid.x += (unsigned)((P.ngrids + 7) & ~7);
+            K.go(f ? "residual_L0" : "residual_Lc", l, 7 * es, -usave(C, l, 4 * es), R4.grid, R4.block,
+                 with_fin ? k_residual4<T, 1, 1> : f ? k_residual4<T, 1> : k_residual4<T, 0>, L.desc, A, rhs,
+                 (const T *)cur, (T *)L.res, Q, fin);
         }
         LevelHost &Lc = C->levels[l + 1];
         if constexpr (sizeof(T) == 4) {
@@ -947,7 +935,6 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
         const OpDesc<T> A = op_of<T>(L);
         const T *id = (const T *)L.idiag;
         const dim3 g(brick_grid(L.nbricks)), b(BLOCK);
-        const dim3 gp(std::min<unsigned>(g.x, PERSIST_BLOCKS));  // persistent kernels
         const bool f = l == 0;
         const int post = f ? P.post : P.post_c;
         T *cur = zcur[l], *oth = zoth[l];
