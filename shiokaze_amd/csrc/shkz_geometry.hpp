@@ -113,31 +113,34 @@ __device__ __forceinline__ double negative_area(const double v[4]) {
     if (n0 && n1 && n2 && n3) return 1.0;
     const int cx[4] = {0, 1, 1, 0};
     const int cy[4] = {0, 0, 1, 1};
-    double px[8], py[8];
-    int m = 0;
+    // the shoelace terms as the vertices come, in their order; the closing one last (a list of the vertices
+    // would be indexed by a count that differs between lanes: selects over the whole list for every entry)
+    double fx = 0.0, fy = 0.0, lx = 0.0, ly = 0.0, sum = 0.0;
+    bool any = false;
+    auto vertex = [&](double x, double y) {
+        if (any) {
+            sum += lx * y - ly * x;
+        } else {
+            fx = x;
+            fy = y;
+            any = true;
+        }
+        lx = x;
+        ly = y;
+    };
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
         const int nn = (n + 1) & 3;
-        if (v[n] < 0.0) {
-            px[m] = cx[n];
-            py[m] = cy[n];
-            ++m;
-        }
+        if (v[n] < 0.0) vertex(cx[n], cy[n]);
         if (v[n] * v[nn] < 0) {
             const double y0 = v[n], y1 = v[nn];
             if (y0 - y1) {
                 const double a = y0 / (y0 - y1);
-                px[m] = (1.0 - a) * cx[n] + a * cx[nn];
-                py[m] = (1.0 - a) * cy[n] + a * cy[nn];
-                ++m;
+                vertex((1.0 - a) * cx[n] + a * cx[nn], (1.0 - a) * cy[n] + a * cy[nn]);
             }
         }
     }
-    double sum = 0.0;
-    for (int a = 0; a < m; ++a) {
-        const int b = (a + 1) % m;
-        sum += px[a] * py[b] - py[a] * px[b];
-    }
+    if (any) sum += lx * fy - ly * fx;
     return 0.5 * sum;
 }
 
@@ -146,6 +149,17 @@ __device__ __forceinline__ double negative_area(const double v[4]) {
 __device__ __forceinline__ float area_from_corners(const GridDesc &G, const double v[4]) {
 #pragma clang fp contract(off)
     double a = 1.0 - negative_area(v);
+    if (a && a < G.eps_solid) a = G.eps_solid;
+    float af = (float)a;
+    if (!G.so_solid && af) af = 1.0f;
+    return af;
+}
+
+// Open fraction of an interior face of a 2D grid, an edge between two nodes: 1 - fraction of the solid
+// samples at its ends (macutility2.cpp:104).
+__device__ __forceinline__ float area_from_ends(const GridDesc &G, double s0, double s1) {
+#pragma clang fp contract(off)
+    double a = 1.0 - liquid_fraction(s0, s1);
     if (a && a < G.eps_solid) a = G.eps_solid;
     float af = (float)a;
     if (!G.so_solid && af) af = 1.0f;
@@ -179,9 +193,7 @@ __device__ __forceinline__ float face_area(const GridDesc &G, const Exist &E, in
         if (boundary) {
             a = 0.0;
         } else if (G.flat) {
-            // 2D face = an edge between two nodes: 1 - fraction of the solid samples at its ends
-            // (macutility2.cpp:104)
-            a = 1.0 - liquid_fraction(solid_at(G, i, j, 0), solid_at(G, i + (dim != 0), j + (dim != 1), 0));
+            return area_from_ends(G, solid_at(G, i, j, 0), solid_at(G, i + (dim != 0), j + (dim != 1), 0));
         } else {
             // corner order of macutility3.cpp:123-138 mapped to (0,0),(1,0),(1,1),(0,1)
             // the face's second and third corner step along a and b (the two axes other than dim)

@@ -9,8 +9,7 @@
 //   k_coarsen, k_idiag multigrid operators (no counterpart: they stand in for MIC(0))
 //   k_defect4 ... k_update_p, V-cycle kernels
 //                      Krylov solve (stands in for PCGSolver::solve, pcg_solver.h:246-295)
-//   k_scatter_pressure m_pressure (:245-248)
-//   k_velocity_update  velocity update (:252-268)
+//   k_output           m_pressure (:245-248) and velocity update (:252-268)
 //
 // Build and output kernels work on one grid's dense arrays.  Solver kernels work on a batch: the
 // stored bricks of every grid of the batch, concatenated, one 512-thread block per brick (thread =
@@ -231,52 +230,208 @@ __global__ void k_surface_tension(GridDesc G, int dim, const float *curv, double
     }
 }
 
+// The kernels that run once per grid of a batch (labelling, assembly, output) take up to
+// GRIDS_PER_LAUNCH grids in one launch: their descriptors travel in the kernel's arguments (which hold 4 KB),
+// and workgroup b works for the grid whose range [first[g], first[g + 1]) holds b.  A launch of its own costs a
+// small grid more than its work (64 cubes of 32 to 160 cells: 5 launches per grid).
+constexpr int GRIDS_PER_LAUNCH = 12;
+template <class D>
+struct GridTable {
+    int n;
+    int first[GRIDS_PER_LAUNCH + 1];
+    D g[GRIDS_PER_LAUNCH];
+};
+// The grid of this workgroup and its workgroup index within it (-1: a workgroup beyond the last grid).
+// Each XCD takes a contiguous range of the launch.
+template <class D>
+__device__ __forceinline__ int table_grid(const GridTable<D> &T, int &local) {
+    const int blk = xcd_brick(blockIdx.x, gridDim.x);
+    int g = 0;
+    while (g < T.n && blk >= T.first[g + 1]) ++g;
+    if (g == T.n) return -1;
+    local = blk - T.first[g];
+    return g;
+}
+
 // Unknown labelling (macpressuresolver3.cpp:121-156): a liquid cell is an unknown when an
-// in-bounds liquid neighbour shares a face with nonzero area (rho is 1 between two liquid
-// cells).  One block per brick position of the dense grid; writes cell flags (bit0 liquid, bit1
-// unknown) and per brick bit0 = holds an unknown, bit1 = holds a liquid cell (so the host learns
-// levelset_exist() of the liquid, array_utility3.h:112-122, on the way).  The face fractions here
-// are only taken beside a liquid cell, so the liquid exists.
-__global__ __launch_bounds__(BLOCK) void k_flags(GridDesc G, int nbx, int nby, int nbz, uint8_t *cflag, uint8_t *bflag) {
-    const int bid = xcd_brick(blockIdx.x, gridDim.x);  // each XCD takes a contiguous slab
-    if (bid >= nbx * nby * nbz) return;
-    const int bz = bid % nbz, by = (bid / nbz) % nby, bx = bid / (nbz * nby);
+// in-bounds liquid neighbour shares a face with nonzero area (rho is nonzero between two liquid
+// cells).  Writes cell flags (bit0 liquid, bit1 unknown) and per brick bit0 = holds an unknown, bit1 =
+// holds a liquid cell (so the host learns levelset_exist() of the liquid, array_utility3.h:112-122, on
+// the way).
+//
+// Without a solid only signs matter, and the kernel is a pass over the level set.  A thread takes a column
+// of 8 cells along x, a workgroup the columns of FLAGS_SPAN bricks along z (FLAGS_SPAN_FLAT along y in a 2D
+// grid), so that a sample is read 1.25 times instead of up to 7: the signs of a column are the bits of one
+// byte, which neighbours take from LDS.  256^3 of FP64 samples: 116 us with one cell per thread and a
+// chain of neighbour tests, 102 us with columns that load their neighbours, 67 to 93 us here; 120x168x89
+// within a solid's reach 40 to 16 us.
+struct FlagsGrid {
+    GridDesc G;
+    int nbx, nby, nbz;
+    uint8_t *cflag, *bflag;
+};
+constexpr int FLAGS_THREADS = 256;
+constexpr int FLAGS_SPAN = FLAGS_THREADS / BRICK / BRICK, FLAGS_SPAN_FLAT = FLAGS_THREADS / BRICK;  // bricks
+// Signs of `ni` cells at stride HD from c0 on: bit p = cell p is liquid.
+template <class Tp>
+__device__ __forceinline__ unsigned column_bits(const void *a, size_t c0, int ni, size_t HD) {
+    const Tp *phi = (const Tp *)a;
+    Tp v[BRICK];
+#pragma unroll
+    for (int p = 0; p < BRICK; ++p) v[p] = phi[c0 + (p < ni ? p : 0) * HD];
+    unsigned m = 0;
+#pragma unroll
+    for (int p = 0; p < BRICK; ++p) m |= (unsigned)(v[p] < Tp(0)) << p;
+    return m & ((1u << ni) - 1);
+}
+// The same of the ni + 1 solid nodes of a column (bit p = node p lies in the solid).
+template <class Ts, int N = BRICK>
+__device__ __forceinline__ unsigned node_bits(const void *a, size_t n0, int ni, size_t stride) {
+    const Ts *solid = (const Ts *)a;
+    Ts v[N + 1];
+#pragma unroll
+    for (int p = 0; p <= N; ++p) v[p] = solid[n0 + (p <= ni ? p : 0) * stride];
+    unsigned m = 0;
+#pragma unroll
+    for (int p = 0; p <= N; ++p) m |= (unsigned)(v[p] < Ts(0)) << p;
+    return m & ((2u << ni) - 1);
+}
+static inline int flags_blocks(const FlagsGrid &F) {
+    if (F.G.flat) return F.nbx * ((F.nby + FLAGS_SPAN_FLAT - 1) / FLAGS_SPAN_FLAT);
+    return F.nbx * F.nby * ((F.nbz + FLAGS_SPAN - 1) / FLAGS_SPAN);
+}
+__global__ __launch_bounds__(FLAGS_THREADS) void k_flags(GridTable<FlagsGrid> T) {
+    // columns of the workgroup with one more on each side: rows along y (one in a 2D grid), contiguous axis
+    constexpr int COLS = FLAGS_SPAN * BRICK, WIDE = COLS + 2;
+    __shared__ uint8_t around[FLAGS_THREADS + 2 > (BRICK + 2) * WIDE ? FLAGS_THREADS + 2 : (BRICK + 2) * WIDE];
+    __shared__ uint16_t nodes[FLAGS_THREADS + 1 > (BRICK + 1) * (COLS + 1) ? FLAGS_THREADS + 1 : (BRICK + 1) * (COLS + 1)];
+    __shared__ int bits[FLAGS_SPAN_FLAT];
+    int local;
+    const int entry = table_grid(T, local);
+    if (entry < 0) return;
+    const FlagsGrid &F = T.g[entry];
+    const GridDesc &G = F.G;
     const int t = threadIdx.x;
-    const int i = bx * BRICK + (t >> 6), j = by * BRICK + ((t >> 3) & 7), k = bz * BRICK + (t & 7);
-    int unknown = 0, any_liquid = 0;
-    const Exist E{true, true};
-    if (i < G.w && j < G.h && k < G.d) {
-        const double pc = phi_at(G, i, j, k);
-        const bool liquid = pc < 0.0;
-        any_liquid = liquid;
-        if (liquid) {
-            const int di[6] = {1, -1, 0, 0, 0, 0}, dj[6] = {0, 0, 1, -1, 0, 0}, dk[6] = {0, 0, 0, 0, 1, -1};
-            for (int nq = 0; nq < 6 && !unknown; ++nq) {
-                const int qi = i + di[nq], qj = j + dj[nq], qk = k + dk[nq];
-                if (qi < 0 || qi >= G.w || qj < 0 || qj >= G.h || qk < 0 || qk >= G.d) continue;
-                const double pq = phi_at(G, qi, qj, qk);
-                if (!(pq < 0.0)) continue;
-                const int dim = nq >> 1;
-                const int fi = (nq & 1) ? i : qi, fj = (nq & 1) ? j : qj, fk = (nq & 1) ? k : qk;
-                // face_rho of this interior face from the two samples in hand: the one at the
-                // face's index cell first (the neighbour for a high face, the cell for a low one)
-                if (face_area(G, E, dim, fi, fj, fk) != 0.0f &&
-                    ((nq & 1) ? rho_from_samples(G, E, pc, pq) : rho_from_samples(G, E, pq, pc)) != 0.0f)
-                    unknown = 1;
+    // the workgroup's bricks: (bx, by, bz) on, along z (along y in a 2D grid); its thread's column (j, k), its
+    // place in `around` and the column of the border that it also reads (at hat, -1: none)
+    int bx, by, bz, j, k, slot, at, row = 0, hj = 0, hk = 0, hat = -1;
+    if (G.flat) {
+        const int nspan = (F.nby + FLAGS_SPAN_FLAT - 1) / FLAGS_SPAN_FLAT;
+        bx = local / nspan, by = (local - bx * nspan) * FLAGS_SPAN_FLAT, bz = 0;
+        j = by * BRICK + t, k = 0, slot = t / BRICK, at = t + 1;
+        if (t < 2) hj = by * BRICK + (t ? FLAGS_THREADS : -1), hat = t ? FLAGS_THREADS + 1 : 0;
+    } else {
+        const int nspan = (F.nbz + FLAGS_SPAN - 1) / FLAGS_SPAN, r = local / nspan;
+        bx = r / F.nby, by = r - bx * F.nby, bz = (local - r * nspan) * FLAGS_SPAN;
+        const int jj = t / COLS, kk = t % COLS;
+        j = by * BRICK + jj, k = bz * BRICK + kk, slot = kk / BRICK, row = WIDE;
+        at = (jj + 1) * WIDE + kk + 1;
+        int a = 0, b = 0;
+        if (t < 2 * COLS) {
+            a = t < COLS ? 0 : BRICK + 1, b = t % COLS + 1;
+        } else if (t < 2 * (COLS + BRICK)) {
+            a = t % BRICK + 1, b = t < 2 * COLS + BRICK ? 0 : COLS + 1;
+        }
+        if (t < 2 * (COLS + BRICK)) hj = by * BRICK + a - 1, hk = bz * BRICK + b - 1, hat = a * WIDE + b;
+    }
+    const size_t HD = (size_t)((unsigned)G.h * (unsigned)G.d);
+    const int i0 = bx * BRICK, ni = min(BRICK, G.w - i0);
+    const bool in = j < G.h && k < G.d, hin = hj >= 0 && hj < G.h && hk >= 0 && hk < G.d;
+    const size_t c0 = in ? cell_index(G, i0, j, k) : 0;
+    unsigned liquid = 0, beyond = 0, border = 0, known = 0;
+    if (in) {
+        // the column's own cells, and those before and after it along x (bits 0 and 1 of beyond)
+        const size_t before = i0 > 0 ? HD : 0, after = i0 + BRICK < G.w ? BRICK * HD : 0;
+        if (G.phi64) {
+            const double *phi = (const double *)G.phi;
+            const double b = phi[c0 - before], a = phi[c0 + after];
+            liquid = column_bits<double>(phi, c0, ni, HD);
+            beyond = (before && b < 0.0 ? 1 : 0) | (after && a < 0.0 ? 2 : 0);
+        } else {
+            const float *phi = (const float *)G.phi;
+            const float b = phi[c0 - before], a = phi[c0 + after];
+            liquid = column_bits<float>(phi, c0, ni, HD);
+            beyond = (before && b < 0.0f ? 1 : 0) | (after && a < 0.0f ? 2 : 0);
+        }
+    }
+    if (hat >= 0 && hin) {
+        const size_t h0 = cell_index(G, i0, hj, hk);
+        border = G.phi64 ? column_bits<double>(G.phi, h0, ni, HD) : column_bits<float>(G.phi, h0, ni, HD);
+    }
+    around[at] = (uint8_t)liquid;
+    if (hat >= 0) around[hat] = (uint8_t)border;
+    // solid nodes of the workgroup's columns: its (j, k) and one more on the high sides
+    int nat = 0;
+    if (G.solid) {
+        const int cols = G.flat ? FLAGS_THREADS : COLS, rows = G.flat ? 1 : BRICK + 1;
+        for (int q = t; q < rows * (cols + 1); q += FLAGS_THREADS) {
+            const int a = G.flat ? 0 : q / (COLS + 1), b = q - a * (COLS + 1);
+            const int nj = min(by * BRICK + (G.flat ? b : a), G.h), nk = G.flat ? 0 : min(bz * BRICK + b, G.d);
+            const size_t n0 = G.flat ? (size_t)((unsigned)i0 * (unsigned)(G.h + 1) + (unsigned)nj) : node_index(G, i0, nj, nk);
+            const size_t stride = G.flat ? (size_t)(G.h + 1) : (size_t)((unsigned)(G.h + 1) * (unsigned)(G.d + 1));
+            nodes[q] = (uint16_t)(G.solid64 ? node_bits<double>(G.solid, n0, ni, stride)
+                                            : node_bits<float>(G.solid, n0, ni, stride));
+        }
+        nat = G.flat ? t : t / COLS * (COLS + 1) + t % COLS;
+    }
+    if (t < FLAGS_SPAN_FLAT) bits[t] = 0;
+    __syncthreads();
+    if (liquid) {
+        const Exist E{true, true};
+        const unsigned xm = ((liquid << 1) | (beyond & 1)) & liquid, xp = ((liquid >> 1) | (beyond >> 1) << (BRICK - 1)) & liquid;
+        const unsigned am = around[at - 1] & liquid, ap = around[at + 1] & liquid;  // along the contiguous axis
+        const unsigned ym = G.flat ? am : around[at - row] & liquid, yp = G.flat ? ap : around[at + row] & liquid;
+        const unsigned zm = G.flat ? 0 : am, zp = G.flat ? 0 : ap;
+        unsigned unknown = xm | xp | ym | yp | zm | zp;
+        if (G.solid) {
+            // per face of a cell, from the signs of its corners: whole with none in the solid, shut with all;
+            // only the others' areas are formed, until one is open
+            const unsigned n00 = nodes[nat], n01 = G.flat ? n00 : nodes[nat + 1];
+            const unsigned n10 = G.flat ? nodes[nat + 1] : nodes[nat + COLS + 1], n11 = G.flat ? n10 : nodes[nat + COLS + 2];
+            unsigned part[6];
+            unknown = 0;
+            auto face = [&](int nq, unsigned both, unsigned any, unsigned all) {
+                unknown |= both & ~any;
+                part[nq] = both & any & ~all;
+            };
+            auto pair = [](unsigned m) { return m | m >> 1; };
+            auto both = [](unsigned m) { return m & m >> 1; };
+            face(0, xp, (n00 | n01 | n10 | n11) >> 1, (n00 & n01 & n10 & n11) >> 1);
+            face(1, xm, n00 | n01 | n10 | n11, n00 & n01 & n10 & n11);
+            face(2, yp, pair(n10 | n11), both(n10 & n11));
+            face(3, ym, pair(n00 | n01), both(n00 & n01));
+            face(4, zp, pair(n01 | n11), both(n01 & n11));
+            face(5, zm, pair(n00 | n10), both(n00 & n10));
+            unsigned left = (part[0] | part[1] | part[2] | part[3] | part[4] | part[5]) & ~unknown;
+            while (left) {
+                const int p = __ffs((int)left) - 1;
+                left &= left - 1;
+                unsigned faces = 0;
+#pragma unroll
+                for (int nq = 0; nq < 6; ++nq) faces |= (part[nq] >> p & 1) << nq;
+                while (faces) {
+                    const int nq = __ffs((int)faces) - 1, dim = nq >> 1, o = (nq & 1) ? 0 : 1;
+                    faces &= faces - 1;
+                    if (face_area(G, E, dim, i0 + p + (dim == 0) * o, j + (dim == 1) * o, k + (dim == 2) * o) != 0.0f) {
+                        unknown |= 1u << p;
+                        break;
+                    }
+                }
             }
         }
-        cflag[cell_index(G, i, j, k)] = (uint8_t)((liquid ? 1 : 0) | (unknown ? 2 : 0));
+        known = unknown;
+        atomicOr(&bits[slot], (unknown ? 1 : 0) | 2);
     }
-    // both bits with one barrier: per-wavefront ballots combined in LDS
-    __shared__ int wbits[BLOCK / 64];
-    const bool wu = __ballot(unknown) != 0, wl = __ballot(any_liquid) != 0;
-    if ((t & 63) == 0) wbits[t >> 6] = (wu ? 1 : 0) | (wl ? 2 : 0);
-    __syncthreads();
-    if (t == 0) {
-        int v = 0;
+    if (in) {
 #pragma unroll
-        for (int w = 0; w < BLOCK / 64; ++w) v |= wbits[w];
-        bflag[bid] = (uint8_t)v;
+        for (int p = 0; p < BRICK; ++p)
+            if (p < ni) F.cflag[c0 + p * HD] = (uint8_t)((liquid >> p & 1) | (known >> p & 1) << 1);
+    }
+    __syncthreads();
+    const int nb = G.flat ? min(FLAGS_SPAN_FLAT, F.nby - by) : min(FLAGS_SPAN, F.nbz - bz);
+    if (t < nb) {
+        const int y = G.flat ? by + t : by, z = G.flat ? 0 : bz + t;
+        F.bflag[((size_t)bx * F.nby + y) * F.nbz + z] = (uint8_t)bits[t];
     }
 }
 
@@ -300,25 +455,33 @@ struct OperatorFinish {
     UniCoef *uni;
     int *counts;      // unknowns per brick (| UNIFORM_COUNT_BIT)
 };
-__global__ __launch_bounds__(BLOCK) void k_operator(GridDesc G, LevelDesc L, GridLevel GL, const uint8_t *__restrict__ cflag,
-                                                    double *dir64, double *gx64, double *gy64, double *gz64,
-                                                    float *dir32, float *gx32, float *gy32, float *gz32, double *b,
-                                                    double *x, const double *__restrict__ warm, double rhs_correct,
-                                                    OperatorFinish FIN) {
+struct OperatorGrid {
+    GridDesc G;
+    GridLevel GL;
+    const uint8_t *cflag;
+    const double *warm;
+    double rhs_correct;
+};
+__global__ __launch_bounds__(BLOCK) void k_operator(GridTable<OperatorGrid> T, LevelDesc L, double *dir64, double *gx64,
+                                                    double *gy64, double *gz64, float *dir32, float *gx32, float *gy32,
+                                                    float *gz32, double *b, double *x, OperatorFinish FIN) {
 #pragma clang fp contract(off)
-    const int local = xcd_brick(blockIdx.x, gridDim.x);
-    if (local >= GL.brick_end - GL.brick_start) return;
-    const int br = GL.brick_start + local;
+    int local;
+    const int entry = table_grid(T, local);
+    if (entry < 0) return;
+    const OperatorGrid &F = T.g[entry];
+    const GridDesc &G = F.G;
+    const int br = F.GL.brick_start + local;
     const int t = threadIdx.x;
     const int bx = L.bxyz[3 * br], by = L.bxyz[3 * br + 1], bz = L.bxyz[3 * br + 2];
     const int i = bx * BRICK + (t >> 6), j = by * BRICK + ((t >> 3) & 7), k = bz * BRICK + (t & 7);
     const long c = (long)br * BRICK_CELLS + t;
     const bool inside = i < G.w && j < G.h && k < G.d;
-    const bool unknown = inside && (cflag[cell_index(G, i, j, k)] & 2);
+    const bool unknown = inside && (F.cflag[cell_index(G, i, j, k)] & 2);
     double dir = -1.0, g[3] = {0.0, 0.0, 0.0}, rhs = 0.0, x0 = 0.0;
     double gp[3] = {0.0, 0.0, 0.0};  // couplings of the high faces (the neighbours' low ones)
-    if (unknown && !G.flat) {
-        // 3D: the cell's 8 solid corners, 7 level-set samples and 6 face velocities are loaded at
+    if (unknown) {
+        // the cell's 8 solid corners (4 in a 2D grid), 7 level-set samples and 6 face velocities are loaded at
         // once; each face's area and liquid fraction then use the face functions' arithmetic
         const Exist E = exist_of(G);
         const double dt = G.dt, dx = G.dx;
@@ -328,7 +491,10 @@ __global__ __launch_bounds__(BLOCK) void k_operator(GridDesc G, LevelDesc L, Gri
         if (G.solid) {
             size_t nidx[8];
 #pragma unroll
-            for (int n = 0; n < 8; ++n) nidx[n] = node_index(G, i + (n >> 2), j + ((n >> 1) & 1), k + (n & 1));
+            for (int n = 0; n < 8; ++n) {
+                const int a = i + (n >> 2), b = j + ((n >> 1) & 1);
+                nidx[n] = G.flat ? (size_t)((unsigned)a * (unsigned)(G.h + 1) + (unsigned)b) : node_index(G, a, b, k + (n & 1));
+            }
             load_samples<8>(G.solid, G.solid64, nidx, sc);
         }
         // level set at the six neighbours (clamped into the grid: out-of-grid ones go unused) and
@@ -340,13 +506,19 @@ __global__ __launch_bounds__(BLOCK) void k_operator(GridDesc G, LevelDesc L, Gri
             pidx[nq] = cell_index(G, clampi(i + di[nq], 0, G.w - 1), clampi(j + dj[nq], 0, G.h - 1),
                                   clampi(k + dk[nq], 0, G.d - 1));
             const int dim = nq >> 1, o = (nq & 1) ? 0 : 1;
-            uf[nq] = G.vel[dim][face_index(G, dim, i + (dim == 0) * o, j + (dim == 1) * o, k + (dim == 2) * o)];
+            uf[nq] = G.flat && dim == 2 ? 0.0f : G.vel[dim][face_index(G, dim, i + (dim == 0) * o, j + (dim == 1) * o, k + (dim == 2) * o)];
         }
         pidx[6] = cell_index(G, i, j, k);
         double ph[7];
         load_samples<7>(G.phi, G.phi64, pidx, ph);
         const double pc = ph[6];
         double dsum = 0.0;
+        // the conductance of a whole face between two liquid cells (most of them): dt * 1 / (dx * dx * 1),
+        // the same bits without a division per face
+        const double whole = dt / (dx * dx);
+        bool deep = E.liquid && rho_from_samples(G, E, -1.0, -1.0) == 1.0f;  // liquid all around
+#pragma unroll
+        for (int n = 0; n < 7; ++n) deep = deep && ph[n] < 0.0;
 #pragma unroll
         for (int nq = 0; nq < 6; ++nq) {
             const int qi = i + di[nq], qj = j + dj[nq], qk = k + dk[nq];
@@ -364,63 +536,33 @@ __global__ __launch_bounds__(BLOCK) void k_operator(GridDesc G, LevelDesc L, Gri
                 } else {
                     v[0] = n(0, 0, o); v[1] = n(1, 0, o); v[2] = n(1, 1, o); v[3] = n(0, 1, o);
                 }
-                area = area_from_corners(G, v);
+                area = G.flat ? area_from_ends(G, v[0], v[1]) : area_from_corners(G, v);
             }
             if (area) {
-                // face_rho: the sample at the face's index cell first, then the one below it
-                const double rho = o ? rho_from_samples(G, E, ph[nq], pc) : rho_from_samples(G, E, pc, ph[nq]);
-                if (rho) {
-                    const double value = dt * (double)area / (dx * dx * rho);
-                    if (ph[nq] < 0.0) {
-                        if (nq & 1) g[dim] = value;
-                        else gp[dim] = value;
-                    } else {
-                        dsum += value;
+                if (deep && area == 1.0f) {
+                    if (nq & 1) g[dim] = whole;
+                    else gp[dim] = whole;
+                } else {
+                    // face_rho: the sample at the face's index cell first, then the one below it
+                    const double rho = o ? rho_from_samples(G, E, ph[nq], pc) : rho_from_samples(G, E, pc, ph[nq]);
+                    if (rho) {
+                        const double value = dt * (double)area / (dx * dx * rho);
+                        if (ph[nq] < 0.0) {
+                            if (nq & 1) g[dim] = value;
+                            else gp[dim] = value;
+                        } else {
+                            dsum += value;
+                        }
                     }
                 }
-                rhs += -sgn[nq] * (double)area * (double)uf[nq] / dx;
+                if (!G.flat) rhs += -sgn[nq] * (double)area * (double)uf[nq] / dx;
             }
+            // the 2D module adds the term for every in-bounds neighbour (macpressuresolver2.cpp:176)
+            if (G.flat) rhs += -sgn[nq] * (double)area * (double)uf[nq] / dx;
         }
         dir = dsum;
-        rhs += rhs_correct;
-        if (warm) x0 = warm[cell_index(G, i, j, k)];
-    } else if (unknown) {
-        const Exist E = exist_of(G);
-        const double dt = G.dt, dx = G.dx;
-        const int di[6] = {1, -1, 0, 0, 0, 0}, dj[6] = {0, 0, 1, -1, 0, 0}, dk[6] = {0, 0, 0, 0, 1, -1};
-        const int sgn[6] = {1, -1, 1, -1, 1, -1};
-        double dsum = 0.0;
-        for (int nq = 0; nq < 6; ++nq) {
-            const int qi = i + di[nq], qj = j + dj[nq], qk = k + dk[nq];
-            if (qi < 0 || qi >= G.w || qj < 0 || qj >= G.h || qk < 0 || qk >= G.d) continue;
-            const int dim = nq >> 1;
-            const int fi = (nq & 1) ? i : qi, fj = (nq & 1) ? j : qj, fk = (nq & 1) ? k : qk;
-            const double area = face_area(G, E, dim, fi, fj, fk);
-            if (area) {
-                const double rho = face_rho(G, E, dim, fi, fj, fk);
-                if (rho) {
-                    const double value = dt * area / (dx * dx * rho);
-                    if (phi_at(G, qi, qj, qk) < 0.0) {
-                        if (nq & 1) g[dim] = value;
-                        else gp[dim] = value;
-                    } else {
-                        dsum += value;
-                    }
-                }
-                if (!G.flat) {
-                    const float u = G.vel[dim][face_index(G, dim, fi, fj, fk)];
-                    rhs += -sgn[nq] * area * (double)u / dx;
-                }
-            }
-            if (G.flat) {
-                // the 2D module adds the term for every in-bounds neighbour (macpressuresolver2.cpp:176)
-                const float u = G.vel[dim][face_index(G, dim, fi, fj, fk)];
-                rhs += -sgn[nq] * area * (double)u / dx;
-            }
-        }
-        dir = dsum;
-        rhs += rhs_correct;
-        if (warm) x0 = warm[cell_index(G, i, j, k)];
+        rhs += F.rhs_correct;
+        if (F.warm) x0 = F.warm[cell_index(G, i, j, k)];
     }
     dir64[c] = dir;
     gx64[c] = g[0];
@@ -450,20 +592,33 @@ __global__ __launch_bounds__(BLOCK) void k_operator(GridDesc G, LevelDesc L, Gri
     }
     if (FIN.id32) FIN.id32[c] = i32;
     if (FIN.id64) FIN.id64[c] = i64;
-    // unknown count and the uniformity vote: the brick's first cell gives the reference values
+    // unknown count and the uniformity vote (the brick's first cell gives the reference values), by ballots
     __shared__ double gref, iref64;
     __shared__ float iref32;
+    __shared__ int counted[BLOCK / 64], agreed[BLOCK / 64];
     if (t == 0) {
         gref = g[0];
         iref64 = i64;
         iref32 = i32;
     }
-    const int n = __syncthreads_count(dir >= 0);
+    __syncthreads();
     const double Gu = gref;
     const bool ok = Gu > 0.0 && dir == 0.0 && g[0] == Gu && g[1] == Gu && g[2] == Gu && gp[0] == Gu && gp[1] == Gu &&
                     gp[2] == Gu && (!FIN.id64 || i64 == iref64) && (!FIN.id32 || i32 == iref32);
-    const bool uniform = __syncthreads_and(ok);
-    if (t == 0) {
+    const unsigned long long unk = __ballot(dir >= 0), agree = __ballot(ok);
+    if ((t & 63) == 0) {
+        counted[t >> 6] = __popcll(unk);
+        agreed[t >> 6] = agree == ~0ull;
+    }
+    __syncthreads();
+    if (t != 0) return;
+    int n = 0, uniform = 1;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; ++w) {
+        n += counted[w];
+        uniform &= agreed[w];
+    }
+    {
         if (uniform) {
             FIN.meta[br].flags = L.meta[br].flags | BM_UNIFORM;
             UniCoef u;
@@ -3158,22 +3313,6 @@ __global__ __launch_bounds__(BOTTOM_THREADS) void k_bottom(const BottomGrid *__r
 }
 
 // ------------------------------------------------------------------------------ output (one grid)
-// m_pressure: dense float (and optional FP64) pressure, 0 off the unknowns
-// (macpressuresolver3.cpp:245-248).
-// With unknown_out, also the unknown mask (the labelling's cell flag, bit 1).
-__global__ void k_scatter_pressure(GridDesc G, LevelDesc L, GridLevel GL, const double *__restrict__ x, float *P,
-                                   double *P64, const uint8_t *__restrict__ cflag, uint8_t *unknown_out) {
-    const size_t M = (size_t)G.w * G.h * G.d;
-    const size_t c = (size_t)xcd_brick(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (c >= M) return;
-    int i, j, k;
-    unflatten((unsigned)c, (unsigned)G.h, (unsigned)G.d, i, j, k);
-    const double v = level_value(L, GL, x, i, j, k);
-    if (P) P[c] = (float)v;
-    if (P64) P64[c] = v;
-    if (unknown_out) unknown_out[c] = (cflag[c] >> 1) & 1;
-}
-
 // Dense export of the level-0 system: diag (0 off the unknowns), the low-face couplings and the
 // right-hand side, all cell-indexed.
 __global__ void k_export_system(GridDesc G, LevelDesc L, GridLevel GL, OpDesc<double> A, const double *__restrict__ b,
@@ -3197,78 +3336,231 @@ __global__ void k_export_system(GridDesc G, LevelDesc L, GridLevel GL, OpDesc<do
     rhs[c] = unk ? level_value(L, GL, b, i, j, k) : 0.0;
 }
 
-// Velocity update (macpressuresolver3.cpp:252-268) of the three faces indexed at node position
-// (i,j,k) in one thread (each level-set sample is read once for the three faces): open faces on
-// the domain boundary become 0, interior open faces lose dt*(P1-P0)/(rho*dx) with P stored in
-// float and P1-P0 taken in float; all other (active) faces are switched off (0).
-__device__ __forceinline__ void update_face(const GridDesc &G, const Exist &E, int dim, int i, int j, int k, float p1,
-                                            float p0, float rho_face) {
-#pragma clang fp contract(off)
-    const size_t f = face_index(G, dim, i, j, k);
-    uint8_t *aout = G.active_out[dim];
-    if (G.active[dim] && !G.active[dim][f]) {
-        if (aout) aout[f] = 0;
-        return;
-    }
-    const int pi[3] = {i, j, k};
-    const int N[3] = {G.w, G.h, G.d};
-    float *U = G.vel[dim];
-    // the area only matters where rho is nonzero: most faces of the domain have air on both sides
-    const double rho = rho_face;
-    const float area = rho != 0.0 ? face_area(G, E, dim, i, j, k) : 0.0f;
-    uint8_t keep = 1;
-    if (area != 0.0f && rho != 0.0) {
-        if (pi[dim] == 0 || pi[dim] == N[dim]) {
-            U[f] = 0.0f;
-        } else {
-            const float diff = p1 - p0;
-            const float delta = (float)(G.dt * (double)diff / (rho * G.dx));
-            U[f] = U[f] - delta;
-        }
-    } else {
-        U[f] = 0.0f;
-        // a closed boundary face stays active (at 0) where the cell inside holds liquid
-        if (pi[dim] == 0) keep = phi_at(G, i, j, k) < 0.0;
-        else if (pi[dim] == N[dim]) keep = phi_at(G, i - (dim == 0), j - (dim == 1), k - (dim == 2)) < 0.0;
-        else keep = 0;
-    }
-    if (aout) aout[f] = keep;
+// Output of a grid: m_pressure, the dense float (and optional FP64) pressure, 0 off the unknowns
+// (macpressuresolver3.cpp:245-248), the unknown mask (the labelling's cell flag, bit 1), and the velocity
+// update (:252-268): open interior faces lose dt*(P1-P0)/(rho*dx) with P stored in float and P1-P0
+// taken in float; all other (active) faces are switched off (0), as the domain's boundary faces are (their
+// area is 0), which stay active where the cell inside holds liquid.
+//
+// One pass for all of it, on columns of OUT_PLANES cells along x per thread and 64 consecutive cells of a
+// plane per wavefront (whatever the row length), so that the index arithmetic is done once per column, a
+// cell's low neighbour along x is in registers, and the pressure comes from the bricks instead of a dense
+// copy.  A wavefront with only air around (most of a domain) reads the level set and writes zeros.
+// Bound by its traffic: at 256^3 (28% liquid, FP64 samples) 176 us, 2.7 TB/s; a scatter and an update
+// with one node per thread took 46 + 223 us.  120x168x89, all liquid with activity masks: 41 us.
+struct OutputGrid {
+    GridDesc G;
+    GridLevel GL;
+    float *P;         // dense outputs (or nullptr)
+    double *P64, *scene;
+    const uint8_t *cflag;
+    uint8_t *unknown_out;
+};
+constexpr int OUT_THREADS = 256, OUT_PLANES = 4;
+static inline int output_blocks(const GridDesc &G) {
+    const unsigned HD = (unsigned)G.h * (unsigned)G.d;
+    return (int)((HD + OUT_THREADS - 1) / OUT_THREADS) * ((G.w + OUT_PLANES - 1) / OUT_PLANES);
 }
 
-// P is the grid's dense float pressure (0 off the unknowns), as k_scatter_pressure writes it.
-__global__ void k_velocity_update(GridDesc G, const float *__restrict__ P) {
-    const int W = G.w + 1, H = G.h + 1, D = G.d + 1;
-    const size_t n = (size_t)W * H * D;
-    const size_t e = (size_t)xcd_brick(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    int i, j, k;
-    unflatten((unsigned)e, (unsigned)H, (unsigned)D, i, j, k);
-    const bool in_i = i < G.w, in_j = j < G.h, in_k = k < G.d;
-    const float pc = (in_i && in_j && in_k) ? P[cell_index(G, i, j, k)] : 0.0f;
-    const Exist E = exist_of(G);
-    // face_rho of the three faces from four level-set samples, read once: the (clamped) node cell
-    // and the (clamped) cell below it along each axis
-    const bool v0 = in_j && in_k, v1 = in_i && in_k, v2 = in_i && in_j && !G.flat;
-    float rho[3] = {1.0f, 1.0f, 1.0f};
-    // the four samples and the three low-side pressures are loaded together; the clamped indices
-    // are in range for every node, and a face that does not exist never uses its values
-    const int ci = clampi(i, 0, G.w - 1), cj = clampi(j, 0, G.h - 1), ck = clampi(k, 0, G.d - 1);
-    const int ci1 = clampi(i - 1, 0, G.w - 1), cj1 = clampi(j - 1, 0, G.h - 1), ck1 = clampi(k - 1, 0, G.d - 1);
-    const size_t idx[4] = {cell_index(G, ci, cj, ck), cell_index(G, ci1, cj, ck), cell_index(G, ci, cj1, ck),
-                           cell_index(G, ci, cj, ck1)};
-    if (E.liquid) {
-        double sm[4];
-        load_samples<4>(G.phi, G.phi64, idx, sm);
-        rho[0] = rho_from_samples(G, E, sm[0], v0 ? sm[1] : 0.0);
-        rho[1] = rho_from_samples(G, E, sm[0], v1 ? sm[2] : 0.0);
-        rho[2] = rho_from_samples(G, E, sm[0], v2 ? sm[3] : 0.0);
-    } else {
-        rho[0] = rho[1] = rho[2] = rho_from_samples(G, E, 0.0, 0.0);
+// A face's new velocity and activity; an inactive face keeps its velocity.
+__device__ __forceinline__ void put_face(const GridDesc &G, int dim, size_t f, float u, bool keep) {
+    const bool inactive = G.active[dim] && !G.active[dim][f];
+    if (!inactive) G.vel[dim][f] = u;
+    if (G.active_out[dim]) G.active_out[dim][f] = keep && !inactive;
+}
+
+// Level set of a column from plane i0 - 1 on and of the low neighbours along y and z (clamped).
+struct OutputPhi {
+    double c[OUT_PLANES + 1], j[OUT_PLANES], k[OUT_PLANES];
+};
+template <class Tp>
+__device__ __forceinline__ void output_phi(const void *a, size_t c0, int n, size_t di, size_t dj, size_t dk, size_t HD,
+                                           OutputPhi &o) {
+    const Tp *__restrict__ phi = (const Tp *)a;
+    o.c[0] = (double)phi[c0 - di];
+#pragma unroll
+    for (int p = 0; p < OUT_PLANES; ++p) {
+        const size_t c = c0 + (size_t)(p < n ? p : 0) * HD;
+        o.c[p + 1] = (double)phi[c];
+        o.j[p] = (double)phi[c - dj];
+        o.k[p] = (double)phi[c - dk];
     }
-    const float px = P[idx[1]], py = P[idx[2]], pz = P[idx[3]];
-    if (v0) update_face(G, E, 0, i, j, k, pc, i > 0 ? px : 0.0f, rho[0]);
-    if (v1) update_face(G, E, 1, i, j, k, pc, j > 0 ? py : 0.0f, rho[1]);
-    if (v2) update_face(G, E, 2, i, j, k, pc, k > 0 ? pz : 0.0f, rho[2]);
+}
+
+__global__ __launch_bounds__(OUT_THREADS) void k_output(GridTable<OutputGrid> T, LevelDesc L,
+                                                        const double *__restrict__ x) {
+#pragma clang fp contract(off)
+    int local;
+    const int entry = table_grid(T, local);
+    if (entry < 0) return;
+    const OutputGrid &F = T.g[entry];
+    const GridDesc &G = F.G;
+    const unsigned HD = (unsigned)G.h * (unsigned)G.d, ne = (HD + OUT_THREADS - 1) / OUT_THREADS;
+    const unsigned slab = (unsigned)local / ne, e = ((unsigned)local - slab * ne) * OUT_THREADS + threadIdx.x;
+    if (e >= HD) return;
+    const int j = (int)(e / (unsigned)G.d), k = (int)(e - (unsigned)j * (unsigned)G.d);
+    const int i0 = (int)slab * OUT_PLANES, n = min(OUT_PLANES, G.w - i0);
+    const Exist E = exist_of(G);
+    const size_t c0 = cell_index(G, i0, j, k);
+    // the bricks of the column and of its low neighbours: the planes lie in one brick layer
+    const int *bm = L.bmap + F.GL.bmap_off;
+    const int layer = F.GL.nby * F.GL.nbz, at = (i0 >> 3) * layer + (j >> 3) * F.GL.nbz + (k >> 3);
+    const int b = bm[at];
+    const int bi = i0 == 0 ? -1 : (i0 & 7) ? b : bm[at - layer];
+    const int bj = j == 0 ? -1 : (j & 7) ? b : bm[at - F.GL.nbz];
+    const int bk = k == 0 ? -1 : (k & 7) ? b : bm[at - 1];
+    OutputPhi ph;
+    const size_t dj = j > 0 ? G.d : 0, dk = k > 0;
+    if (G.phi64) output_phi<double>(G.phi, c0, n, i0 > 0 ? HD : 0, dj, dk, HD, ph);
+    else output_phi<float>(G.phi, c0, n, i0 > 0 ? HD : 0, dj, dk, HD, ph);
+    // pressures of the column and of the low neighbours
+    double v[OUT_PLANES] = {};
+    float lx = 0.0f, ly[OUT_PLANES] = {}, lz[OUT_PLANES] = {};
+    const int cell = ((i0 & 7) * 8 + (j & 7)) * 8 + (k & 7);
+    if (b >= 0) {
+#pragma unroll
+        for (int p = 0; p < OUT_PLANES; ++p) v[p] = x[(long)b * BRICK_CELLS + cell + 64 * p];
+    }
+    if (bi >= 0) lx = (float)x[(long)bi * BRICK_CELLS + ((cell - 64) & 511)];
+    const int cj = (cell & ~56) | ((cell - 8) & 56), ck = (cell & ~7) | ((cell - 1) & 7);
+    if (bj >= 0) {
+#pragma unroll
+        for (int p = 0; p < OUT_PLANES; ++p) ly[p] = (float)x[(long)bj * BRICK_CELLS + cj + 64 * p];
+    }
+    if (bk >= 0) {
+#pragma unroll
+        for (int p = 0; p < OUT_PLANES; ++p) lz[p] = (float)x[(long)bk * BRICK_CELLS + ck + 64 * p];
+    }
+    bool air = ph.c[0] >= 0.0;
+#pragma unroll
+    for (int p = 0; p < OUT_PLANES; ++p) air = air && ph.c[p + 1] >= 0.0 && ph.j[p] >= 0.0 && ph.k[p] >= 0.0;
+    const bool quiet = E.liquid && __ballot(!air) == 0;  // every face around is closed
+#pragma unroll
+    for (int p = 0; p < OUT_PLANES; ++p) {
+        if (p >= n) break;
+        const size_t c = c0 + (size_t)p * HD;
+        if (F.P) F.P[c] = (float)v[p];
+        if (F.P64) F.P64[c] = v[p];
+        if (F.scene) F.scene[c] = v[p];
+        if (F.unknown_out) F.unknown_out[c] = (F.cflag[c] >> 1) & 1;
+    }
+    const bool last_j = j == G.h - 1, last_k = k == G.d - 1 && !G.flat;
+    const size_t f0[3] = {c0, c0 + (size_t)i0 * G.d, c0 + (size_t)((unsigned)i0 * G.h + j)};
+    const size_t df[3] = {HD, HD + G.d, HD + G.h};
+    // no activity in or out: plain stores
+    const bool plain = !(G.active[0] || G.active[1] || G.active[2] || G.active_out[0] || G.active_out[1] || G.active_out[2]);
+    if (quiet) {
+#pragma unroll
+        for (int p = 0; p < OUT_PLANES; ++p) {
+            if (p >= n) break;
+            if (plain) {
+                G.vel[0][f0[0] + p * df[0]] = 0.0f;
+                G.vel[1][f0[1] + p * df[1]] = 0.0f;
+                if (!G.flat) G.vel[2][f0[2] + p * df[2]] = 0.0f;
+            } else {
+                put_face(G, 0, f0[0] + p * df[0], 0.0f, false);
+                put_face(G, 1, f0[1] + p * df[1], 0.0f, false);
+                if (!G.flat) put_face(G, 2, f0[2] + p * df[2], 0.0f, false);
+            }
+            if (i0 + p == G.w - 1) put_face(G, 0, f0[0] + (p + 1) * HD, 0.0f, false);
+            if (last_j) put_face(G, 1, f0[1] + p * df[1] + G.d, 0.0f, false);
+            if (last_k) put_face(G, 2, f0[2] + p * df[2] + 1, 0.0f, false);
+        }
+        return;
+    }
+    // interior low faces (bit 3 p + dim) that are not shut by the solid; the area only matters where the
+    // liquid fraction is nonzero
+    unsigned open = 0;
+#pragma unroll
+    for (int p = 0; p < OUT_PLANES; ++p) {
+        const bool dry = E.liquid && ph.c[p + 1] >= 0.0;
+        if (p < n) {
+            if (i0 + p > 0 && !(dry && ph.c[p] >= 0.0)) open |= 1u << (3 * p);
+            if (j > 0 && !(dry && ph.j[p] >= 0.0)) open |= 2u << (3 * p);
+            if (k > 0 && !(dry && ph.k[p] >= 0.0)) open |= 4u << (3 * p);
+        }
+    }
+    if (G.solid && __ballot(open != 0)) {
+        // signs of the column's nodes at its four corners: a face with no corner in the solid is whole, one
+        // with all four has none; only the others' areas are formed
+        unsigned s00, s01, s10, s11;
+        const size_t stride = G.flat ? (size_t)(G.h + 1) : (size_t)((unsigned)(G.h + 1) * (unsigned)(G.d + 1));
+        const size_t n00 = G.flat ? (size_t)((unsigned)i0 * (unsigned)(G.h + 1) + (unsigned)j) : node_index(G, i0, j, k);
+        const size_t up = G.flat ? 1 : (size_t)(G.d + 1), right = G.flat ? 0 : 1;
+        if (G.solid64) {
+            s00 = node_bits<double, OUT_PLANES>(G.solid, n00, n, stride), s01 = node_bits<double, OUT_PLANES>(G.solid, n00 + right, n, stride);
+            s10 = node_bits<double, OUT_PLANES>(G.solid, n00 + up, n, stride);
+            s11 = node_bits<double, OUT_PLANES>(G.solid, n00 + up + right, n, stride);
+        } else {
+            s00 = node_bits<float, OUT_PLANES>(G.solid, n00, n, stride), s01 = node_bits<float, OUT_PLANES>(G.solid, n00 + right, n, stride);
+            s10 = node_bits<float, OUT_PLANES>(G.solid, n00 + up, n, stride);
+            s11 = node_bits<float, OUT_PLANES>(G.solid, n00 + up + right, n, stride);
+        }
+        unsigned part = 0;
+#pragma unroll
+        for (int p = 0; p < OUT_PLANES; ++p) {
+            auto face = [&](int dim, unsigned any, unsigned all) {
+                const unsigned bit = 1u << (3 * p + dim);
+                if (all & 1) open &= ~bit;
+                else if (any & 1) part |= bit;
+            };
+            const unsigned a = s00 >> p, b = s01 >> p, c = s10 >> p, d = s11 >> p;
+            face(0, a | b | c | d, a & b & c & d);
+            face(1, a | b | (a | b) >> 1, a & b & (a & b) >> 1);
+            if (!G.flat) face(2, a | c | (a | c) >> 1, a & c & (a & c) >> 1);
+        }
+        for (unsigned left = open & part; left; left &= left - 1) {
+            const int bit = __ffs((int)left) - 1, p = bit / 3;
+            if (face_area(G, E, bit - 3 * p, i0 + p, j, k) == 0.0f) open &= ~(1u << bit);
+        }
+    }
+    // the velocities of the open faces, loaded together
+    float *const U[3] = {G.vel[0], G.vel[1], G.vel[2]};
+    float u[OUT_PLANES][3];
+#pragma unroll
+    for (int p = 0; p < OUT_PLANES; ++p) {
+#pragma unroll
+        for (int dim = 0; dim < 3; ++dim) {
+            u[p][dim] = 0.0f;
+            if (open >> (3 * p + dim) & 1) u[p][dim] = U[dim][f0[dim] + p * df[dim]];
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < OUT_PLANES; ++p) {
+        const double c = ph.c[p + 1], low[3] = {ph.c[p], ph.j[p], ph.k[p]};
+        const float p1 = (float)v[p], p0[3] = {p ? (float)v[p ? p - 1 : 0] : lx, ly[p], lz[p]};
+#pragma unroll
+        for (int dim = 0; dim < 3; ++dim) {
+            if (!(open >> (3 * p + dim) & 1)) continue;
+            const double rho = rho_from_samples(G, E, c, low[dim]);
+            if (rho != 0.0) {
+                const float diff = p1 - p0[dim];
+                const float delta = (float)(G.dt * (double)diff / (rho * G.dx));
+                u[p][dim] = u[p][dim] - delta;
+            } else {
+                u[p][dim] = 0.0f;
+                open &= ~(1u << (3 * p + dim));
+            }
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < OUT_PLANES; ++p) {
+        if (p >= n) break;
+        const int i = i0 + p;
+        const bool liquid = ph.c[p + 1] < 0.0;
+        const int edge[3] = {i, j, k};
+#pragma unroll
+        for (int dim = 0; dim < 3; ++dim) {
+            if (dim == 2 && G.flat) continue;
+            const size_t f = f0[dim] + p * df[dim];
+            if (plain) U[dim][f] = u[p][dim];
+            else put_face(G, dim, f, u[p][dim], (open >> (3 * p + dim) & 1) || (edge[dim] == 0 && liquid));
+        }
+        // the domain's high faces
+        if (i == G.w - 1) put_face(G, 0, f0[0] + (p + 1) * HD, 0.0f, liquid);
+        if (last_j) put_face(G, 1, f0[1] + p * df[1] + G.d, 0.0f, liquid);
+        if (last_k) put_face(G, 2, f0[2] + p * df[2] + 1, 0.0f, liquid);
+    }
 }
 
 }  // namespace shkz

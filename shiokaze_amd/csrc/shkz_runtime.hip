@@ -6,7 +6,7 @@
 //   assembly (matrix-free)         k_operator, k_coarsen, k_idiag        (:159-199)
 //   volume correction, warm start  host PI controller, scene state       (:203-230, :239-242)
 //   linear solve                   CG / MGPCG / mixed-precision MGPCG    (:233-237 -> pcg.cpp:45-73)
-//   scatter + velocity update      k_scatter_pressure, k_velocity_update (:245-268)
+//   pressure + velocity update     k_output                             (:245-268)
 // A call may project a batch of independent grids at once.  Their stored bricks are concatenated
 // into one tile table per multigrid level, so every solver launch covers every grid of the batch,
 // while reductions, scalars, convergence and the multigrid depth stay per grid: each grid's result
@@ -599,6 +599,20 @@ static inline unsigned brick_grid(int nbricks) { return (unsigned)(((nbricks + 7
 // Blocks of `per` threads over n items, a multiple of 8 (kernels remap block ids XCD-aware and
 // bounds-check the index).
 static inline unsigned xcd_blocks(size_t n, unsigned per) { return (unsigned)((((n + per - 1) / per) + 7) / 8 * 8); }
+
+// Launches a kernel over the grids of a batch, GRIDS_PER_LAUNCH of them at a time: describe(g, entry,
+// bytes) fills grid g's entry, adds its bytes to the timing model and returns its workgroups.
+template <class D, class Describe, class... P, class... Args>
+static void launch_grids(Launcher &K, const char *name, int ngrids, int threads, Describe describe,
+                         void (*kernel)(GridTable<D>, P...), Args... args) {
+    for (int g0 = 0; g0 < ngrids; g0 += GRIDS_PER_LAUNCH) {
+        GridTable<D> T{};
+        double bytes = 0;
+        T.n = std::min(GRIDS_PER_LAUNCH, ngrids - g0);
+        for (int q = 0; q < T.n; ++q) T.first[q + 1] = T.first[q] + describe(g0 + q, T.g[q], bytes);
+        K.go(name, -1, 0, bytes, dim3(brick_grid(T.first[T.n])), dim3((unsigned)threads), kernel, T, args...);
+    }
+}
 
 // Resolves pending timing events into totals (after a stream synchronisation).
 static void resolve_timing(shkz_ctx *C) {
@@ -1782,8 +1796,12 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
     SHKZ_TRY(arena_get(AR, "cflag", cflag_total, &cflag_all));
     SHKZ_TRY(arena_get(AR, "bflag", bflag_total, &bflag_all));
     SHKZ_TRY(arena_get(AR, "exist", (size_t)4 * ngrids, &exist_all));
-    K.go("reset", -1, 0, 16.0 * ngrids, dim3((unsigned)((4 * ngrids + 255) / 256)), dim3(256), k_reset_ints, exist_all,
-         4 * ngrids);
+    // levelset_exist() of the liquid: the labelling finds it on the way (read back with the brick flags),
+    // unless surface tension needs it first (the solid needs no scan, as the face fractions show)
+    const bool scan_liquid = prm->surface_tension != 0.0;
+    if (scan_liquid)
+        K.go("reset", -1, 0, 16.0 * ngrids, dim3((unsigned)((4 * ngrids + 255) / 256)), dim3(256), k_reset_ints,
+             exist_all, 4 * ngrids);
     for (int g = 0; g < ngrids; ++g) {
         GridJob &J = jobs[g];
         const shkz_grid *grid = &grids[g];
@@ -1816,10 +1834,6 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
         G.flat = flat ? 1 : 0;
         J.exist = exist_all + 4 * g;
         G.exist = J.exist;
-        // levelset_exist() of the liquid: the labelling finds it on the way (read back with the brick
-        // flags), unless surface tension needs it first (the solid needs no scan, as the face
-        // fractions show)
-        const bool scan_liquid = prm->surface_tension != 0.0;
         if (scan_liquid) {
             const unsigned nbk = (unsigned)std::min<size_t>((J.M + 255) / 256, 4096);
             K.go("any_negative", -1, 0, (double)J.M * (G.phi64 ? 8 : 4), dim3(nbk), dim3(256), k_any_negative,
@@ -1840,12 +1854,17 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
             }
         }
         grid_level_dims(J.l0, w, h, d);
-        const int npos = J.l0.nbx * J.l0.nby * J.l0.nbz;
         J.cflag = cflag_all + cflag_off[g];
         J.bflag = bflag_all + bflag_off[g];
-        K.go("flags", -1, 0, (double)J.M * ((G.phi64 ? 8 : 4) + 1 + (grid->solid ? 4 : 0)), dim3(brick_grid(npos)),
-             dim3(BLOCK), k_flags, G, J.l0.nbx, J.l0.nby, J.l0.nbz, J.cflag, J.bflag);
     }
+    launch_grids<FlagsGrid>(K, "flags", ngrids, FLAGS_THREADS,
+                            [&](int g, FlagsGrid &F, double &bytes) {
+                                GridJob &J = jobs[g];
+                                F = FlagsGrid{J.G, J.l0.nbx, J.l0.nby, J.l0.nbz, J.cflag, J.bflag};
+                                bytes += (double)J.M * ((J.G.phi64 ? 8 : 4) + 1 + (J.in->solid ? 4 : 0));
+                                return flags_blocks(F);
+                            },
+                            k_flags);
     const double t_queued = now_ms();
     {
         void *hflags = nullptr;
@@ -2040,15 +2059,21 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
             J.rhs_correct = -(kp * xv + ki * y) / (xv + 1.0);
         }
         res[g].rhs_correct = J.rhs_correct;
-        const double *warm = (prm->warm_start && J.scene && J.scene->has_pressure) ? J.scene->p : nullptr;
-        const GridLevel &GL = F0.gl[g];
-        const int nbg = GL.brick_end - GL.brick_start;
-        K.go("operator", -1, 0,
-             (double)nbg * BRICK_CELLS *
-                 ((J.G.phi64 ? 8 : 4) + (grid->solid ? 4 : 0) + 12 + 1 + 6 * 8 + (P.mixed ? 16 : 0)),
-             dim3(brick_grid(nbg)), dim3(BLOCK), k_operator, J.G, F0.desc, GL, (const uint8_t *)J.cflag, P.dir64,
-             P.gx64, P.gy64, P.gz64, dir32, gx32, gy32, gz32, P.b64, P.x64, warm, J.rhs_correct, FIN);
     }
+    launch_grids<OperatorGrid>(K, "operator", ngrids, BLOCK,
+                               [&](int g, OperatorGrid &F, double &bytes) {
+                                   GridJob &J = jobs[g];
+                                   const double *warm = (prm->warm_start && J.scene && J.scene->has_pressure)
+                                                            ? J.scene->p : nullptr;
+                                   F = OperatorGrid{J.G, F0.gl[g], J.cflag, warm, J.rhs_correct};
+                                   const int nbg = F.GL.brick_end - F.GL.brick_start;
+                                   bytes += (double)nbg * BRICK_CELLS *
+                                            ((J.G.phi64 ? 8 : 4) + (J.in->solid ? 4 : 0) + 12 + 1 + 6 * 8 +
+                                             (P.mixed ? 16 : 0));
+                                   return nbg;
+                               },
+                               k_operator, F0.desc, P.dir64, P.gx64, P.gy64, P.gz64, dir32, gx32, gy32, gz32, P.b64,
+                               P.x64, FIN);
     // the coarser levels and the transfer tables, built on the host while the assembly runs
     const double t_assembly = now_ms();
     int max_bricks = 8;
@@ -2347,29 +2372,20 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
     const double t_solve = now_ms();
 
     // ---------------------------------------------------------------- per grid: scatter + update
-    float *pdense = nullptr;
-    {
-        size_t maxM = 1;
-        for (const GridJob &J : jobs) maxM = std::max(maxM, J.M);
-        SHKZ_TRY(arena_get(AR, "pdense", maxM, &pdense));
-    }
+    launch_grids<OutputGrid>(K, "output", ngrids, OUT_THREADS,
+                             [&](int g, OutputGrid &F, double &bytes) {
+                                 GridJob &J = jobs[g];
+                                 const shkz_grid *in = J.in;
+                                 F = OutputGrid{J.G, F0.gl[g], in->pressure, in->pressure64,
+                                                J.scene ? J.scene->p : nullptr, J.cflag, in->unknown_out};
+                                 bytes += (double)J.M * (24 + (J.G.phi64 ? 8 : 4) + (in->solid ? 4 : 0) +
+                                                         (in->pressure ? 4 : 0) + (in->pressure64 ? 8 : 0) +
+                                                         (J.scene ? 8 : 0) + (in->unknown_out ? 2 : 0));
+                                 return output_blocks(J.G);
+                             },
+                             k_output, F0.desc, (const double *)P.x64);
     for (int g = 0; g < ngrids; ++g) {
         GridJob &J = jobs[g];
-        const shkz_grid *grid = J.in;
-        const GridLevel &GL = F0.gl[g];
-        // the velocity update reads a dense float pressure: the caller's, or the scratch array
-        float *P32 = grid->pressure ? grid->pressure : pdense;
-        uint8_t *unk_out = grid->unknown_out;
-        K.go("scatter_pressure", -1, 0, (double)J.M * (4 + (grid->pressure64 ? 8 : 0) + (unk_out ? 2 : 0)),
-             dim3(xcd_blocks(J.M, 256)), dim3(256), k_scatter_pressure, J.G, F0.desc, GL, (const double *)P.x64, P32,
-             grid->pressure64, (const uint8_t *)J.cflag, unk_out);
-        if (J.scene)
-            K.go("scatter_pressure", -1, 0, (double)J.M * 8, dim3(xcd_blocks(J.M, 256)), dim3(256),
-                 k_scatter_pressure, J.G, F0.desc, GL, (const double *)P.x64, (float *)nullptr, J.scene->p,
-                 (const uint8_t *)nullptr, (uint8_t *)nullptr);
-        const size_t ne = (size_t)(grid->w + 1) * (grid->h + 1) * (grid->d + 1);
-        K.go("velocity_update", -1, 0, (double)J.M * (24 + 4 + (J.G.phi64 ? 8 : 4) + (grid->solid ? 4 : 0)),
-             dim3(xcd_blocks(ne, 256)), dim3(256), k_velocity_update, J.G, (const float *)P32);
         if (J.scene) J.scene->has_pressure = true;
         res[g].iterations = total_iters[g];
         res[g].outer_iterations = outer_passes[g];

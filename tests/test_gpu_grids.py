@@ -1,0 +1,86 @@
+"""The per-grid kernels (labelling, assembly, output) at the edges of their tiles: unknown set, right-hand
+side, activity and velocity update equal to the oracle's, bit for bit, on rough level sets (every combination
+of signs around a face, zeros included) at sizes around a brick, a row of 32 cells, a column of 4
+planes and 256 cells of a plane; and more grids than one launch takes, each as when projected alone.
+"""
+import numpy as np
+import pytest
+
+import shiokaze_amd as S
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 1), (2, 9, 3), (4, 7, 31), (5, 8, 32), (8, 17, 33), (9, 16, 16), (13, 3, 65), (17, 33, 8), (3, 2, 130)]
+SHAPES_2D = [(1, 1), (7, 255), (9, 256), (16, 257), (33, 8), (5, 300)]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = S.Context(0)
+    yield c
+    c.close()
+
+
+def rough(shape, rng, dtype):
+    a = rng.standard_normal(shape) - 0.4
+    a[rng.random(shape) < 0.05] = 0.0
+    return a.astype(dtype)
+
+
+def scene(shape, seed, solid):
+    rng = np.random.default_rng(seed)
+    flat = len(shape) == 2
+    sc = (S.make_scene2d if flat else S.make_scene)(S.SCENE_DROP_SOLIDS, *shape, seed=seed)
+    sc.fluid = rough(sc.fluid.shape, rng, (np.float32, np.float64)[seed % 2])
+    sc.solid = rough(tuple(n + 1 for n in shape), rng, (np.float32, np.float64)[seed // 2 % 2]) + 0.3 if solid else None
+    if sc.solid is not None:
+        sc.solid = sc.solid.astype((np.float32, np.float64)[seed // 2 % 2])
+    for f in (sc.u, sc.v) if flat else (sc.u, sc.v, sc.wv):
+        f[...] = rng.standard_normal(f.shape).astype(np.float32)
+    return sc
+
+
+@pytest.mark.parametrize("solid", [False, True])
+@pytest.mark.parametrize("shape", SHAPES + SHAPES_2D)
+def test_grid_kernels_match_oracle(ctx, shape, solid):
+    print(f"[gpu-case] grid kernels {shape} solid={solid}", flush=True)
+    sc = scene(shape, sum(shape), solid)
+    flat = len(shape) == 2
+    A = (O.assemble2 if flat else O.assemble)(sc)
+    unk = A["index_map"] >= 0
+    exp = (ctx.export_system2d if flat else ctx.export_system)(sc)
+    assert np.array_equal(exp["diag"] > 0, unk)
+    assert np.array_equal(exp["rhs"][unk][np.argsort(A["index_map"][unk])], A["b"])
+    work, ref = sc.copy(), sc.copy()
+    prm = S.default_params(residual=1e-1)
+    if flat:
+        r, P, _ = ctx.project2d(work, prm)
+        O.velocity_update2(ref, P, A["area"], A["rho"])
+        pairs = [(work.u, ref.u), (work.v, ref.v)]
+    else:
+        act = [np.full(s, 7, np.uint8) for s in O.face_shapes(*shape)]
+        mask = np.full(shape, 7, np.uint8)
+        r, P, _ = ctx.project(work, prm, active_out=act, unknown_out=mask)
+        act_o = O.velocity_update(ref, P, A["area"], A["rho"], active_out=True)
+        assert np.array_equal(mask, unk.astype(np.uint8))
+        pairs = [(work.u, ref.u), (work.v, ref.v), (work.wv, ref.wv)] + list(zip(act, act_o))
+    assert r.status == 0
+    assert not P[~unk].any()
+    for a, b in pairs:
+        assert np.array_equal(a, b)
+
+
+def test_more_grids_than_one_launch(ctx):
+    shapes = SHAPES[1:] + [s[::-1] for s in SHAPES[1:]]
+    scenes = [scene(s, 100 + i, i % 2 == 1) for i, s in enumerate(shapes)]
+    alone = []
+    for sc in scenes:
+        one = sc.copy()
+        r, P, P64 = ctx.project(one, S.default_params(residual=1e-6), pressure64=True)
+        alone.append((one, P, P64))
+    work = [sc.copy() for sc in scenes]
+    res, Ps, P64s = ctx.project_batch(work, S.default_params(residual=1e-6), pressure64=True)
+    for w, (one, P, P64), bP, bP64 in zip(work, alone, Ps, P64s):
+        assert np.array_equal(P, bP) and np.array_equal(P64, bP64)
+        assert np.array_equal(w.u, one.u) and np.array_equal(w.v, one.v) and np.array_equal(w.wv, one.wv)
