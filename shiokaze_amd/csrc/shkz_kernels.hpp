@@ -1256,16 +1256,13 @@ constexpr int ROW4_THREADS = ROW4_GROUP;
 __device__ __forceinline__ float4 ld4(const float *__restrict__ a, long i) {
     return *reinterpret_cast<const float4 *>(a + i);
 }
-__device__ __forceinline__ float4 ld4z(const float *__restrict__ a, long i) {
-    return i >= 0 ? ld4(a, i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-}
 __device__ __forceinline__ void unpack4(const float4 v, float o[4]) {
     o[0] = v.x;
     o[1] = v.y;
     o[2] = v.z;
     o[3] = v.w;
 }
-// Four consecutive values (16-byte loads: one float4 or two double2), zeros where i < 0.
+// Four consecutive values (16-byte loads: one float4 or two double2).
 __device__ __forceinline__ void load4(const float *__restrict__ a, long i, float o[4]) { unpack4(ld4(a, i), o); }
 __device__ __forceinline__ void load4(const double *__restrict__ a, long i, double o[4]) {
     const double2 u = *reinterpret_cast<const double2 *>(a + i), w = *reinterpret_cast<const double2 *>(a + i + 2);
@@ -1273,15 +1270,6 @@ __device__ __forceinline__ void load4(const double *__restrict__ a, long i, doub
     o[1] = u.y;
     o[2] = w.x;
     o[3] = w.y;
-}
-template <class T>
-__device__ __forceinline__ void load4z(const T *__restrict__ a, long i, T o[4]) {
-    if (i >= 0) {
-        load4(a, i, o);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = T(0);
-    }
 }
 __device__ __forceinline__ void store4(float *__restrict__ a, long i, const float v[4]) {
     *reinterpret_cast<float4 *>(a + i) = make_float4(v[0], v[1], v[2], v[3]);
@@ -1291,51 +1279,109 @@ __device__ __forceinline__ void store4(double *__restrict__ a, long i, const dou
     *reinterpret_cast<double2 *>(a + i + 2) = make_double2(v[2], v[3]);
 }
 
+// The value of the pair's other lane (q ^ 1), a register move.
+__device__ __forceinline__ float swap_pairs(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), DPP_QUAD_1032, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double swap_pairs(double v) { return dpp_move<DPP_QUAD_1032>(v); }
+
 // The six neighbour rows of lane q's cells: x and y neighbours as whole rows (index of their first
-// cell, -1 where no brick is stored), z neighbours as the row shifted by one cell.
+// cell), z neighbours as the row shifted by one cell.
+//
+// On the coarse levels a wavefront has its SIMD nearly to itself, and a kernel's time is its longest
+// chain of instructions and round trips: the indices are formed by selects and always in range, so that no load
+// waits behind a branch; where no brick is stored (out*) the value is set to 0 afterwards.
 struct Row4Nbrs {
     long c, ixm, ixp, iym, iyp, iz;  // iz: the end cell across the z face (k = -1 for h = 0, 8 for h = 1)
+    bool outxm, outxp, outym, outyp, outz;
+    bool edge;  // any of them, on any lane of the brick
     int h;
 };
 __device__ __forceinline__ Row4Nbrs row4_nbrs(const BrickMeta &m, int br, int q) {
     Row4Nbrs N;
     const int li = q >> 4, lj = (q >> 1) & 7, h = q & 1;
     const int o = li * 64 + lj * 8 + 4 * h;
+    const long own = (long)br * BRICK_CELLS;
+    auto base = [&](int d) { return m.nbr[d] >= 0 ? (long)m.nbr[d] * BRICK_CELLS : own; };
+    // (both sides formed before the choice: a select, not a branch)
+    const long xm = base(NB_XM) + 448, xp = base(NB_XP) - 448, ym = base(NB_YM) + 56, yp = base(NB_YP) - 56;
+    const long zm = base(NB_ZM) + 7, zp = base(NB_ZP) - 4;
+    const long xl = own - 64, xh = own + 64, yl = own - 8, yh = own + 8;
+    const int nzm = m.nbr[NB_ZM], nzp = m.nbr[NB_ZP];
     N.h = h;
-    N.c = (long)br * BRICK_CELLS + o;
-    N.ixm = li > 0 ? N.c - 64 : (m.nbr[NB_XM] >= 0 ? (long)m.nbr[NB_XM] * BRICK_CELLS + o + 448 : -1);
-    N.ixp = li < 7 ? N.c + 64 : (m.nbr[NB_XP] >= 0 ? (long)m.nbr[NB_XP] * BRICK_CELLS + o - 448 : -1);
-    N.iym = lj > 0 ? N.c - 8 : (m.nbr[NB_YM] >= 0 ? (long)m.nbr[NB_YM] * BRICK_CELLS + o + 56 : -1);
-    N.iyp = lj < 7 ? N.c + 8 : (m.nbr[NB_YP] >= 0 ? (long)m.nbr[NB_YP] * BRICK_CELLS + o - 56 : -1);
-    const int nz = h ? m.nbr[NB_ZP] : m.nbr[NB_ZM];
-    N.iz = nz >= 0 ? (long)nz * BRICK_CELLS + li * 64 + lj * 8 + (h ? 0 : 7) : -1;
+    N.c = own + o;
+    N.ixm = (li > 0 ? xl : xm) + o;
+    N.ixp = (li < 7 ? xh : xp) + o;
+    N.iym = (lj > 0 ? yl : ym) + o;
+    N.iyp = (lj < 7 ? yh : yp) + o;
+    N.iz = (h ? zp : zm) + o;
+    N.outxm = li == 0 && m.nbr[NB_XM] < 0;
+    N.outxp = li == 7 && m.nbr[NB_XP] < 0;
+    N.outym = lj == 0 && m.nbr[NB_YM] < 0;
+    N.outyp = lj == 7 && m.nbr[NB_YP] < 0;
+    N.outz = (h ? nzp : nzm) < 0;
+    N.edge = (m.nbr[NB_XM] | m.nbr[NB_XP] | m.nbr[NB_YM] | m.nbr[NB_YP] | m.nbr[NB_ZM] | m.nbr[NB_ZP]) < 0;
     return N;
 }
+template <class T>
+__device__ __forceinline__ void zero4(bool out, T v[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = out ? T(0) : v[j];
+}
 
-// The values of v at the six neighbours of the lane's four cells (0 where no brick is stored).
+// The values of v at the six neighbours of the lane's four cells (0 where no brick is stored): the loads,
+// and what follows once they are there (row4_join), apart so that other loads can be issued in between.
+template <class T>
+struct Row4Raw {
+    T c[4], xm[4], xp[4], ym[4], yp[4], end;
+};
 template <class T>
 struct Row4Vals {
     T c[4], xm[4], xp[4], ym[4], yp[4], zm[4], zp[4];
 };
 template <class T>
-__device__ __forceinline__ Row4Vals<T> row4_vals(const T *__restrict__ v, const Row4Nbrs &N) {
-    Row4Vals<T> o;
+__device__ __forceinline__ Row4Raw<T> row4_load(const T *__restrict__ v, const Row4Nbrs &N) {
+    Row4Raw<T> o;
     load4(v, N.c, o.c);
-    load4z(v, N.ixm, o.xm);
-    load4z(v, N.ixp, o.xp);
-    load4z(v, N.iym, o.ym);
-    load4z(v, N.iyp, o.yp);
-    const T end = N.iz >= 0 ? v[N.iz] : T(0);
+    load4(v, N.ixm, o.xm);
+    load4(v, N.ixp, o.xp);
+    load4(v, N.iym, o.ym);
+    load4(v, N.iyp, o.yp);
+    o.end = v[N.iz];
+    return o;
+}
+template <class T>
+__device__ __forceinline__ Row4Vals<T> row4_join(Row4Raw<T> r, const Row4Nbrs &N) {
+    if (N.edge) {
+        zero4(N.outxm, r.xm);
+        zero4(N.outxp, r.xp);
+        zero4(N.outym, r.ym);
+        zero4(N.outyp, r.yp);
+        r.end = N.outz ? T(0) : r.end;
+    }
+    Row4Vals<T> o;
     // lane swap: h = 0 receives the cell k = 4 of its partner, h = 1 the cell k = 3
-    const T swap = __shfl_xor(N.h ? o.c[0] : o.c[3], 1, 64);
-    o.zm[0] = N.h ? swap : end;
-    o.zp[3] = N.h ? end : swap;
+    const T swap = swap_pairs(N.h ? r.c[0] : r.c[3]);
+    o.zm[0] = N.h ? swap : r.end;
+    o.zp[3] = N.h ? r.end : swap;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        o.c[j] = r.c[j];
+        o.xm[j] = r.xm[j];
+        o.xp[j] = r.xp[j];
+        o.ym[j] = r.ym[j];
+        o.yp[j] = r.yp[j];
+    }
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-        o.zm[j + 1] = o.c[j];
-        o.zp[j] = o.c[j + 1];
+        o.zm[j + 1] = r.c[j];
+        o.zp[j] = r.c[j + 1];
     }
     return o;
+}
+template <class T>
+__device__ __forceinline__ Row4Vals<T> row4_vals(const T *__restrict__ v, const Row4Nbrs &N) {
+    return row4_join(row4_load(v, N), N);
 }
 
 // The couplings of the lane's cells: low faces from the cell itself, high faces from the next cell
@@ -1345,19 +1391,45 @@ struct Row4Coef {
     T gxm[4], gym[4], gzm[4], gxp[4], gyp[4], gzp[4];
 };
 template <class T>
-__device__ __forceinline__ Row4Coef<T> row4_coef(const OpDesc<T> &A, const Row4Nbrs &N) {
-    Row4Coef<T> o;
+struct Row4CoefRaw {
+    T gxm[4], gym[4], gzm[4], gxp[4], gyp[4], end;
+};
+template <class T>
+__device__ __forceinline__ Row4CoefRaw<T> row4_coef_load(const OpDesc<T> &A, const Row4Nbrs &N) {
+    Row4CoefRaw<T> o;
     load4(A.gx, N.c, o.gxm);
     load4(A.gy, N.c, o.gym);
     load4(A.gz, N.c, o.gzm);
-    load4z(A.gx, N.ixp, o.gxp);
-    load4z(A.gy, N.iyp, o.gyp);
-    const T end = (N.h && N.iz >= 0) ? A.gz[N.iz] : T(0);  // the coupling across k = 8
-    const T swap = __shfl_xor(o.gzm[0], 1, 64);            // h = 0: the partner's k = 4
-#pragma unroll
-    for (int j = 0; j < 3; ++j) o.gzp[j] = o.gzm[j + 1];
-    o.gzp[3] = N.h ? end : swap;
+    load4(A.gx, N.ixp, o.gxp);
+    load4(A.gy, N.iyp, o.gyp);
+    o.end = A.gz[N.iz];  // (h = 1: the coupling across k = 8)
     return o;
+}
+template <class T>
+__device__ __forceinline__ Row4Coef<T> row4_coef_join(Row4CoefRaw<T> r, const Row4Nbrs &N) {
+    if (N.edge) {
+        zero4(N.outxp, r.gxp);
+        zero4(N.outyp, r.gyp);
+        r.end = N.outz ? T(0) : r.end;
+    }
+    Row4Coef<T> o;
+    const T swap = swap_pairs(r.gzm[0]);  // h = 0: the partner's k = 4
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        o.gxm[j] = r.gxm[j];
+        o.gym[j] = r.gym[j];
+        o.gzm[j] = r.gzm[j];
+        o.gxp[j] = r.gxp[j];
+        o.gyp[j] = r.gyp[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) o.gzp[j] = r.gzm[j + 1];
+    o.gzp[3] = N.h ? r.end : swap;
+    return o;
+}
+template <class T>
+__device__ __forceinline__ Row4Coef<T> row4_coef(const OpDesc<T> &A, const Row4Nbrs &N) {
+    return row4_coef_join(row4_coef_load(A, N), N);
 }
 
 // jacobi_brick on the lane's four cells (same per-cell arithmetic); DOT adds rhs.zout of the
@@ -1368,11 +1440,12 @@ __device__ __forceinline__ void jacobi_row4(const LevelDesc &L, const OpDesc<T> 
                                             T *__restrict__ zout, T omega, int br, const BrickMeta &m, int q,
                                             double &part) {
     const Row4Nbrs N = row4_nbrs(m, br, q);
-    const Row4Vals<T> z = row4_vals(zin, N);
+    const Row4Raw<T> raw = row4_load(zin, N);
     T r[4], out[4];
     load4(rhs, N.c, r);
     if (m.flags & BM_UNIFORM) {
         const UniT<T> u = uni_load<T>(L, br);
+        const Row4Vals<T> z = row4_join(raw, N);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const T off = u.g * z.xm[j] + u.g * z.xp[j] + u.g * z.ym[j] + u.g * z.yp[j] + u.g * z.zm[j] +
@@ -1381,9 +1454,11 @@ __device__ __forceinline__ void jacobi_row4(const LevelDesc &L, const OpDesc<T> 
             if (DOT) part += (double)r[j] * (double)out[j];
         }
     } else {
-        const Row4Coef<T> g = row4_coef(A, N);
+        const Row4CoefRaw<T> graw = row4_coef_load(A, N);
         T id[4];
         load4(idiag, N.c, id);
+        const Row4Vals<T> z = row4_join(raw, N);
+        const Row4Coef<T> g = row4_coef_join(graw, N);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const T off = g.gxm[j] * z.xm[j] + g.gxp[j] * z.xp[j] + g.gym[j] * z.ym[j] + g.gyp[j] * z.yp[j] +
@@ -1396,7 +1471,7 @@ __device__ __forceinline__ void jacobi_row4(const LevelDesc &L, const OpDesc<T> 
     store4(zout, N.c, out);
 }
 
-// Sweep: workgroups take blockDim.x / 128 consecutive bricks per virtual block (virtual blocks
+// Sweep: workgroups take 4 (coarse levels: 1) consecutive bricks per virtual block (virtual blocks
 // vb = blockIdx.x + k * gridDim.x < nvirt, nvirt a multiple of 8, XCD-preserving); each wavefront
 // works alone on half a brick (no barrier).  Bound by the latency of its loads: four cells per lane keep
 // the brick's seven reads of z in 16-byte loads with a quarter of the index work.  FP64 at 128^3: 8.5 us
@@ -1406,9 +1481,11 @@ __global__ __launch_bounds__(BLOCK) void k_jacobi4(LevelDesc L, OpDesc<T> A, con
                                                    const T *__restrict__ rhs, const T *__restrict__ zin,
                                                    T *__restrict__ zout, T omega, Gate Q, int nvirt) {
     if (all_done(Q)) return;
-    const int bpb = blockDim.x / ROW4_THREADS, slot = threadIdx.x / ROW4_THREADS, q = threadIdx.x % ROW4_THREADS;
+    constexpr int BPB = FINEST ? BLOCK / ROW4_THREADS : 1;
+    const int slot = FINEST ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ROW4_THREADS)) : 0;
+    const int q = threadIdx.x % ROW4_THREADS;
     for (int vb = blockIdx.x; vb < nvirt; vb += gridDim.x) {
-        const int br = bpb * xcd_brick(vb, nvirt) + slot;
+        const int br = BPB * xcd_brick(vb, nvirt) + slot;
         if (br >= L.nbricks) continue;
         const BrickMeta m = L.meta[br];
         if (skip_smooth(Q, L, m)) continue;
@@ -1743,13 +1820,15 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_post_local4(LevelDesc L, OpDes
     if (all_done(Q) || skip_smooth(Q, L, m)) return;
     const int q = threadIdx.x;
     const Row4Nbrs N = row4_nbrs(m, br, q);
-    const Row4Vals<float> v = row4_vals(zin, N);
+    const Row4Raw<float> raw = row4_load(zin, N);
+    Row4Vals<float> v;
     float r[4], id[4], e[4], res[4];
     unpack4(ld4(rhs, N.c), r);
     Row4Coef<float> c;
     bool unk[4];
-    if (m.flags & BM_UNIFORM) {
+    if (FINEST && (m.flags & BM_UNIFORM)) {
         const UniT<float> u = uni_load<float>(L, br);
+        v = row4_join(raw, N);
         const float diag = 0.0f + ((u.g + u.g) + (u.g + u.g) + (u.g + u.g));
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1761,10 +1840,12 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_post_local4(LevelDesc L, OpDes
         }
         c = row4_uniform(u.g);
     } else {
-        const Row4Coef<float> g = row4_coef(A, N);
+        const Row4CoefRaw<float> graw = row4_coef_load(A, N);
         float dir[4];
         load4(A.dir, N.c, dir);
-        unpack4(ld4(idiag, N.c), id);
+        load4(idiag, N.c, id);
+        v = row4_join(raw, N);
+        const Row4Coef<float> g = row4_coef_join(graw, N);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const float off = g.gxm[j] * v.xm[j] + g.gxp[j] * v.xp[j] + g.gym[j] * v.ym[j] + g.gyp[j] * v.yp[j] +
@@ -1796,11 +1877,12 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_post_local4(LevelDesc L, OpDes
 }
 
 // (A v) on the lane's four cells, with the unknown mask: apply_row / apply_row_uniform per cell.
-template <class T>
+template <int FINEST, class T>
 __device__ __forceinline__ void apply_row4(const LevelDesc &L, const OpDesc<T> &A, int br, const BrickMeta &m,
-                                           const Row4Nbrs &N, const Row4Vals<T> &v, T av[4], bool unk[4]) {
-    if (m.flags & BM_UNIFORM) {
+                                           const Row4Nbrs &N, const Row4Raw<T> &raw, T av[4], bool unk[4]) {
+    if (FINEST && (m.flags & BM_UNIFORM)) {
         const UniT<T> u = uni_load<T>(L, br);
+        const Row4Vals<T> v = row4_join(raw, N);
         const T diag = T(0) + ((u.g + u.g) + (u.g + u.g) + (u.g + u.g));
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1809,9 +1891,11 @@ __device__ __forceinline__ void apply_row4(const LevelDesc &L, const OpDesc<T> &
             unk[j] = true;
         }
     } else {
-        const Row4Coef<T> g = row4_coef(A, N);
+        const Row4CoefRaw<T> graw = row4_coef_load(A, N);
         T dir[4];
         load4(A.dir, N.c, dir);
+        const Row4Vals<T> v = row4_join(raw, N);
+        const Row4Coef<T> g = row4_coef_join(graw, N);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const T off = g.gxm[j] * v.xm[j] + g.gxp[j] * v.xp[j] + g.gym[j] * v.ym[j] + g.gyp[j] * v.yp[j] +
@@ -1831,7 +1915,9 @@ __device__ __forceinline__ void apply_row4(const LevelDesc &L, const OpDesc<T> &
 template <int FINEST>
 __device__ __forceinline__ void row4_slot(const LevelDesc &L, int &br, int &q, int skip = 0) {
     constexpr int BPB = FINEST ? BLOCK / ROW4_THREADS : 1;
-    br = BPB * xcd_brick(blockIdx.x - skip, gridDim.x - skip) + (int)(threadIdx.x / ROW4_THREADS);
+    br = BPB * xcd_brick(blockIdx.x - skip, gridDim.x - skip);
+    // a wavefront works on one brick (whose record is then a scalar load)
+    if (FINEST) br += __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ROW4_THREADS));
     q = threadIdx.x % ROW4_THREADS;
 }
 
@@ -1873,11 +1959,11 @@ __global__ __launch_bounds__(BLOCK) void k_residual4(LevelDesc L, OpDesc<T> A, c
     const BrickMeta m = L.meta[br];
     if (all_done(Q) || skip_smooth(Q, L, m)) return;
     const Row4Nbrs N = row4_nbrs(m, br, q);
-    const Row4Vals<T> v = row4_vals(z, N);
+    const Row4Raw<T> v = row4_load(z, N);
     T r[4], av[4], out[4];
     bool unk[4];
     load4(rhs, N.c, r);
-    apply_row4(L, A, br, m, N, v, av, unk);
+    apply_row4<FINEST>(L, A, br, m, N, v, av, unk);
 #pragma unroll
     for (int j = 0; j < 4; ++j) out[j] = unk[j] ? r[j] - av[j] : T(0);
     store4(res, N.c, out);
@@ -2163,11 +2249,11 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_defect4(LevelDesc L, OpDesc<do
     if (br < 0) return;
     const BrickMeta m = L.meta[br];
     const Row4Nbrs N = row4_nbrs(m, br, threadIdx.x);
-    const Row4Vals<double> v = row4_vals(x, N);
+    const Row4Raw<double> v = row4_load(x, N);
     double bv[4], av[4], out[4];
     bool unk[4];
     load4(b, N.c, bv);
-    apply_row4(L, A, br, m, N, v, av, unk);
+    apply_row4<1>(L, A, br, m, N, v, av, unk);
     double mx = 0.0, sq = 0.0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
