@@ -886,10 +886,11 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
                     if (f)
                         K.go("post_local_L0", 0, 8 * es, -usave(C, 0, 5 * es), dim3(brick_grid(L.nbricks)),
                              dim3(ROW4_THREADS), k3 ? k_post_local4<0, 3> : k_post_local4<0, 2>, L.desc, A, id, rhs,
-                             (const T *)cur, oth, Q, P.red);
+                             (const T *)cur, oth, Q, P.red, (const T *)nullptr);
                     else
                         K.go("post_local_Lc", l, 8 * es, 0, dim3(brick_grid(L.nbricks)), dim3(ROW4_THREADS),
-                             k_post_local4<0, LOCAL_SGS_SWEEPS_COARSE, 0>, L.desc, A, id, rhs, (const T *)cur, oth, Q, P.red);
+                             k_post_local4<0, LOCAL_SGS_SWEEPS_COARSE, 0>, L.desc, A, id, rhs, (const T *)cur, oth, Q, P.red,
+                             (const T *)nullptr);
                     std::swap(cur, oth);
                 }
             }
@@ -961,7 +962,9 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
             zoth[l] = oth;
             continue;
         }
-        if constexpr (sizeof(T) == 4)
+        if (brick_smoother) {
+            // joins the first post-smoothing application
+        } else if constexpr (sizeof(T) == 4)
             K.go(f ? "prolong_L0" : "prolong_Lc", l, 3 * es, es * (double)Lc.unknowns - usave(C, l, es),
                  row4_launch(L.nbricks, f).grid, row4_launch(L.nbricks, f).block, f ? k_prolong4<1> : k_prolong4<0>,
                  L.desc, A, (const T *)zcur[l + 1], zcur[l], Q);
@@ -973,19 +976,26 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
             if constexpr (sizeof(T) == 4) {
                 if (brick_smoother) {
                     const dim3 gb(brick_grid(L.nbricks));
-                    const bool k3 = P.local_k == 3;
+                    const bool k3 = P.local_k == 3, pro = s == 0;
+                    const T *zc = (const T *)zcur[l + 1];
+                    const double zc_bytes = pro ? es * (double)Lc.unknowns : 0;
                     if (last_dot)
-                        K.go("post_local_dot_L0", 0, 8 * es, -usave(C, 0, 5 * es), gb, dim3(ROW4_THREADS),
-                             k3 ? k_post_local4<1, 3> : k_post_local4<1, 2>, L.desc, A, id, rhs, (const T *)cur, oth, Q,
-                             P.red);
+                        K.go(pro ? "prolong_post_dot_L0" : "post_local_dot_L0", 0, 8 * es, zc_bytes - usave(C, 0, 5 * es),
+                             gb, dim3(ROW4_THREADS),
+                             pro ? (k3 ? k_post_local4<1, 3, 1, 1> : k_post_local4<1, 2, 1, 1>)
+                                 : (k3 ? k_post_local4<1, 3> : k_post_local4<1, 2>),
+                             L.desc, A, id, rhs, (const T *)cur, oth, Q, P.red, zc);
                     else if (f)
-                        K.go("post_local_L0", 0, 8 * es, -usave(C, 0, 5 * es), gb, dim3(ROW4_THREADS),
-                             k3 ? k_post_local4<0, 3> : k_post_local4<0, 2>, L.desc, A, id, rhs, (const T *)cur, oth, Q,
-                             P.red);
+                        K.go(pro ? "prolong_post_L0" : "post_local_L0", 0, 8 * es, zc_bytes - usave(C, 0, 5 * es), gb,
+                             dim3(ROW4_THREADS),
+                             pro ? (k3 ? k_post_local4<0, 3, 1, 1> : k_post_local4<0, 2, 1, 1>)
+                                 : (k3 ? k_post_local4<0, 3> : k_post_local4<0, 2>),
+                             L.desc, A, id, rhs, (const T *)cur, oth, Q, P.red, zc);
                     else
-                        K.go("post_local_Lc", l, 8 * es, 0, gb, dim3(ROW4_THREADS),
-                             k_post_local4<0, LOCAL_SGS_SWEEPS_COARSE, 0>, L.desc, A, id, rhs, (const T *)cur, oth, Q,
-                             P.red);
+                        K.go(pro ? "prolong_post_Lc" : "post_local_Lc", l, 8 * es, zc_bytes, gb, dim3(ROW4_THREADS),
+                             pro ? k_post_local4<0, LOCAL_SGS_SWEEPS_COARSE, 0, 1>
+                                 : k_post_local4<0, LOCAL_SGS_SWEEPS_COARSE, 0>,
+                             L.desc, A, id, rhs, (const T *)cur, oth, Q, P.red, zc);
                     std::swap(cur, oth);
                     continue;
                 }
