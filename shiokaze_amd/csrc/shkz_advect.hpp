@@ -74,20 +74,29 @@ __device__ __forceinline__ void full_face(const VelField &F, const float *const 
             out[ud] = MASKED ? face_val(U[ud], F.act[ud], q) : U[ud][q];
             continue;
         }
+        // the two cells on the sides of the face along dim (clamped into the grid), their two faces along
+        // ud (in range)
+        const unsigned st[3] = {(unsigned)s[1] * (unsigned)s[2], (unsigned)s[2], 1u};
+        const int lo = clamp_i(pc[dim] - 1, s[dim]), hi = clamp_i(pc[dim], s[dim]);
+        const unsigned n0 = (unsigned)flat3(dim == 0 ? lo : i, dim == 1 ? lo : j, dim == 2 ? lo : k, s);
+        const unsigned n1 = n0 + (hi > lo ? st[dim] : 0u);
+        const unsigned n[4] = {n0, n0 + st[ud], n1, n1 + st[ud]};
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = MASKED ? face_val(U[ud], F.act[ud], n[q]) : U[ud][n[q]];
         double u = 0.0;
 #pragma unroll
-        for (int ii = 0; ii < 2; ++ii)
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj) {
-                int q[3];
-#pragma unroll
-                for (int a = 0; a < 3; ++a) q[a] = clamp_i(pc[a] - (a == dim) + ii * (a == dim) + jj * (a == ud), s[a]);
-                const size_t n = flat3(q[0], q[1], q[2], s);
-                u += (double)(MASKED ? face_val(U[ud], F.act[ud], n) : U[ud][n]);
-            }
+        for (int q = 0; q < 4; ++q) u += (double)v[q];
         u /= 4.0;
         out[ud] = (float)u;
     }
+}
+
+__device__ __forceinline__ void cell_decode(const VelField &F, size_t c, int &i, int &j, int &k) {
+    const unsigned t = divide((unsigned)c, F.cell2), ii = divide(t, F.cell1);
+    k = (int)((unsigned)c - t * (unsigned)F.d);
+    j = (int)(t - ii * (unsigned)F.h);
+    i = (int)ii;
 }
 
 // macarray3::convert_to_full at cell (i,j,k): valid when both faces of every axis are active.
@@ -127,11 +136,10 @@ __device__ __forceinline__ void full_cell(const VelField &F, int i, int j, int k
 // bounds computed from them: the value pass and the min/max pass share their stencil unless the
 // two departure points (float and double arithmetic) fall in different cells.
 __device__ __forceinline__ void load8(const float *U, const uint8_t *A, const int s[3], const Corner &c, float v[8]) {
+    unsigned q[8];
+    corner_indices(c, s, q);
 #pragma unroll
-    for (int n = 0; n < 8; ++n) {
-        const size_t q = corner_index(c, n, s);
-        v[n] = A ? face_val(U, A, q) : U[q];
-    }
+    for (int n = 0; n < 8; ++n) v[n] = A ? face_val(U, A, q[n]) : U[q[n]];
 }
 __device__ __forceinline__ float interp8(const Corner &c, const float v[8]) {
 #pragma clang fp contract(off)
@@ -163,32 +171,20 @@ __device__ __forceinline__ bool same_cell(const Corner &a, const Corner &b) {
     return a.i == b.i && a.j == b.j && a.k == b.k;
 }
 
-// min and max of the 8 corner values at p (interpolate_coef's stencil), from the given initial
-// bounds (the reference's numeric_limits initialisers)
-__device__ __forceinline__ void corner_bounds(const float *U, const uint8_t *A, const int s[3], const double p[3],
-                                              double &lo, double &hi) {
-    const Corner c = corner_of(s, p);
-#pragma unroll
-    for (int n = 0; n < 8; ++n) {
-        const size_t q = corner_index(c, n, s);
-        const double v = A ? (double)face_val(U, A, q) : (double)U[q];
-        lo = v < lo ? v : lo;  // std::min
-        hi = hi < v ? v : hi;  // std::max
-    }
-}
-
 // the liquid level set at p (cell index space): float accumulation for a float level set
 __device__ __forceinline__ double interp_level(const void *phi, int f64, const int s[3], const double p[3]) {
 #pragma clang fp contract(off)
     const Corner c = corner_of(s, p);
     double w[8];
     interp_weights(c, w);
+    unsigned q[8];
+    corner_indices(c, s, q);
     // all eight corners are loaded at once (advection asks for at least 2 cells per axis, so they
     // lie in the array); zero weights still skip the accumulation
     if (f64) {
         double v[8];
 #pragma unroll
-        for (int n = 0; n < 8; ++n) v[n] = ((const double *)phi)[corner_index(c, n, s)];
+        for (int n = 0; n < 8; ++n) v[n] = ((const double *)phi)[q[n]];
         double val = 0.0;
 #pragma unroll
         for (int n = 0; n < 8; ++n)
@@ -197,7 +193,7 @@ __device__ __forceinline__ double interp_level(const void *phi, int f64, const i
     }
     float v[8];
 #pragma unroll
-    for (int n = 0; n < 8; ++n) v[n] = ((const float *)phi)[corner_index(c, n, s)];
+    for (int n = 0; n < 8; ++n) v[n] = ((const float *)phi)[q[n]];
     float val = 0.0f;
 #pragma unroll
     for (int n = 0; n < 8; ++n)
@@ -317,16 +313,12 @@ __device__ __forceinline__ float sample_arr(const float *U, const uint8_t *A, co
 // MacCormack bounds and the narrow-band flag.  `in` is the field being advected (its own full
 // velocity moves it, :72-73).
 template <int WENO>
-__global__ void k_adv_face_fwd(VelField F, const float *in0, const float *in1, const float *in2, AdvScratch S,
-                               const void *fluid, int fluid64, double dt, int trim, int minmax) {
+__device__ __forceinline__ void adv_face_fwd(const VelField &F, int a, size_t f, const float *in0, const float *in1,
+                                             const float *in2, const AdvScratch &S, const void *fluid, int fluid64,
+                                             double dt, int trim, int minmax) {
 #pragma clang fp contract(off)
-    int a, i, j, k;
-    size_t f;
-    if (!vf_decode(F, a, f, i, j, k)) return;
-    if (!F.act[a][f]) {
-        S.v0[a][f] = 0.0f;  // what the activity mask reads there
-        return;
-    }
+    int i, j, k;
+    vf_decode(F, a, f, i, j, k);
     const float *const in[3] = {in0, in1, in2};
     float u[3];
     full_face<true>(F, in, a, i, j, k, u);
@@ -384,21 +376,28 @@ __global__ void k_adv_face_fwd(VelField F, const float *in0, const float *in1, c
     S.hi[a][f] = hi;
     S.nb[a][f] = interp_level(fluid, fluid64, sc, q) > -F.dx * (double)trim ? 1 : 0;
 }
+// (One group per wavefront whatever the size: bound by its arithmetic, and the registers of the loop over
+// groups would cost wavefronts: 473 us against 439 at 256^3.)
+template <int WENO>
+__global__ void k_adv_face_fwd(VelField F, const float *in0, const float *in1, const float *in2, AdvScratch S,
+                               const void *fluid, int fluid64, double dt, int trim, int minmax) {
+    const VfFaces<1> V = vf_faces<1>(F);
+    if (V.code(0)) adv_face_fwd<WENO>(F, V.a, V.f0, in0, in1, in2, S, fluid, fluid64, dt, trim, minmax);
+    else if (V.f0 < F.n[V.a]) S.v0[V.a][V.f0] = 0.0f;  // what the activity mask reads there
+}
 
 // Backward pass from S.v0 (-dt) fused with MacCormack's final step, written over F.vel (the
 // input field, read only at the thread's own face).
 template <int WENO>
-__global__ void k_adv_face_bwd(VelField F, AdvScratch S, double dt_back) {
+__device__ __forceinline__ void adv_face_bwd(const VelField &F, int a, size_t f, const AdvScratch &S, double dt_back) {
 #pragma clang fp contract(off)
-    int a, i, j, k;
-    size_t f;
-    if (!vf_decode(F, a, f, i, j, k)) return;
-    if (!F.act[a][f]) return;
     const float v0 = S.v0[a][f];
     if (S.nb[a][f]) {
         F.vel[a][f] = v0;
         return;
     }
+    int i, j, k;
+    vf_decode(F, a, f, i, j, k);
     const float *const in[3] = {S.v0[0], S.v0[1], S.v0[2]};
     float u[3];
     full_face<false>(F, in, a, i, j, k, u);
@@ -423,13 +422,22 @@ __global__ void k_adv_face_bwd(VelField F, AdvScratch S, double dt_back) {
     const double r = (double)v0 + 0.5 * (double)diff;
     F.vel[a][f] = r < lo ? (float)lo : (r > hi ? (float)hi : (float)r);
 }
+template <int WENO, int G>
+__global__ void k_adv_face_bwd(VelField F, AdvScratch S, double dt_back) {
+    const VfFaces<G> V = vf_faces<G>(F);
+    if (!V.codes) return;
+#pragma unroll 1
+    for (int g = 0; g < G; ++g)
+        if (V.code(g)) adv_face_bwd<WENO>(F, V.a, V.face(g), S, dt_back);
+}
 
 // semi-Lagrangian only: the forward result over the active faces
+template <int G>
 __global__ void k_adv_face_copy(VelField F, AdvScratch S) {
-    int a, i, j, k;
-    size_t f;
-    if (!vf_decode(F, a, f, i, j, k)) return;
-    if (F.act[a][f]) F.vel[a][f] = S.v0[a][f];
+    const VfFaces<G> V = vf_faces<G>(F);
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+        if (V.code(g)) F.vel[V.a][V.face(g)] = S.v0[V.a][V.face(g)];
 }
 
 // Forward pass over the cells of q (advected by F): S.v0[0] = the semi-Lagrangian value, or
@@ -447,7 +455,7 @@ __global__ void k_adv_cell_fwd(VelField F, const float *q, const uint8_t *aq, Ad
         return;
     }
     int i, j, k;
-    unflatten((unsigned)c, (unsigned)F.h, (unsigned)F.d, i, j, k);
+    cell_decode(F, c, i, j, k);
     double u[3];
     full_cell(F, i, j, k, u);
     const bool empty = u[0] == 0.0 && u[1] == 0.0 && u[2] == 0.0;
@@ -497,7 +505,7 @@ __global__ void k_adv_cell_bwd(VelField F, float *q, const uint8_t *aq, AdvScrat
         return;
     }
     int i, j, k;
-    unflatten((unsigned)c, (unsigned)F.h, (unsigned)F.d, i, j, k);
+    cell_decode(F, c, i, j, k);
     double u[3];
     full_cell(F, i, j, k, u);
     const int s[3] = {F.w, F.h, F.d};

@@ -92,6 +92,22 @@ __device__ __forceinline__ void unflatten(unsigned e, unsigned nj, unsigned nk, 
     j = (int)(t - a * nj);
 }
 
+// Division of any 32-bit n by an invariant d >= 1: a high multiply, an add and two shifts (Granlund and
+// Montgomery, "Division by invariant integers using multiplication", PLDI 1994, figure 4.1), where the
+// hardware, without an integer divide, takes about twenty instructions.
+struct FastDiv {
+    unsigned mul, sh1, sh2;
+};
+static inline FastDiv fast_div(unsigned d) {
+    unsigned l = 0;
+    while (l < 32 && ((uint64_t)1 << l) < d) ++l;
+    return FastDiv{(unsigned)((((uint64_t)1 << 32) * (((uint64_t)1 << l) - d)) / d + 1), l < 1 ? l : 1, l < 1 ? 0 : l - 1};
+}
+__host__ __device__ __forceinline__ unsigned divide(unsigned n, const FastDiv &D) {
+    const unsigned t = (unsigned)(((uint64_t)D.mul * n) >> 32);
+    return (t + ((n - t) >> D.sh1)) >> D.sh2;
+}
+
 // Liquid fraction between two level-set samples (utility.h:162-170).
 __device__ __forceinline__ double liquid_fraction(double phi0, double phi1) {
 #pragma clang fp contract(off)

@@ -134,41 +134,49 @@ __global__ void k_reset_ints(int *a, int n) {
 
 // flag |= 1 when any of the n values is negative.  A 16-byte aligned array is read 16 bytes per
 // load, four loads in flight per thread.
-__global__ void k_any_negative(const void *a, int is64, size_t n, int *flag) {
-    int found = 0;
-    const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x, nt = (size_t)gridDim.x * blockDim.x;
+constexpr int NEGATIVE_THREADS = 256;
+template <class T>
+__device__ __forceinline__ bool any_negative(const T *a, size_t n, size_t tid, size_t nt) {
+    constexpr int PER = 16 / sizeof(T);  // values per 16 bytes
+    typedef T Vec __attribute__((ext_vector_type(PER)));
+    bool found = false;
+    size_t done = 0;
     if (((uintptr_t)a & 15) == 0) {
-        const size_t per = is64 ? 2 : 4;  // values per 16 bytes
-        const size_t nv = n / per;
-        const float4 *v4 = (const float4 *)a;
-        auto neg = [&](const float4 x) -> int {
-            if (is64) {
-                const double2 d = *reinterpret_cast<const double2 *>(&x);
-                return (d.x < 0.0) | (d.y < 0.0);
-            }
-            return (x.x < 0.0f) | (x.y < 0.0f) | (x.z < 0.0f) | (x.w < 0.0f);
+        const Vec *v = (const Vec *)a;
+        const size_t nv = n / PER;
+        auto negative = [](const Vec x) {
+            bool neg = false;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) neg |= x[j] < T(0);
+            return neg;
         };
         size_t i = tid;
         for (; i + 3 * nt < nv; i += 4 * nt) {
-            float4 x[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) x[u] = v4[i + u * nt];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) found |= neg(x[u]);
+            const Vec x0 = v[i], x1 = v[i + nt], x2 = v[i + 2 * nt], x3 = v[i + 3 * nt];
+            found |= negative(x0) | negative(x1) | negative(x2) | negative(x3);  // (no short cut: the loads go out together)
         }
-        for (; i < nv; i += nt) found |= neg(v4[i]);
-        for (size_t j = nv * per + tid; j < n; j += nt)
-            found |= is64 ? (((const double *)a)[j] < 0.0) : (((const float *)a)[j] < 0.0f);
-    } else {
-        for (size_t i = tid; i < n; i += nt) {
-            const double v = is64 ? ((const double *)a)[i] : (double)((const float *)a)[i];
-            found |= (v < 0.0);
-        }
+        for (; i < nv; i += nt) found |= negative(v[i]);
+        done = nv * PER;
     }
-    found = __syncthreads_or(found);
-    // the flag only ever goes from 0 to 1: a plain store, skipped once it is seen set (thousands of
-    // blocks finding a negative value would otherwise queue read-modify-writes on one address)
-    if (threadIdx.x == 0 && found && __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+    for (size_t i = done + tid; i < n; i += nt) found |= a[i] < T(0);
+    return found;
+}
+__global__ __launch_bounds__(NEGATIVE_THREADS) void k_any_negative(const void *a, int is64, size_t n, int *flag) {
+    const size_t tid = (size_t)blockIdx.x * NEGATIVE_THREADS + threadIdx.x, nt = (size_t)gridDim.x * NEGATIVE_THREADS;
+    const bool found = is64 ? any_negative((const double *)a, n, tid, nt) : any_negative((const float *)a, n, tid, nt);
+    // (a vote through LDS: __syncthreads_or, like an array that the compiler moves to LDS, reads the dispatch
+    // packet, from host memory, 3 us of a short launch)
+    __shared__ int votes[NEGATIVE_THREADS / 64];
+    const bool wave = __ballot(found) != 0;
+    if ((threadIdx.x & 63) == 0) votes[threadIdx.x >> 6] = wave;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < NEGATIVE_THREADS / 64; ++w) any |= votes[w];
+    // the flag only ever goes from 0 to 1: a plain store, skipped once it is seen set; even the look at it costs 6 ns
+    // per workgroup, one after another, so that a launch has few of them (any_negative_blocks)
+    if (any && __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
         __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

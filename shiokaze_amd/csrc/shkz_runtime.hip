@@ -614,6 +614,11 @@ static void launch_grids(Launcher &K, const char *name, int ngrids, int threads,
     }
 }
 
+// Four 16-byte loads of floats per thread, and no more than 1024 workgroups: all that find a negative value look at
+// the one flag, one after another (256^3 nodes: 30 us with 4096, 22 us with 1024; 61x90x77: 16.7 us with
+// a value per thread, 3.3 us here).
+static inline unsigned any_negative_blocks(size_t n) { return (unsigned)std::min<size_t>((n + 4095) / 4096, 1024); }
+
 // Resolves pending timing events into totals (after a stream synchronisation).
 static void resolve_timing(shkz_ctx *C) {
     for (const TimedLaunch &t : C->pending) {
@@ -1845,7 +1850,7 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
         J.exist = exist_all + 4 * g;
         G.exist = J.exist;
         if (scan_liquid) {
-            const unsigned nbk = (unsigned)std::min<size_t>((J.M + 255) / 256, 4096);
+            const unsigned nbk = any_negative_blocks(J.M);
             K.go("any_negative", -1, 0, (double)J.M * (G.phi64 ? 8 : 4), dim3(nbk), dim3(256), k_any_negative,
                  grid->fluid, (int)G.phi64, J.M, J.exist + 0);
         }
@@ -2634,6 +2639,7 @@ static void vf_set_dx(VelField &F, const shkz_velocity_field *f) {
     const double mant = std::frexp(F.dx, &ex);
     F.dx_pow2 = (mant == 0.5 && ex > -400 && ex < 400) ? 1 : 0;
     F.inv_dx = 1.0 / F.dx;
+    vf_set_divisors(F);
 }
 
 // macutility3::extrapolate_and_constrain_velocity (macutility3.cpp:89-93) on the work stream:
@@ -2657,13 +2663,14 @@ static int extrapolate_stages(shkz_ctx *C, const shkz_velocity_field *f, int wid
     }
     const size_t total = F.n[0] + F.n[1] + F.n[2];
     const size_t nodes = (size_t)(f->w + 1) * (f->h + 1) * (f->d + 1);
-    const dim3 grid = vf_grid(F.n), block(VF_BLOCK);
+    const bool many = vf_many(F.n);
+    const dim3 grid = vf_grid(F.n, many ? VF_GROUPS : 1), block(VF_BLOCK);
     int *exist = nullptr;
     SHKZ_TRY(arena_get(AR, "vx_exist", 1, &exist));
     K.go("reset", -1, 0, 4.0, dim3(1), dim3(256), k_reset_ints, exist, 1);
     const bool with_solid = constrain && solid;
     if (with_solid) {
-        const unsigned nbs = (unsigned)std::min<size_t>((nodes + 255) / 256, 4096);
+        const unsigned nbs = any_negative_blocks(nodes);
         K.go("any_negative", -1, 0, (double)nodes * (F.solid64 ? 8 : 4), dim3(nbs), dim3(256), k_any_negative, solid,
              (int)F.solid64, nodes, exist);
     }
@@ -2687,13 +2694,13 @@ static int extrapolate_stages(shkz_ctx *C, const shkz_velocity_field *f, int wid
             for (int a = 0; a < 3; ++a) {
                 B[c].bits[a] = bits + off;
                 B[c].W[a] = W[a];
+                B[c].by[a] = fast_div((unsigned)W[a]);
                 off += (size_t)(f->w + (a == 0)) * (f->h + (a == 1)) * W[a];
             }
-        const dim3 gpack((unsigned)((wmax * 32 + 256 * PACK_GROUPS - 1) / (256 * PACK_GROUPS)), 3),
-            gword((unsigned)((wmax + 255) / 256), 3);
+        const dim3 gword((unsigned)((wmax + VF_BLOCK - 1) / VF_BLOCK), 3);
         // byte models: the pack reads the activity bytes and writes the bits; a pass reads and
         // writes the bits (the values of the faces it activates are few)
-        K.go("extrap_pack", -1, 0, (double)total + 4.0 * words, gpack, block, k_pack_activity, F, B[0]);
+        K.go("extrap_pack", -1, 0, (double)total + 4.0 * words, gword, block, k_pack_activity, F, B[0]);
         for (int p = 1; p <= width; ++p)
             K.go("extrap_pass", -1, 0, 8.0 * words, gword, block, k_extrap_pass, F, B[p == 1 ? 0 : 1 + (p & 1)],
                  B[1 + ((p + 1) & 1)]);
@@ -2706,9 +2713,10 @@ static int extrapolate_stages(shkz_ctx *C, const shkz_velocity_field *f, int wid
     }
     // the side buffers are written and read only at constrained faces
     K.go("constrain", -1, 0, with_solid ? (double)total + (double)nodes * (F.solid64 ? 8 : 4) : (double)total, grid,
-         block, k_constrain, F, xs[0], xs[1], xs[2], (const int *)exist, with_solid ? 1 : 0);
+         block, many ? k_constrain<VF_GROUPS> : k_constrain<1>, F, xs[0], xs[1], xs[2], (const int *)exist, with_solid ? 1 : 0);
     if (with_solid)
-        K.go("constrain_apply", -1, 0, (double)total, grid, block, k_constrain_apply, F, (const float *)xs[0],
+        K.go("constrain_apply", -1, 0, (double)total, grid, block,
+             many ? k_constrain_apply<VF_GROUPS> : k_constrain_apply<1>, F, (const float *)xs[0],
              (const float *)xs[1], (const float *)xs[2], (const int *)exist, 1);
     SHKZ_HIP(hipGetLastError());
     return SHKZ_OK;
@@ -2790,7 +2798,8 @@ static int advect_velocity_stages(shkz_ctx *C, const shkz_velocity_field *f, con
     Launcher K{C, s};
     VelField F = vel_field_of(f, vel, act);
     const size_t total = F.n[0] + F.n[1] + F.n[2];
-    const dim3 grid = vf_grid(F.n), block(VF_BLOCK);
+    const bool many = vf_many(F.n);
+    const dim3 grid = vf_grid(F.n), grid_many = vf_grid(F.n, VF_GROUPS), block(VF_BLOCK);
     AdvScratch S;
     const char *nv[3] = {"adv_v0", "adv_v1", "adv_v2"}, *nl[3] = {"adv_lo0", "adv_lo1", "adv_lo2"},
                *nh[3] = {"adv_hi0", "adv_hi1", "adv_hi2"}, *nn[3] = {"adv_nb0", "adv_nb1", "adv_nb2"};
@@ -2817,11 +2826,15 @@ static int advect_velocity_stages(shkz_ctx *C, const shkz_velocity_field *f, con
              (const float *)vel[0], (const float *)vel[1], (const float *)vel[2], S, fluid, f64, p->dt,
              (int)p->trim_narrowband, mc ? 1 : 0);
     if (mc && p->weno)
-        K.go("adv_face_bwd_weno", -1, 0, (double)total * 22, grid, block, k_adv_face_bwd<1>, F, S, -p->dt);
+        K.go("adv_face_bwd_weno", -1, 0, (double)total * 22, grid, block, k_adv_face_bwd<1, 1>, F, S, -p->dt);
+    else if (mc && many)
+        K.go("adv_face_bwd", -1, 0, (double)total * 22, grid_many, block, k_adv_face_bwd<0, VF_GROUPS>, F, S, -p->dt);
     else if (mc)
-        K.go("adv_face_bwd", -1, 0, (double)total * 22, grid, block, k_adv_face_bwd<0>, F, S, -p->dt);
+        K.go("adv_face_bwd", -1, 0, (double)total * 22, grid, block, k_adv_face_bwd<0, 1>, F, S, -p->dt);
+    else if (many)
+        K.go("adv_face_copy", -1, 0, (double)total * 9, grid_many, block, k_adv_face_copy<VF_GROUPS>, F, S);
     else
-        K.go("adv_face_copy", -1, 0, (double)total * 9, grid, block, k_adv_face_copy, F, S);
+        K.go("adv_face_copy", -1, 0, (double)total * 9, grid, block, k_adv_face_copy<1>, F, S);
     SHKZ_HIP(hipGetLastError());
     return SHKZ_OK;
 }
