@@ -796,10 +796,13 @@ __global__ __launch_bounds__(BLOCK) void k_apply_dot(LevelDesc L, OpDesc<T> A, c
 
 // x += alpha p, r -= alpha q with ||r||_inf and r.r partials (FIN_UPDATE runs the convergence
 // test of pcg_solver.h:278-285).
-template <class T>
+// ZFIRST (preconditioned): also the V-cycle's first sweep from zero, z = omega * idiag * r (k_smooth_first's, which
+// read r again in a launch of its own: 7.1 + 4.7 us at 128^3 in FP64, 8.6 here).
+template <class T, int ZFIRST>
 __global__ __launch_bounds__(BLOCK) void k_cg_update(LevelDesc L, T *__restrict__ x, T *__restrict__ r,
                                                      const T *__restrict__ p, const T *__restrict__ q,
-                                                     const SolveScalars *S, const BatchCtl *ctl, RedBuf R) {
+                                                     const SolveScalars *S, const BatchCtl *ctl, RedBuf R,
+                                                     const T *__restrict__ idiag, T *__restrict__ z, T omega) {
     __shared__ double lds[32];
     const int br = brick_or_idle(L);
     if (br < 0) return;
@@ -808,12 +811,20 @@ __global__ __launch_bounds__(BLOCK) void k_cg_update(LevelDesc L, T *__restrict_
     // only on an iteration past convergence); in a batch, bricks of finished grids load nothing.
     if (L.ngrids > 1 && (ctl->all_done || S[grid_of(L, br)].done)) return;
     const T xv = x[c], pv = p[c], r0 = r[c], qv = q[c];
+    T id = T(0);
+    bool first = false;
+    if (ZFIRST) {
+        const BrickMeta m = L.meta[br];
+        first = !(m.flags & BM_COARSEST);  // (a grid's last level is its coarse solve's)
+        id = (m.flags & BM_UNIFORM) ? uni_load<T>(L, br).id : idiag[c];
+    }
     const SolveScalars &Sg = S[grid_of(L, br)];
     if (ctl->all_done || Sg.done) return;
     const T alpha = (T)Sg.alpha;
     x[c] = xv + alpha * pv;
     const T rv = r0 - alpha * qv;
     r[c] = rv;
+    if (ZFIRST && first) z[c] = omega * id * rv;
     double mx = fabs((double)rv), sq = (double)rv * (double)rv;
     block_reduce2<true>(mx, sq, lds);
     store_partials(R, br, mx, sq);

@@ -1192,6 +1192,8 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
                  q, (const SolveScalars *)S, (const BatchCtl *)ctl, pq);
         if (!fold) finalize(K, P, L0.desc, S, ctl, FIN_PQ);
     }
+    // FP64: the residual update performs the V-cycle's first sweep as well
+    const bool zfirst = sizeof(T) == 8 && precond && P.nlev > 1;
     auto iteration = [&]() {
         if (fused) {
             half(p, p2, 0);
@@ -1210,11 +1212,12 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
                  (const T *)q, S, ctl, P.red, (const T *)nullptr, (T *)nullptr, (T)0, op_of<float>(L0),
                  (const double *)nullptr, 0);
         else
-            K.go("cg_update", 0, 6 * es, 0, g, b, k_cg_update<T>, L0.desc, x, r, (const T *)p, (const T *)q,
-                 (const SolveScalars *)S, (const BatchCtl *)ctl, P.red);
+            K.go(zfirst ? "cg_update_z" : "cg_update", 0, (zfirst ? 8 : 6) * es, zfirst ? -usave(C, 0, es) : 0, g, b,
+                 zfirst ? k_cg_update<T, 1> : k_cg_update<T, 0>, L0.desc, x, r, (const T *)p, (const T *)q,
+                 (const SolveScalars *)S, (const BatchCtl *)ctl, P.red, (const T *)L0.idiag, z, (T)P.omega);
         finalize(K, P, L0.desc, S, ctl, precond ? FIN_UPDATE : FIN_UPDATE_CG);
         if (precond) {
-            const T *zz = vcycle<T>(C, K, P, r, z, tmp, Q, fused_dot);
+            const T *zz = vcycle<T>(C, K, P, r, z, tmp, Q, fused_dot, zfirst);
             if (!fused_dot)
                 K.go("dot_rz", 0, 2 * es, 0, g, b, k_dot_rz<T>, L0.desc, (const T *)r, zz, (const SolveScalars *)S,
                      (const BatchCtl *)ctl, P.red);
