@@ -11,7 +11,7 @@
 //                      Krylov solve (stands in for PCGSolver::solve, pcg_solver.h:246-295)
 //   k_output           m_pressure (:245-248) and velocity update (:252-268)
 //
-// Build and output kernels work on one grid's dense arrays.  Solver kernels work on a batch: the
+// Build and output kernels work on dense arrays, up to twelve grids in a launch.  Solver kernels work on a batch: the
 // stored bricks of every grid of the batch, concatenated, one 512-thread block per brick (thread =
 // cell) with an XCD-aware block-to-brick remap.  Stencil neighbours in the same brick are read at
 // +-1/8/64, the others through the brick's neighbour table.  Reductions are per grid and
