@@ -271,14 +271,15 @@ __device__ __forceinline__ int table_grid(const GridTable<D> &T, int &local) {
 // of 8 cells along x, a workgroup the columns of FLAGS_SPAN bricks along z (FLAGS_SPAN_FLAT along y in a 2D
 // grid), so that a sample is read 1.25 times instead of up to 7: the signs of a column are the bits of one
 // byte, which neighbours take from LDS.  256^3 of FP64 samples: 116 us with one cell per thread and a
-// chain of neighbour tests, 102 us with columns that load their neighbours, 67 to 93 us here; 120x168x89
-// within a solid's reach 40 to 16 us.
+// chain of neighbour tests, 102 us with columns that load their neighbours, 67 us
+// with 32 columns a workgroup along z, 60 with the 64 here (a border cell costs its whole cache line); 120x168x89
+// within a solid's reach 40 to 17 us.
 struct FlagsGrid {
     GridDesc G;
     int nbx, nby, nbz;
     uint8_t *cflag, *bflag;
 };
-constexpr int FLAGS_THREADS = 256;
+constexpr int FLAGS_THREADS = 512;
 constexpr int FLAGS_SPAN = FLAGS_THREADS / BRICK / BRICK, FLAGS_SPAN_FLAT = FLAGS_THREADS / BRICK;  // bricks
 // Signs of `ni` cells at stride HD from c0 on: bit p = cell p is liquid.
 template <class Tp>

@@ -1,6 +1,6 @@
 """The per-grid kernels (labelling, assembly, output) at the edges of their tiles: unknown set, right-hand
 side, activity and velocity update equal to the oracle's, bit for bit, on rough level sets (every combination
-of signs around a face, zeros included) at sizes around a brick, a row of 32 cells, a column of 4
+of signs around a face, zeros included) at sizes around a brick, rows of 32 and 64 cells, a column of 4
 planes and 256 cells of a plane; and more grids than one launch takes, each as when projected alone.
 """
 import numpy as np
@@ -12,7 +12,7 @@ from oracle import oracle as O
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 1, 1), (2, 9, 3), (4, 7, 31), (5, 8, 32), (8, 17, 33), (9, 16, 16), (13, 3, 65), (17, 33, 8), (3, 2, 130)]
-SHAPES_2D = [(1, 1), (7, 255), (9, 256), (16, 257), (33, 8), (5, 300)]
+SHAPES_2D = [(1, 1), (7, 255), (9, 256), (16, 257), (33, 8), (5, 300), (4, 512), (9, 513)]
 
 
 @pytest.fixture(scope="module")
