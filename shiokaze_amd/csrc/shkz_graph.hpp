@@ -1,7 +1,8 @@
-// shkz_graph.hpp -- kernel nodes of an explicitly built hipGraph.
+// shkz_graph.hpp -- kernel nodes of an explicitly built hipGraph, and the key under which one is kept.
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <string>
 #include <tuple>
 #include <type_traits>
 #include <utility>
@@ -30,5 +31,17 @@ inline hipError_t add_kernel_node(hipGraph_t graph, hipGraphNode_t *last, dim3 g
         },
         values);
 }
+
+// The key of a kept graph: the bytes of every value that its kernels' arguments depend on, each whole and
+// in a fixed order.  (Formatted text in a buffer of a fixed size would lose its end when the pointers of a
+// level grow long: two graphs of different arrays under one key.)
+struct GraphKey {
+    std::string bytes;
+    template <class... V>
+    void add(const V &...v) {
+        static_assert(((std::is_arithmetic_v<V> || std::is_pointer_v<V>) && ...), "values without padding");
+        (bytes.append(reinterpret_cast<const char *>(&v), sizeof(V)), ...);
+    }
+};
 
 }  // namespace shkz

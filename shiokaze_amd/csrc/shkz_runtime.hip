@@ -1069,31 +1069,19 @@ static void finalize(Launcher &K, const Problem &P, const LevelDesc &L0, SolveSc
 
 template <class T>
 static std::string graph_key(shkz_ctx *C, const Problem &P, const void *const *vecs, int nvec, bool precond) {
-    std::string k;
-    char buf[256];
-    std::snprintf(buf, sizeof(buf), "T%zu pc%d g%d nl%d pre%d post%d prc%d poc%d cs%d mm%d sm%d lk%d om%.17g red%p|",
-                  sizeof(T), precond ? 1 : 0, P.ngrids, P.nlev, P.pre, P.post, P.pre_c, P.post_c, P.coarse_sweeps,
-                  P.multi_max_bricks, P.smoother, P.local_k, P.omega, (void *)P.red.partials);
-    k += buf;
-    std::snprintf(buf, sizeof(buf), "bt%p %d|", (const void *)P.bottom, P.bottom_level);
-    k += buf;
-    for (int i = 0; i < nvec; ++i) {
-        std::snprintf(buf, sizeof(buf), "%p,", vecs[i]);
-        k += buf;
-    }
+    GraphKey k;
+    k.add(sizeof(T), precond, P.ngrids, P.nlev, P.pre, P.post, P.pre_c, P.post_c, P.coarse_sweeps, P.multi_max_bricks,
+          P.smoother, P.local_k, P.omega, P.red.partials, P.red2.partials, P.bottom, P.bottom_level);
+    for (int i = 0; i < nvec; ++i) k.add(vecs[i]);
     const int nl = precond ? P.nlev : 1;
     for (int l = 0; l < nl; ++l) {
         const LevelHost &L = C->levels[l];
-        // the transfer kernels branch on flat (bilinear in 2D) and the reductions on ngrids
-        std::snprintf(buf, sizeof(buf), "|%d %d f%d g%d %p %p %p %p %p %p %p %p %p %p %p %p %p %p %p %p %p %p",
-                      L.nbricks, L.any_coarsest ? 1 : 0, L.desc.flat, L.desc.ngrids, (const void *)L.desc.bmap, L.dir,
-                      L.gx, L.gy, L.gz, L.idiag, L.rhs, L.z,
-                      L.tmp, L.res, (const void *)L.desc.bxyz, (const void *)L.desc.meta, (const void *)L.desc.gl,
-                      (const void *)L.desc.child64, (const void *)L.desc.parent8, (const void *)L.desc.uni,
-                      (const void *)L.desc.nb27, (const void *)L.ccode);
-        k += buf;
+        // (the transfer kernels branch on flat, bilinear in 2D, and the reductions on ngrids)
+        k.add(L.nbricks, L.any_coarsest, L.desc.flat, L.desc.ngrids, L.desc.bmap, L.dir, L.gx, L.gy, L.gz, L.idiag, L.rhs,
+              L.z, L.tmp, L.res, L.desc.bxyz, L.desc.meta, L.desc.gl, L.desc.child64, L.desc.parent8, L.desc.uni,
+              L.desc.nb27, L.ccode);
     }
-    return k;
+    return k.bytes;
 }
 
 // Krylov loop on level 0 for every grid of the batch: T = element type; precond = V-cycle or

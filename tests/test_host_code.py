@@ -1,0 +1,20 @@
+"""CPU checks of host code inside the HIP sources: a check program includes the source, is compiled for the host alone
+(no device code, no GPU involved) and reports OK."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def build_and_run(tmp_path, name):
+    exe = tmp_path / name
+    subprocess.check_call(["hipcc", "--offload-host-only", "-x", "hip", "-std=c++17", "-Wno-unused-result",
+                           os.path.join(ROOT, "tests", name + ".cpp"), "-o", str(exe),
+                           "-Wl,--unresolved-symbols=ignore-all", "-lpthread"])
+    p = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0 and "OK" in p.stdout, p.stdout + p.stderr
+    return p.stdout
+
+
+def test_graph_key_tells_every_argument_apart(tmp_path):
+    build_and_run(tmp_path, "graph_key_check")
