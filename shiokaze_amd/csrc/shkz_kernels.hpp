@@ -1011,29 +1011,37 @@ __device__ __forceinline__ void finalize_update(const FinUpdate &F, const LevelD
 // The first partials of the n <= FOLD_BRICKS bricks of a single grid, summed by every 128-thread
 // workgroup of the kernel that uses the sum, so that no finalize launch (3 to 4 us, most of it its
 // boundary and one trip to memory) stands between the producer and it.  load() issues the loads,
-// sum() adds; all threads call both.  lds: 16 doubles.  The limit keeps what all workgroups read
+// sum() adds; all threads call both.  The limit keeps what all workgroups read
 // together (8 n^2 bytes) well under the time of a launch: 8 MB from the L2s at 1024.
+//
+// A breakdown that such a kernel finds is recorded in the flags that it tests on entry, by the workgroup of
+// brick 0 while others still enter.  So the two wavefronts of a workgroup don't go by flags of their own: sum()
+// hands all of them the reading of the first thread (stop), behind its barrier, and a workgroup that
+// reads the flags too early forms the same sum and leaves on it.
 constexpr int FOLD_BRICKS = 1024;
 struct FoldPartials {
-    double v[FOLD_BRICKS / ROW4_GROUP];
+    static constexpr int ROUNDS = FOLD_BRICKS / ROW4_GROUP, LDS = 2 * ROUNDS + 1;  // (in doubles)
+    double v[ROUNDS];
     int n;
     __device__ __forceinline__ void load(const double *__restrict__ partials, int nb) {
         n = nb;
 #pragma unroll
-        for (int k = 0; k < FOLD_BRICKS / ROW4_GROUP; ++k) {
+        for (int k = 0; k < ROUNDS; ++k) {
             const int i = k * ROW4_GROUP + (int)threadIdx.x;
             v[k] = i < nb ? partials[2 * i] : 0.0;
         }
     }
-    __device__ __forceinline__ double sum(double *lds) const {
+    __device__ __forceinline__ double sum(double *lds, bool &stop) const {
         const int w = threadIdx.x >> 6;
+        if (threadIdx.x == 0) lds[2 * ROUNDS] = stop ? 1.0 : 0.0;
 #pragma unroll
-        for (int k = 0; k < FOLD_BRICKS / ROW4_GROUP; ++k) {
+        for (int k = 0; k < ROUNDS; ++k) {
             if (k * ROW4_GROUP >= n) break;
             const double s = wave_sum(v[k]);
             if ((threadIdx.x & 63) == 0) lds[2 * k + w] = s;
         }
         __syncthreads();
+        stop = lds[2 * ROUNDS] != 0.0;
         double total = 0.0;
         const int waves = 2 * ((n + ROW4_GROUP - 1) / ROW4_GROUP);
         for (int i = 0; i < waves; ++i) total += lds[i];
@@ -2227,7 +2235,7 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_apply_dot4p(LevelDesc L, OpDes
                                                               float *__restrict__ pnew, float *__restrict__ qv,
                                                               SolveScalars *S, BatchCtl *ctl, RedBuf R,
                                                               const double *__restrict__ rz, int slot) {
-    __shared__ double lds[FOLD ? 16 : 4];
+    __shared__ double lds[FOLD ? FoldPartials::LDS : 4];
     const int br = brick_or_idle(L);
     if (br < 0) return;
     const BrickMeta m = L.meta[br];
@@ -2238,10 +2246,12 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_apply_dot4p(LevelDesc L, OpDes
     if (FOLD) P.load(rz, L.nbricks);
     const Row4Vals<float> zv = row4_vals(z, N);
     const Row4Vals<float> po = row4_vals(pold, N);
-    if (ctl->all_done) return;
+    bool stop = ctl->all_done != 0;
+    if (!FOLD && stop) return;
     float beta;
     if (FOLD) {
-        const double now = P.sum(lds), b64 = now / S->rz[slot];
+        const double now = P.sum(lds, stop), b64 = now / S->rz[slot];
+        if (stop) return;
         if (br == 0 && threadIdx.x == 0) {
             S->beta = b64;
             S->rz[slot ^ 1] = now;
@@ -2298,7 +2308,7 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_cg_update4(LevelDesc L, double
                                                              const float *__restrict__ idiag, float *__restrict__ z,
                                                              float omega, OpDesc<float> A32,
                                                              const double *__restrict__ pq, int slot) {
-    __shared__ double lds[FOLD ? 16 : 4];
+    __shared__ double lds[FOLD ? FoldPartials::LDS : 4];
     const int br = brick_or_idle(L);
     if (br < 0) return;
     const long c = (long)br * BRICK_CELLS + 4 * threadIdx.x;
@@ -2326,10 +2336,12 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_cg_update4(LevelDesc L, double
         }
     }
     const SolveScalars &Sg = S[g];
-    if (ctl->all_done || Sg.done) return;
+    bool stop = ctl->all_done || Sg.done;
+    if (!FOLD && stop) return;
     double alpha;
     if (FOLD) {
-        const double now = P.sum(lds);
+        const double now = P.sum(lds, stop);
+        if (stop) return;
         alpha = S->rz[slot] / now;
         const bool bad = !(alpha == alpha) || alpha - alpha != 0.0;
         if (br == 0 && threadIdx.x == 0) {
