@@ -234,7 +234,7 @@ __device__ __forceinline__ double wave_max(double v) {
     return v;
 }
 
-// Block-wide sum / max of one value per thread (BLOCK threads).  Result valid in every thread.
+// Block-wide sum of one value per thread (BLOCK threads).  Result valid in every thread.
 __device__ __forceinline__ double block_sum(double v, double *lds) {
     v = wave_sum(v);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -246,21 +246,9 @@ __device__ __forceinline__ double block_sum(double v, double *lds) {
     for (int i = 0; i < nw; ++i) s += lds[i];
     return s;
 }
-__device__ __forceinline__ double block_max(double v, double *lds) {
-    v = wave_max(v);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) lds[wid] = v;
-    __syncthreads();
-    double s = 0.0;
-    const int nw = blockDim.x >> 6;
-    for (int i = 0; i < nw; ++i) s = fmax(s, lds[i]);
-    return s;
-}
 
-// Two block-wide reductions in one LDS round: a by max (AMAX) or sum, b by sum.  Same operations
-// in the same order as block_max / block_sum, so the results are identical to theirs.  lds holds
-// 32 doubles.
+// Two block-wide reductions in one LDS round: a by max (AMAX) or sum, b by sum.  The sum's
+// operations and their order are block_sum's.  lds holds 32 doubles.
 template <bool AMAX>
 __device__ __forceinline__ void block_reduce2(double &a, double &b, double *lds) {
     a = AMAX ? wave_max(a) : wave_sum(a);

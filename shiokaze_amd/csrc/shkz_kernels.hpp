@@ -3023,29 +3023,36 @@ __global__ __launch_bounds__(BRICK_CELLS) void k_coarse_components(LevelDesc L, 
 }
 
 // Sums and sizes of the components of one brick in LDS, one entry per root cell.  The values are added
-// as integers, scaled so that the largest has 53 bits: integer sums do not depend on the order of the
-// atomic adds, 512 of them fit 64 bits, and the scaling loses at most 2^-54 of the largest value per
-// term, no more than a sum in FP64 does.  (One thread adding a component of the whole brick in cell
-// order took 35 us of the 47 us coarse solve of an all-fluid box; this takes about 1 us.)
+// as integers, scaled so that the component's largest has 53 bits: integer sums do not depend on the order of the
+// atomic adds, 512 of them fit 64 bits, and the scaling loses at most 2^-54 of that value per
+// term, no more than a sum in FP64 does.  Each component has a scale of its own: its values may be any
+// number of orders of magnitude below those of another one in the brick.  (One thread adding a component
+// of the whole brick in cell order took 35 us of the 47 us coarse solve of an all-fluid box; this takes
+// about 1 us.)
+//
+// A barrier of the workgroup follows clear(), bound() and add() each.
 struct ComponentSums {
     unsigned long long s[BRICK_CELLS];
     int n[BRICK_CELLS];
+    unsigned top[BRICK_CELLS];  // upper half of the largest |value|
     __device__ __forceinline__ void clear(int e) {
         s[e] = 0;
         n[e] = 0;
+        top[e] = 0;
     }
-    __device__ __forceinline__ static int shift(double mx) {
-        int ex = 0;
-        (void)frexp(mx, &ex);
-        return 53 - ex;
+    __device__ __forceinline__ void bound(int root, double v) {
+        if (root >= 0) atomicMax(&top[root], (unsigned)(__builtin_bit_cast(unsigned long long, fabs(v)) >> 32));
     }
-    __device__ __forceinline__ void add(int root, double v, int sh) {
+    // (biased exponent b: the largest is below 2^(b - 1022))
+    __device__ __forceinline__ int shift(int root) const { return 1075 - max((int)(top[root] >> 20), 1); }
+    __device__ __forceinline__ void add(int root, double v) {
         if (root < 0) return;
-        atomicAdd(&s[root], (unsigned long long)(long long)rint(ldexp(v, sh)));
+        atomicAdd(&s[root], (unsigned long long)(long long)rint(ldexp(v, shift(root))));
         atomicAdd(&n[root], 1);
     }
-    __device__ __forceinline__ double mean(int root, int sh) const {
-        return ldexp((double)(long long)s[root], -sh) / n[root];
+    __device__ __forceinline__ double mean(int root) const {
+        if (top[root] >= 0x7ff00000u) return __builtin_nan("");  // an infinity or NaN among the values
+        return ldexp((double)(long long)s[root], -shift(root)) / n[root];
     }
 };
 
@@ -3100,19 +3107,18 @@ __global__ __launch_bounds__(BRICK_CELLS / CPT) void k_coarse_solve(LevelDesc L,
 #pragma unroll
     for (int u = 0; u < CPT; ++u) rs[u] = r[u];
     if (__syncthreads_or(sing)) {
-        double mx = 0.0;
 #pragma unroll
-        for (int u = 0; u < CPT; ++u) {
-            if (cc[t + u * NT] >= 0) mx = fmax(mx, fabs((double)r[u]));
-            sums.clear(t + u * NT);
-        }
-        const int sh = ComponentSums::shift(block_max(mx, lds));  // its barriers follow the clearing
+        for (int u = 0; u < CPT; ++u) sums.clear(t + u * NT);
+        __syncthreads();
 #pragma unroll
-        for (int u = 0; u < CPT; ++u) sums.add(cc[t + u * NT], (double)r[u], sh);
+        for (int u = 0; u < CPT; ++u) sums.bound(cc[t + u * NT], (double)r[u]);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < CPT; ++u) sums.add(cc[t + u * NT], (double)r[u]);
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < CPT; ++u)
-            if (cc[t + u * NT] >= 0) rs[u] = r[u] - (T)sums.mean(cc[t + u * NT], sh);
+            if (cc[t + u * NT] >= 0) rs[u] = r[u] - (T)sums.mean(cc[t + u * NT]);
     }
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
@@ -3238,7 +3244,6 @@ __global__ __launch_bounds__(BOTTOM_THREADS) void k_bottom(const BottomGrid *__r
     __shared__ __align__(16) int pb[BOTTOM_BRICKS][8];
     __shared__ int16_t code[BRICK_CELLS];
     __shared__ int any[4];
-    __shared__ double red[32];
     __shared__ ComponentSums sums;
     const BottomGrid &G = grids[blockIdx.x];
     const int n = G.n;
@@ -3463,7 +3468,6 @@ __global__ __launch_bounds__(BOTTOM_THREADS) void k_bottom(const BottomGrid *__r
         BottomCells c[2]{};
         int cc[2] = {-1, -1};
         float cz[2] = {0.0f, 0.0f};
-        double mx = 0.0;
         __syncthreads();
         if (mine) {
             const float *gx = cop[0], *gy = cop[1], *gz = cop[2], *dir = cop[3];
@@ -3481,7 +3485,6 @@ __global__ __launch_bounds__(BOTTOM_THREADS) void k_bottom(const BottomGrid *__r
                 o.inv = dir[e] >= 0 && o.diag > 0 ? omega / o.diag : 0.0f;
                 o.rs = n == 1 ? L.rhs[e] : dir[e] >= 0 ? rc[e] : 0.0f;
                 cc[j] = code[e];
-                if (cc[j] >= 0) mx = fmax(mx, fabs((double)o.rs));
             }
         }
         const unsigned long long vote = __ballot(cc[0] >= 0 || cc[1] >= 0);
@@ -3489,13 +3492,16 @@ __global__ __launch_bounds__(BOTTOM_THREADS) void k_bottom(const BottomGrid *__r
         __syncthreads();
         if (any[0] | any[1] | any[2] | any[3]) {
             if (t < BRICK_CELLS) sums.clear(t);
-            const int sh = ComponentSums::shift(block_max(mx, red));
+            __syncthreads();
 #pragma unroll
-            for (int j = 0; j < 2; ++j) sums.add(cc[j], (double)c[j].rs, sh);
+            for (int j = 0; j < 2; ++j) sums.bound(cc[j], (double)c[j].rs);
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 2; ++j) sums.add(cc[j], (double)c[j].rs);
             __syncthreads();
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-                if (cc[j] >= 0) c[j].rs = c[j].rs - (float)sums.mean(cc[j], sh);
+                if (cc[j] >= 0) c[j].rs = c[j].rs - (float)sums.mean(cc[j]);
         }
         bottom_solve(c, cz, t1, sweeps, mine, base, kqlo);
         if (mine) {
