@@ -468,18 +468,24 @@ int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, 
                 if (*e) (void)hipGraphExecDestroy(*e);
                 *e = nullptr;
             }
-            for (int k = 0; k < 2; ++k) {
-                LS_HIP(hipGraphCreate(&building, 0));
+            // both or neither are kept, and with the key that they were built for
+            hipGraphExec_t made[2] = {};
+            for (int k = 0; k < 2 && err == hipSuccess; ++k) {
+                err = hipGraphCreate(&building, 0);
+                if (err != hipSuccess) break;
                 last = nullptr;
                 for (int i = 0; i < (k ? many : 1); ++i) step();
-                hipGraphExec_t made = nullptr;
-                if (err == hipSuccess) err = hipGraphInstantiateWithFlags(&made, building, 0);
+                if (err == hipSuccess) err = hipGraphInstantiateWithFlags(&made[k], building, 0);
                 (void)hipGraphDestroy(building);
                 building = nullptr;
-                if (err != hipSuccess)
-                    return shkz_fail(SHKZ_ERR_DEVICE, "building an iteration's graph failed: %s", hipGetErrorString(err));
-                (k ? L->exec_many : L->exec) = made;
             }
+            if (err != hipSuccess) {
+                for (hipGraphExec_t e : made)
+                    if (e) (void)hipGraphExecDestroy(e);
+                return shkz_fail(SHKZ_ERR_DEVICE, "building an iteration's graph failed: %s", hipGetErrorString(err));
+            }
+            L->exec = made[0];
+            L->exec_many = made[1];
             L->exec_key = key;
             L->exec_n = n;
             L->exec_prec = (int)jacobi;

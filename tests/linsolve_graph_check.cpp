@@ -1,0 +1,114 @@
+// LinSolver's kept graphs after a failed build: the solver reports the failure, holds nothing of it, and the next
+// system replays graphs of its own size only.  The HIP calls that ls_solve_device makes are stand-ins: a graph is a
+// record of its first kernel argument (the system's size), and one chosen call fails.
+#include "../shiokaze_amd/csrc/shkz_linsolve.hip"
+#include "host_hip.hpp"
+
+#include <cstdio>
+
+int shkz_set_error(int code, const char *) { return code; }
+
+namespace {
+struct Graph {
+    int n = 0;
+};
+int live_execs = 0, wrong_launches = 0, launches = 0, want_n = 0, polls = 0;
+int calls_left = -1;  // the call that fails (counted over the building calls), -1: none
+bool fails() { return calls_left >= 0 && calls_left-- == 0; }
+}  // namespace
+
+extern "C" {
+hipError_t hipGraphCreate(hipGraph_t *g, unsigned) {
+    if (fails()) return hipErrorOutOfMemory;
+    *g = (hipGraph_t) new Graph;
+    return hipSuccess;
+}
+hipError_t hipGraphAddKernelNode(hipGraphNode_t *node, hipGraph_t g, const hipGraphNode_t *, size_t,
+                                 const hipKernelNodeParams *p) {
+    if (fails()) return hipErrorOutOfMemory;
+    const int n = *(const int *)p->kernelParams[0];
+    if (!((Graph *)g)->n) ((Graph *)g)->n = n;
+    *node = (hipGraphNode_t)g;
+    return hipSuccess;
+}
+hipError_t hipGraphInstantiateWithFlags(hipGraphExec_t *e, hipGraph_t g, unsigned long long) {
+    if (fails()) return hipErrorOutOfMemory;
+    *e = (hipGraphExec_t) new Graph(*(Graph *)g);
+    ++live_execs;
+    return hipSuccess;
+}
+hipError_t hipGraphDestroy(hipGraph_t g) {
+    delete (Graph *)g;
+    return hipSuccess;
+}
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) {
+    if (!e) return hipErrorInvalidValue;
+    delete (Graph *)e;
+    --live_execs;
+    return hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
+    ++launches;
+    wrong_launches += !e || ((Graph *)e)->n != want_n;
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *dst, const void *, size_t, hipMemcpyKind, hipStream_t) {
+    auto *s = (LsScalars *)dst;
+    std::memset(s, 0, sizeof(*s));
+    s->maxit = 1000;
+    s->done = polls++ > 1;
+    s->iter = 8 * polls;  // the second chunk: long enough for the longer graph
+    s->r0 = 1.0;
+    s->rinf = 0.9;
+    s->tol = 1e-6;
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
+}
+
+static int solve(shkz_linsolver &L, int n) {
+    static double memory[1 << 12];
+    const LsArrays D{(const int *)memory, (const int *)memory + 1, memory, memory, memory + 100, memory + 200, memory + 300,
+                     memory + 400, memory + 500, memory + 600, memory + 700, memory + 800, memory + 900,
+                     (LsScalars *)(memory + 1000)};
+    shkz_linsolve_params prm;
+    shkz_linsolve_default_params(&prm);
+    shkz_linsolve_result res;
+    polls = 0;
+    want_n = n;
+    return ls_solve_device(&L, nullptr, D, n, &prm, &res, true);
+}
+
+int main() {
+    int bad = 0, builds = 0;
+    for (int n : {100, LS_FOLD_ROWS + 100}) {  // both forms of an iteration
+        for (int fail_at = 0;; ++fail_at) {
+            shkz_linsolver L;
+            LsScalars host;
+            L.host_s = &host;
+            launches = wrong_launches = live_execs = 0;
+            const int first = solve(L, n);
+            calls_left = fail_at;
+            const int other = solve(L, n - 1);
+            const bool failed = calls_left < 0;
+            calls_left = -1;
+            if (!failed) break;  // fewer building calls than that
+            ++builds;
+            const int held = live_execs;
+            const int again = solve(L, n);
+            if (first != SHKZ_OK || other != SHKZ_ERR_DEVICE || held != 0 || again != SHKZ_OK || live_execs != 2 ||
+                wrong_launches || !launches || L.exec_n != n) {
+                ++bad;
+                std::printf("n=%d, failure at call %d: %d %d %d, held %d, live %d, %d of %d launches of another graph\n", n, fail_at,
+                            first, other, again, held, live_execs, wrong_launches, launches);
+            }
+        }
+    }
+    std::printf("%d failed builds, %d went wrong\n", builds, bad);
+    if (!bad && builds > 4) std::printf("OK\n");
+    return bad;
+}

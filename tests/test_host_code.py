@@ -8,7 +8,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 def build_and_run(tmp_path, name):
     exe = tmp_path / name
-    subprocess.check_call(["hipcc", "--offload-host-only", "-x", "hip", "-std=c++17", "-Wno-unused-result",
+    subprocess.check_call(["hipcc", "--offload-host-only", "-x", "hip", "-std=c++17", "-O0", "-Wno-unused-result",
                            os.path.join(ROOT, "tests", name + ".cpp"), "-o", str(exe),
                            "-Wl,--unresolved-symbols=ignore-all", "-lpthread"])
     p = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
@@ -18,3 +18,7 @@ def build_and_run(tmp_path, name):
 
 def test_graph_key_tells_every_argument_apart(tmp_path):
     build_and_run(tmp_path, "graph_key_check")
+
+
+def test_linsolver_after_a_failed_graph_build(tmp_path):
+    build_and_run(tmp_path, "linsolve_graph_check")
