@@ -2438,6 +2438,9 @@ static int host_copies(shkz_ctx *C, const std::vector<HostCopy> &copies, hipMemc
             if (c.bytes) SHKZ_HIP(hipMemcpy(c.dst, c.src, c.bytes, kind));
         return SHKZ_OK;
     }
+    // As hipMemcpy does, after the caller's work on the null stream, which may still fill or read its arrays.  The
+    // host waits: what a copy of pageable memory reads, it reads during the call.
+    SHKZ_HIP(hipStreamSynchronize(nullptr));
     std::vector<HostCopy> pieces;
     for (const HostCopy &c : copies)
         for (size_t o = 0; o < c.bytes; o += COPY_PIECE)

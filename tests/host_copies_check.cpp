@@ -1,0 +1,61 @@
+// Copies between the caller's host arrays and the device (host_copies) against a stand-in for the HIP calls they make:
+// device memory is host memory, and the caller's own work on the null stream is done when that stream is waited for.
+#include "../shiokaze_amd/csrc/shkz_runtime.hip"
+#include "host_hip.hpp"
+
+#include <cstdio>
+
+static std::function<void()> null_stream_work;
+static void wait_null_stream() {
+    if (null_stream_work) std::exchange(null_stream_work, nullptr)();
+}
+
+extern "C" {
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+    static char streams[64];
+    static int n;
+    *s = (hipStream_t)&streams[n++];
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) {
+    if (!s) wait_null_stream();
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void *dst, const void *src, size_t n, hipMemcpyKind) {
+    wait_null_stream();
+    std::memcpy(dst, src, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t) {
+    std::memcpy(dst, src, n);
+    return hipSuccess;
+}
+}
+
+// The caller's arrays are still being written by its own work on the null stream when it calls.
+static bool after_null_stream(size_t bytes, hipMemcpyKind kind) {
+    shkz_ctx C;
+    std::vector<char> src(bytes, 'a'), other(100, 'a'), dst(bytes, 'x'), dst2(100, 'x');
+    null_stream_work = [&]() {
+        std::fill(src.begin(), src.end(), 'b');
+        std::fill(other.begin(), other.end(), 'c');
+    };
+    const int rc = host_copies(&C, {{dst.data(), src.data(), bytes}, {dst2.data(), other.data(), other.size()}}, kind);
+    null_stream_work = nullptr;
+    return rc == SHKZ_OK && dst == std::vector<char>(bytes, 'b') && dst2 == std::vector<char>(100, 'c');
+}
+
+int main(int, char **argv) {
+    const std::string what = argv[1];
+    bool ok = true;
+    if (what == "null-stream")
+        for (size_t bytes : {COPY_PARALLEL / 2, COPY_PARALLEL, 5 * COPY_PARALLEL / 2 + 17})
+            for (hipMemcpyKind kind : {hipMemcpyHostToDevice, hipMemcpyDeviceToHost}) {
+                const bool good = after_null_stream(bytes, kind);
+                if (!good) std::printf("%zu bytes, kind %d: the arrays as they were before\n", bytes, (int)kind);
+                ok = ok && good;
+            }
+    if (ok) std::printf("OK\n");
+    return ok ? 0 : 1;
+}

@@ -6,12 +6,12 @@ import subprocess
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def build_and_run(tmp_path, name):
+def build_and_run(tmp_path, name, *args):
     exe = tmp_path / name
     subprocess.check_call(["hipcc", "--offload-host-only", "-x", "hip", "-std=c++17", "-O0", "-Wno-unused-result",
                            os.path.join(ROOT, "tests", name + ".cpp"), "-o", str(exe),
                            "-Wl,--unresolved-symbols=ignore-all", "-lpthread"])
-    p = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    p = subprocess.run([str(exe), *args], capture_output=True, text=True, timeout=120)
     assert p.returncode == 0 and "OK" in p.stdout, p.stdout + p.stderr
     return p.stdout
 
@@ -22,3 +22,7 @@ def test_graph_key_tells_every_argument_apart(tmp_path):
 
 def test_linsolver_after_a_failed_graph_build(tmp_path):
     build_and_run(tmp_path, "linsolve_graph_check")
+
+
+def test_host_copies_follow_the_null_stream(tmp_path):
+    build_and_run(tmp_path, "host_copies_check", "null-stream")
