@@ -2433,7 +2433,16 @@ constexpr size_t COPY_PARALLEL = (size_t)4 << 20, COPY_PIECE = (size_t)1 << 20;
 static int host_copies(shkz_ctx *C, const std::vector<HostCopy> &copies, hipMemcpyKind kind) {
     size_t total = 0;
     for (const HostCopy &c : copies) total += c.bytes;
-    if (total < COPY_PARALLEL) {
+    // in order where two of them write the same bytes (an output that the grids of a batch share keeps the last
+    // grid's values)
+    std::vector<std::pair<uintptr_t, size_t>> written;
+    for (const HostCopy &c : copies)
+        if (c.bytes) written.emplace_back((uintptr_t)c.dst, c.bytes);
+    std::sort(written.begin(), written.end());
+    bool overlap = false;
+    for (size_t i = 1; i < written.size(); ++i)
+        overlap = overlap || written[i - 1].first + written[i - 1].second > written[i].first;
+    if (total < COPY_PARALLEL || overlap) {
         for (const HostCopy &c : copies)
             if (c.bytes) SHKZ_HIP(hipMemcpy(c.dst, c.src, c.bytes, kind));
         return SHKZ_OK;

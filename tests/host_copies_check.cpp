@@ -3,6 +3,7 @@
 #include "../shiokaze_amd/csrc/shkz_runtime.hip"
 #include "host_hip.hpp"
 
+#include <chrono>
 #include <cstdio>
 
 static std::function<void()> null_stream_work;
@@ -28,6 +29,7 @@ hipError_t hipMemcpy(void *dst, const void *src, size_t n, hipMemcpyKind) {
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t) {
+    if (*(const char *)src == 's') std::this_thread::sleep_for(std::chrono::milliseconds(20));  // a slow copy
     std::memcpy(dst, src, n);
     return hipSuccess;
 }
@@ -46,6 +48,17 @@ static bool after_null_stream(size_t bytes, hipMemcpyKind kind) {
     return rc == SHKZ_OK && dst == std::vector<char>(bytes, 'b') && dst2 == std::vector<char>(100, 'c');
 }
 
+// Two grids of a batch share an output array, whole or in part: the last one's values stay.
+static bool last_of_overlapping(size_t bytes, size_t offset) {
+    shkz_ctx C;
+    std::vector<char> first(bytes, 's'), last(bytes, 'b'), dst(offset + bytes, 'x'), want(dst);
+    std::fill_n(want.begin(), bytes, 's');
+    std::fill_n(want.begin() + (ptrdiff_t)offset, bytes, 'b');
+    const int rc = host_copies(&C, {{dst.data(), first.data(), bytes}, {dst.data() + offset, last.data(), bytes}},
+                               hipMemcpyDeviceToHost);
+    return rc == SHKZ_OK && dst == want;
+}
+
 int main(int, char **argv) {
     const std::string what = argv[1];
     bool ok = true;
@@ -54,6 +67,13 @@ int main(int, char **argv) {
             for (hipMemcpyKind kind : {hipMemcpyHostToDevice, hipMemcpyDeviceToHost}) {
                 const bool good = after_null_stream(bytes, kind);
                 if (!good) std::printf("%zu bytes, kind %d: the arrays as they were before\n", bytes, (int)kind);
+                ok = ok && good;
+            }
+    if (what == "overlap")
+        for (size_t bytes : {COPY_PARALLEL / 4, 6 * COPY_PIECE})
+            for (size_t offset : {(size_t)0, bytes / 2, bytes}) {
+                const bool good = last_of_overlapping(bytes, offset);
+                if (!good) std::printf("%zu bytes at %zu: values of the copy before\n", bytes, offset);
                 ok = ok && good;
             }
     if (ok) std::printf("OK\n");

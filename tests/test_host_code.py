@@ -26,3 +26,7 @@ def test_linsolver_after_a_failed_graph_build(tmp_path):
 
 def test_host_copies_follow_the_null_stream(tmp_path):
     build_and_run(tmp_path, "host_copies_check", "null-stream")
+
+
+def test_host_copies_of_overlapping_arrays_in_order(tmp_path):
+    build_and_run(tmp_path, "host_copies_check", "overlap")
