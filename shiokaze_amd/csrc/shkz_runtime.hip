@@ -33,9 +33,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -2472,8 +2472,8 @@ static int host_copies(shkz_ctx *C, const std::vector<HostCopy> &copies, hipMemc
     for (int t = 1; t < WORKERS; ++t) {
         try {
             threads.emplace_back(worker, t);
-        } catch (const std::system_error &) {
-            break;  // fewer threads copy the same pieces
+        } catch (const std::exception &) {
+            break;  // no thread, or no memory for one: fewer threads copy the same pieces
         }
     }
     worker(0);

@@ -35,6 +35,15 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, h
 }
 }
 
+// Allocations left before one fails (-1: none does).
+static std::atomic<int> allocations_left{-1};
+void *operator new(size_t n) {
+    if (allocations_left >= 0 && allocations_left-- == 0) throw std::bad_alloc();
+    return std::malloc(n);
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
 // The caller's arrays are still being written by its own work on the null stream when it calls.
 static bool after_null_stream(size_t bytes, hipMemcpyKind kind) {
     shkz_ctx C;
@@ -59,6 +68,30 @@ static bool last_of_overlapping(size_t bytes, size_t offset) {
     return rc == SHKZ_OK && dst == want;
 }
 
+// Each allocation of a call fails in turn: the call copies everything with fewer threads, or ends with the exception,
+// never with the process.
+static bool short_of_memory() {
+    bool ok = true;
+    int copied = 0;
+    for (int left = 0;; ++left) {
+        shkz_ctx C;
+        std::vector<char> src(2 * COPY_PARALLEL, 'b'), dst(src.size(), 'x');
+        const std::vector<HostCopy> copies{{dst.data(), src.data(), src.size()}};
+        allocations_left = left;
+        try {
+            const int rc = host_copies(&C, copies, hipMemcpyHostToDevice);
+            const bool reached = allocations_left < 0;
+            allocations_left = -1;
+            ok = ok && rc == SHKZ_OK && dst == src;
+            if (!reached) break;  // fewer allocations than that
+            ++copied;
+        } catch (const std::bad_alloc &) {
+            allocations_left = -1;
+        }
+    }
+    return ok && copied > 0;
+}
+
 int main(int, char **argv) {
     const std::string what = argv[1];
     bool ok = true;
@@ -76,6 +109,7 @@ int main(int, char **argv) {
                 if (!good) std::printf("%zu bytes at %zu: values of the copy before\n", bytes, offset);
                 ok = ok && good;
             }
+    if (what == "memory") ok = short_of_memory();
     if (ok) std::printf("OK\n");
     return ok ? 0 : 1;
 }

@@ -30,3 +30,7 @@ def test_host_copies_follow_the_null_stream(tmp_path):
 
 def test_host_copies_of_overlapping_arrays_in_order(tmp_path):
     build_and_run(tmp_path, "host_copies_check", "overlap")
+
+
+def test_host_copies_short_of_memory(tmp_path):
+    build_and_run(tmp_path, "host_copies_check", "memory")
