@@ -515,6 +515,9 @@ struct shkz_ctx {
     // each grid's last levels in one workgroup (SHKZ_NO_BOTTOM=1: one launch per level and step, as on
     // the levels above them; the results are the same)
     bool use_bottom = true;
+    // brick-local V-cycle: the prolongation inside the first post-smoothing application (SHKZ_NO_JOIN=1: a
+    // launch of its own; the results are the same)
+    bool join_prolong = true;
     // coarse levels of at most this many stored bricks smooth with multi-sweep launches unless the
     // autotuner picks another limit (SHKZ_MULTI_MAX_BRICKS overrides the default; the results do
     // not depend on it)
@@ -824,6 +827,7 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
     const T om = (T)P.omega;
     const double es = (double)sizeof(T);
     const bool bottom = brick_smoother && P.with_bottom();
+    const bool join = brick_smoother && C->join_prolong;
     // which of a coarse level's two vectors holds its smoothed z
     const int bottom_slot = final_slot(P.pre_c, P.post_c, false, false, true);
     // coarse levels small enough smooth with one multi-sweep launch per smoothing step (Jacobi);
@@ -970,8 +974,8 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
             zoth[l] = oth;
             continue;
         }
-        if (brick_smoother) {
-            // joins the first post-smoothing application
+        if (join) {
+            // in the first post-smoothing application
         } else if constexpr (sizeof(T) == 4)
             K.go(f ? "prolong_L0" : "prolong_Lc", l, 3 * es, es * (double)Lc.unknowns - usave(C, l, es),
                  row4_launch(L.nbricks, f).grid, row4_launch(L.nbricks, f).block, f ? k_prolong4<1> : k_prolong4<0>,
@@ -984,7 +988,7 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
             if constexpr (sizeof(T) == 4) {
                 if (brick_smoother) {
                     const dim3 gb(brick_grid(L.nbricks));
-                    const bool k3 = P.local_k == 3, pro = s == 0;
+                    const bool k3 = P.local_k == 3, pro = join && s == 0;
                     const T *zc = (const T *)zcur[l + 1];
                     const double zc_bytes = pro ? es * (double)Lc.unknowns : 0;
                     if (last_dot)
@@ -3010,6 +3014,8 @@ int shkz_create(int device, uint64_t hbm_budget_bytes, shkz_ctx **out) {
     C->fuse_krylov = !(nf && nf[0] == '1');
     const char *nbt = std::getenv("SHKZ_NO_BOTTOM");
     C->use_bottom = !(nbt && nbt[0] == '1');
+    const char *njn = std::getenv("SHKZ_NO_JOIN");
+    C->join_prolong = !(njn && njn[0] == '1');
     C->under_profiler = std::getenv("ROCP_TOOL_LIBRARIES") || std::getenv("ROCPROF_OUTPUT_PATH");
     const char *mb = std::getenv("SHKZ_MULTI_MAX_BRICKS");
     if (mb && mb[0]) C->multi_max_bricks = std::atoi(mb);
