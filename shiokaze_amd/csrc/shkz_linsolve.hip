@@ -36,7 +36,7 @@ constexpr int LS_ROWS = LS_BLOCK / LS_LANES;       // rows per SpMV block
 
 struct LsScalars {
     double rz, alpha, beta, rinf, r0, tol;
-    int32_t iter, maxit, done, converged, status, pad;
+    int32_t iter, maxit, done, converged, status, nnz;
 };
 
 // Block reduction of (a: max or sum, b: sum) into partials[2*block].
@@ -168,15 +168,27 @@ __device__ __forceinline__ void ls_after_update(LsScalars &s, double a, double b
     }
 }
 
-// ---- Small systems (at most LS_FOLD_ROWS rows): an iteration in two launches instead of five, each a
+// ---- Small systems (ls_folds): an iteration in two launches instead of five, each a
 // launch's boundary and a trip or two to memory (2.3 to 3.8 us) for under 1 us of work.  Every
 // workgroup of the kernel that needs a scalar forms it from the block partials itself, with
 // k_ls_finalize's sums in its order, so both forms give the same bits.  The record S alternates between
 // two slots (all workgroups read one, the first writes the other), the direction between two buffers
 // (its neighbours' new values are formed from the old ones on the fly), and the two kinds of partials
-// have a buffer each.  The limit keeps what the workgroups of the update read together, 16 n^2 / 8192
-// bytes of partials, at 8 MB or 2 us from the L2s; a larger system gains less and less of its time.
+// have a buffer each.
+//
+// Two costs grow with the system.  The workgroups of the update read 16 n^2 / 8192 bytes of partials together
+// (us per iteration, five launches / two: 20,112 rows of a pressure system 14.1 / 9.8, 59,932 15.4 / 12.6,
+// 81,524 16.3 / 15.4, 119,356 18.9 / 20.3, 446,368 37.3 / 68.5).  And the product reads two vectors per
+// non-zero instead of one, which costs more the wider apart a row's columns lie (rows of neighbours / of
+// random columns: 60,000 of 129 46.2 / 44.1 and 64.2 / 53.6, of 193 40.8 / 43.0 and 62.8 / 67.5, of 513 127 / 138 and
+// 169 / 201; 30,000 of 513 65.3 / 58.8 and 71.4 / 72.0; 20,000 of 385 43.6 / 41.5 and 56.0 / 51.8; 4,000 of 513
+// 59.1 / 54.6 and 36.9 / 36.2, of about 1000 138 / 113 and 70 / 86): past the limits the random columns lose, and
+// all of the large systems.
 constexpr int LS_FOLD_ROWS = 1 << 16;
+constexpr int64_t LS_FOLD_NNZ = 10 << 20, LS_FOLD_ROW_NNZ = 640;
+inline bool ls_folds(int64_t n, int64_t nnz) {
+    return n <= LS_FOLD_ROWS && nnz <= LS_FOLD_NNZ && nnz <= LS_FOLD_ROW_NNZ * n;
+}
 
 // Sums (or max and sum) of nb partials as k_ls_finalize's 1024 threads form them, in LS_BLOCK threads:
 // thread t stands for t, t + 256, t + 512 and t + 768.  Valid in every thread.
@@ -295,9 +307,9 @@ __global__ __launch_bounds__(LS_BLOCK) void k_ls_update_folded(int n, double *__
 enum { LS_FIN_INIT = 0, LS_FIN_PQ = 1, LS_FIN_UPDATE = 2 };
 
 // One block combines the partials of nb blocks in block order and updates the scalars, as the
-// reference's loop does between its BLAS calls (pcg_solver.h:250-290).
+// reference's loop does between its BLAS calls (pcg_solver.h:250-290).  nnz: the last row pointer (LS_FIN_INIT only).
 __global__ __launch_bounds__(1024) void k_ls_finalize(const double *__restrict__ partials, int nb, LsScalars *S, int op,
-                                                      double residual, int maxit) {
+                                                      double residual, int maxit, const int *nnz) {
     __shared__ double lds[2][16];
     if (op != LS_FIN_INIT && S->done) return;
     const bool amax = op != LS_FIN_PQ;
@@ -328,6 +340,7 @@ __global__ __launch_bounds__(1024) void k_ls_finalize(const double *__restrict__
         s.rz = b;
         s.iter = 0;
         s.maxit = maxit;
+        s.nnz = *nnz;
         s.tol = (residual < 1e-30 ? 1e-30 : residual) * a;
         s.status = 0;
         s.converged = 0;
@@ -368,7 +381,7 @@ struct shkz_linsolver {
     LsScalars *host_s = nullptr;
     hipGraphExec_t exec = nullptr, exec_many = nullptr;  // the shortest replay and a longer one
     std::vector<const void *> exec_key;
-    int exec_n = -1, exec_prec = -1;
+    int exec_n = -1, exec_prec = -1, exec_fold = -1;
 };
 
 namespace {
@@ -426,7 +439,6 @@ int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, 
     double *zz = jacobi ? z : r;  // without a preconditioner z is r itself
     const unsigned nb_v = blocks_of(n, LS_BLOCK), nb_m = blocks_of(n, LS_ROWS);
     const int maxit = prm->max_iterations > 0 ? prm->max_iterations : 30000;
-    const bool fold = n <= LS_FOLD_ROWS;
     // a launch on the stream, or a node of the graph under construction
     hipGraph_t building = nullptr;
     hipGraphNode_t last = nullptr;
@@ -437,11 +449,21 @@ int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, 
     };
     if (jacobi) go(nb_v, LS_BLOCK, k_ls_idiag, n, rp, cl, vl, id);
     go(nb_v, LS_BLOCK, k_ls_init, n, b, x, r, z, M, part);
-    go(1, 1024, k_ls_finalize, part, (int)nb_v, S, (int)LS_FIN_INIT, prm->residual, maxit);
-    if (fold)
+    go(1, 1024, k_ls_finalize, part, (int)nb_v, S, (int)LS_FIN_INIT, prm->residual, maxit, rp + n);
+    // the first direction (p = z), with its product where the scalars may be folded
+    if (n <= LS_FOLD_ROWS)
         go(nb_m, LS_BLOCK, k_ls_direction_spmv<true>, n, rp, cl, vl, zz, p, p, q, S, S, part, (int)nb_v, D.partials2);
     else
         go(nb_v, LS_BLOCK, k_ls_direction, n, zz, p, S, 1);
+    LsScalars h;
+    auto read = [&]() -> int {
+        LS_HIP(hipMemcpyAsync(L->host_s, S, sizeof(LsScalars), hipMemcpyDeviceToHost, s));
+        LS_HIP(hipStreamSynchronize(s));
+        h = *L->host_s;
+        return SHKZ_OK;
+    };
+    LS_TRY(read());
+    const bool fold = ls_folds(n, h.nnz);  // (known with the first record: the row pointers may be on the device only)
     // one step: an iteration, or with the scalars folded two, which alternate the records and directions
     auto step = [&]() {
         if (fold) {
@@ -454,16 +476,16 @@ int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, 
             return;
         }
         go(nb_m, LS_BLOCK, k_ls_spmv_dot, n, rp, cl, vl, p, q, S, part);
-        go(1, 1024, k_ls_finalize, part, (int)nb_m, S, (int)LS_FIN_PQ, 0.0, 0);
+        go(1, 1024, k_ls_finalize, part, (int)nb_m, S, (int)LS_FIN_PQ, 0.0, 0, (const int *)nullptr);
         go(nb_v, LS_BLOCK, k_ls_update, n, x, r, z, p, q, M, S, part);
-        go(1, 1024, k_ls_finalize, part, (int)nb_v, S, (int)LS_FIN_UPDATE, 0.0, 0);
+        go(1, 1024, k_ls_finalize, part, (int)nb_v, S, (int)LS_FIN_UPDATE, 0.0, 0, (const int *)nullptr);
         go(nb_v, LS_BLOCK, k_ls_direction, n, zz, p, S, 0);
     };
     const int per_step = fold ? 2 : 1, many = 8;  // iterations of a step, steps of the longer graph
-    if (graph) {
+    if (graph && !h.done) {
         // reused while the arrays and sizes stay the same
         std::vector<const void *> key = {rp, cl, vl, x, r, z, p, q, id, part, S, D.p2, D.partials2};
-        if (!L->exec || L->exec_key != key || L->exec_n != n || L->exec_prec != (int)jacobi) {
+        if (!L->exec || L->exec_key != key || L->exec_n != n || L->exec_prec != (int)jacobi || L->exec_fold != (int)fold) {
             for (hipGraphExec_t *e : {&L->exec, &L->exec_many}) {
                 if (*e) (void)hipGraphExecDestroy(*e);
                 *e = nullptr;
@@ -489,14 +511,11 @@ int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, 
             L->exec_key = key;
             L->exec_n = n;
             L->exec_prec = (int)jacobi;
+            L->exec_fold = (int)fold;
         }
     }
     int chunk = 8;
-    for (;;) {
-        LS_HIP(hipMemcpyAsync(L->host_s, S, sizeof(LsScalars), hipMemcpyDeviceToHost, s));
-        LS_HIP(hipStreamSynchronize(s));
-        const LsScalars h = *L->host_s;
-        if (h.done) break;
+    while (!h.done) {
         // size the next chunk from the observed contraction rate (the replays after convergence
         // return at once)
         int next = chunk;
@@ -511,9 +530,9 @@ int ls_solve_device(shkz_linsolver *L, hipStream_t s, const LsArrays &D, int n, 
             if (graph) LS_HIP(hipGraphLaunch(L->exec, s));
             else step();
         }
+        LS_TRY(read());
     }
     LS_HIP(hipGetLastError());
-    const LsScalars h = *L->host_s;
     res->iterations = h.iter;
     res->converged = h.converged;
     res->reresid = h.r0 > 0 ? h.rinf / h.r0 : 0.0;

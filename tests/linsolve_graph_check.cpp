@@ -1,6 +1,7 @@
-// LinSolver's kept graphs after a failed build: the solver reports the failure, holds nothing of it, and the next
-// system replays graphs of its own size only.  The HIP calls that ls_solve_device makes are stand-ins: a graph is a
-// record of its first kernel argument (the system's size), and one chosen call fails.
+// LinSolver's kept graphs.  After a failed build the solver reports the failure, holds nothing of it, and the next
+// system replays graphs of its own size only; and the form of an iteration (two launches or five) follows the rows and non-zeros of each system, whatever
+// was solved before on the same arrays.  The HIP calls that ls_solve_device makes are stand-ins: a graph is a
+// record of its first kernel argument (the system's size) and its launches, and one chosen call fails.
 #include "../shiokaze_amd/csrc/shkz_linsolve.hip"
 #include "host_hip.hpp"
 
@@ -10,9 +11,9 @@ int shkz_set_error(int code, const char *) { return code; }
 
 namespace {
 struct Graph {
-    int n = 0;
+    int n = 0, nodes = 0;
 };
-int live_execs = 0, wrong_launches = 0, launches = 0, want_n = 0, polls = 0;
+int live_execs = 0, wrong_launches = 0, launches = 0, want_n = 0, polls = 0, nnz = 0;
 int calls_left = -1;  // the call that fails (counted over the building calls), -1: none
 bool fails() { return calls_left >= 0 && calls_left-- == 0; }
 }  // namespace
@@ -28,6 +29,7 @@ hipError_t hipGraphAddKernelNode(hipGraphNode_t *node, hipGraph_t g, const hipGr
     if (fails()) return hipErrorOutOfMemory;
     const int n = *(const int *)p->kernelParams[0];
     if (!((Graph *)g)->n) ((Graph *)g)->n = n;
+    ++((Graph *)g)->nodes;
     *node = (hipGraphNode_t)g;
     return hipSuccess;
 }
@@ -56,6 +58,7 @@ hipError_t hipMemcpyAsync(void *dst, const void *, size_t, hipMemcpyKind, hipStr
     auto *s = (LsScalars *)dst;
     std::memset(s, 0, sizeof(*s));
     s->maxit = 1000;
+    s->nnz = nnz;
     s->done = polls++ > 1;
     s->iter = 8 * polls;  // the second chunk: long enough for the longer graph
     s->r0 = 1.0;
@@ -83,7 +86,7 @@ static int solve(shkz_linsolver &L, int n) {
     return ls_solve_device(&L, nullptr, D, n, &prm, &res, true);
 }
 
-int main() {
+static int after_failed_builds() {
     int bad = 0, builds = 0;
     for (int n : {100, LS_FOLD_ROWS + 100}) {  // both forms of an iteration
         for (int fail_at = 0;; ++fail_at) {
@@ -112,3 +115,31 @@ int main() {
     if (!bad && builds > 4) std::printf("OK\n");
     return bad;
 }
+
+static int forms() {
+    int bad = 0;
+    // the form: four launches for two iterations, or five for one
+    shkz_linsolver L;
+    LsScalars host;
+    L.host_s = &host;
+    const int rows = 1000, most = LS_FOLD_ROWS;
+    const struct {
+        int n, nnz, nodes;
+    } systems[] = {{rows, 7 * rows, 4},  {rows, 640 * rows, 4},     {rows, 640 * rows + 1, 5}, {rows, 7 * rows, 4},
+                   {most, 7 * most, 4},  {most, 10 << 20, 4},       {most, (10 << 20) + 1, 5},  {most + 1, 7 * most, 5},
+                   {1, 1, 4},            {most, 2147483647, 5}};
+    for (const auto &x : systems) {
+        nnz = x.nnz;
+        wrong_launches = 0;
+        const int rc = solve(L, x.n);
+        const int nodes = L.exec ? ((Graph *)L.exec)->nodes : 0, longer = L.exec_many ? ((Graph *)L.exec_many)->nodes : 0;
+        if (rc != SHKZ_OK || wrong_launches || nodes != x.nodes || longer != 8 * x.nodes) {
+            ++bad;
+            std::printf("n=%d with %d non-zeros: %d, graphs of %d and %d launches\n", x.n, x.nnz, rc, nodes, longer);
+        }
+    }
+    if (!bad) std::printf("OK\n");
+    return bad;
+}
+
+int main(int argc, char **argv) { return argc > 1 && argv[1] == std::string("form") ? forms() : after_failed_builds(); }

@@ -34,3 +34,7 @@ def test_host_copies_of_overlapping_arrays_in_order(tmp_path):
 
 def test_host_copies_short_of_memory(tmp_path):
     build_and_run(tmp_path, "host_copies_check", "memory")
+
+
+def test_linsolver_form_follows_rows_and_nonzeros(tmp_path):
+    build_and_run(tmp_path, "linsolve_graph_check", "form")
