@@ -46,8 +46,12 @@ enum {
     BM_COARSEST = 1,  // the brick's grid ends on this level (its coarse solve handles it)
     BM_UNIFORM = 2,   // level 0: the operator is one constant on the brick (UniCoef)
     BM_BOTTOM = 4,    // a level of the grid's bottom (BottomGrid): k_bottom works on it
-    BM_BELOW = 8      // ... and not the bottom's first level, whose right-hand side the restriction forms
+    BM_BELOW = 8,     // ... and not the bottom's first level, whose right-hand side the restriction forms
+    BM_LOOSE = 16     // a cell across one of its faces may be coupled to it and yet be no unknown (COUPLED_OUT)
 };
+// A NaN in the level set leaves the liquid cells beside it with a NaN for their diagonal, so that no kernel takes them
+// as unknowns (dir >= 0), but with their couplings.  A coarse cell over such cells and no unknown has this dir instead of -1.
+constexpr int COUPLED_OUT = -2;
 struct __align__(32) BrickMeta {
     int nbr[6];
     int grid;

@@ -261,6 +261,14 @@ __device__ __forceinline__ int table_grid(const GridTable<D> &T, int &local) {
     return g;
 }
 
+// Marks the bricks beside brick br (BM_LOOSE) if one of this wavefront's cells in it is coupled and no unknown.
+__device__ __forceinline__ void mark_loose(BrickMeta *meta, int br, bool coupled_out) {
+    if (__ballot(coupled_out) == 0) return;
+    const int lane = threadIdx.x & 63;
+    const int nb = lane < 6 ? meta[br].nbr[lane] : -1;
+    if (nb >= 0) atomicOr(&meta[nb].flags, BM_LOOSE);
+}
+
 // Unknown labelling (macpressuresolver3.cpp:121-156): a liquid cell is an unknown when an
 // in-bounds liquid neighbour shares a face with nonzero area (rho is nonzero between two liquid
 // cells).  Writes cell flags (bit0 liquid, bit1 unknown) and per brick bit0 = holds an unknown, bit1 =
@@ -573,6 +581,7 @@ __global__ __launch_bounds__(BLOCK) void k_operator(GridTable<OperatorGrid> T, L
         rhs += F.rhs_correct;
         if (F.warm) x0 = F.warm[cell_index(G, i, j, k)];
     }
+    mark_loose(FIN.meta, br, dir != dir);
     dir64[c] = dir;
     gx64[c] = g[0];
     gy64[c] = g[1];
@@ -629,7 +638,7 @@ __global__ __launch_bounds__(BLOCK) void k_operator(GridTable<OperatorGrid> T, L
     }
     {
         if (uniform) {
-            FIN.meta[br].flags = L.meta[br].flags | BM_UNIFORM;
+            atomicOr(&FIN.meta[br].flags, BM_UNIFORM);  // (the bricks beside may mark this one)
             UniCoef u;
             u.g64 = Gu;
             u.id64 = iref64;
@@ -660,7 +669,7 @@ __global__ __launch_bounds__(BLOCK) void k_coarsen(LevelDesc Lf, OpDesc<Ti> Af, 
               K = Lc.bxyz[3 * br + 2] * BRICK + (t & 7);
     const long c = (long)br * BRICK_CELLS + t;
     double sdir = 0.0, sg[3] = {0.0, 0.0, 0.0};
-    bool any = false;
+    bool any = false, coupled = false;
     const int fi0 = 2 * I, fj0 = 2 * J, fk0 = 2 * K;
     if (fi0 < F.ni && fj0 < F.nj && fk0 < F.nk) {
         const int fb = Lf.bmap[F.bmap_off + ((fi0 >> 3) * F.nby + (fj0 >> 3)) * F.nbz + (fk0 >> 3)];
@@ -675,13 +684,15 @@ __global__ __launch_bounds__(BLOCK) void k_coarsen(LevelDesc Lf, OpDesc<Ti> Af, 
                             any = true;
                             sdir += d;
                         }
+                        coupled = coupled | !(d >= -1.0);
                         if (a == 0) sg[0] += (double)Af.gx[f];
                         if (bb == 0) sg[1] += (double)Af.gy[f];
                         if (cc == 0) sg[2] += (double)Af.gz[f];
                     }
         }
     }
-    dir[c] = any ? (To)sdir : (To)(-1);
+    mark_loose(const_cast<BrickMeta *>(Lc.meta), br, coupled && !any);
+    dir[c] = any ? (To)sdir : (To)(coupled ? COUPLED_OUT : -1);
     gx[c] = any ? (To)(0.5 * sg[0]) : (To)0;
     gy[c] = any ? (To)(0.5 * sg[1]) : (To)0;
     gz[c] = any ? (To)(0.5 * sg[2]) : (To)0;
@@ -1865,7 +1876,8 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_pre_local4(LevelDesc L, OpDesc
 // same 6^3, interpolated axis by axis through LDS (12 operations per row at the end where eight
 // corners per cell take 84); the rows beside a cell's own come from the
 // lanes that hold them (through LDS) or, across a face, are loaded and corrected here as well.  A cell
-// across a face that is no unknown is corrected too: its coupling is 0.  Two launches took 29.5 us on the
+// across a face that is no unknown is corrected too, where its coupling is 0 (else BM_LOOSE; reading every such cell's
+// dir instead took 25.6 us on 256^3's finest level, 22.6 without).  Two launches took 29.5 us on the
 // finest level of 256^3 (9248 bricks) and 9 us on a level of 40, this one 21.7 and 5.6.
 constexpr int PRO_EDGE = 6, PRO_FINE = 10;  // coarse and fine rows per axis, those across the faces included
 constexpr float PRO_NEAR = 0.75f, PRO_FAR = 0.25f;
@@ -1957,7 +1969,18 @@ __global__ __launch_bounds__(ROW4_THREADS) void k_post_local4(LevelDesc L, OpDes
         unpack4(mix4(P.y[at(pro_near(li), lj)], P.y[at(pro_far(li), lj)]), own);
         unpack4(mix4(P.y[at(pro_near(gi), lj)], P.y[at(pro_far(gi), lj)]), gx);
         unpack4(mix4(P.y[at(pro_near(li), gj)], P.y[at(pro_far(li), gj)]), gy);
-        raw.end += pro_mix(P.ye[at(pro_near(li), lj)], P.ye[at(pro_far(li), lj)]);
+        float end = pro_mix(P.ye[at(pro_near(li), lj)], P.ye[at(pro_far(li), lj)]);
+        if (m.flags & BM_LOOSE) {
+            float d[4];
+            load4(A.dir, li == 0 ? N.ixm : N.ixp, d);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) gx[j] = d[j] >= 0 ? gx[j] : 0.0f;
+            load4(A.dir, lj == 0 ? N.iym : N.iyp, d);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) gy[j] = d[j] >= 0 ? gy[j] : 0.0f;
+            end = A.dir[N.iz] >= 0 ? end : 0.0f;
+        }
+        raw.end += end;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             raw.c[j] = (uniform || dir[j] >= 0) ? raw.c[j] + own[j] : raw.c[j];
