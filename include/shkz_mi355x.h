@@ -61,13 +61,14 @@ enum shkz_precision {
     SHKZ_PREC_FP64 = 1   /* every vector and operator in FP64 */
 };
 
-/* Finest-level smoother of the V-cycle.  Coarser levels always use damped Jacobi. */
+/* Smoother of the V-cycle. */
 enum shkz_smoother {
     SHKZ_SMOOTH_DEFAULT = 0, /* brick-local in mixed precision, Jacobi in FP64 (or the tuner's choice) */
     SHKZ_SMOOTH_JACOBI = 1,  /* damped Jacobi, one sweep per mg_pre/post_sweeps */
-    SHKZ_SMOOTH_BRICK = 2    /* brick-local symmetric Gauss-Seidel (block Jacobi across 8^3 bricks, two
-                                red-black sweeps inside each), one application per mg_pre/post_sweeps;
-                                mixed precision only (FP64 solves use Jacobi) */
+    SHKZ_SMOOTH_BRICK = 2    /* brick-local symmetric Gauss-Seidel on every level (block Jacobi across 8^3
+                                bricks, mg_local_sweeps red-black sweeps inside each on the finest level, three
+                                on the others), one application per mg_pre/post_sweeps; mixed precision only
+                                (FP64 solves use Jacobi) */
 };
 
 enum shkz_norm {
@@ -137,7 +138,7 @@ typedef struct shkz_params {
                                      (repeated solves of the built system; the returned projection
                                      uses the best controls).  Cached per process, and in the file
                                      named by the environment variable SHKZ_TUNE_CACHE if set. */
-    int32_t mg_smoother;          /* finest-level smoother (shkz_smoother; 0 = library default / tuned) */
+    int32_t mg_smoother;          /* smoother (shkz_smoother; 0 = library default / tuned) */
     int32_t mg_local_sweeps;      /* brick-local smoother: symmetric Gauss-Seidel sweeps per finest-level
                                      application, 2 or 3 (0 = library default 2 / tuned) */
     int32_t reserved[2];

@@ -78,8 +78,10 @@ constexpr int VF_BLOCK = 256;
 // A wavefront takes G groups of 64 consecutive faces, all of their activity bytes loaded at once.  Most
 // groups of a domain are inactive, and with one group per wavefront the launch is bound by how many wavefronts
 // are resident over the round trip of one byte load (256^3, 50 million faces: k_constrain 223 us against 157,
-// k_constrain_apply 67 against 33, k_adv_face_bwd 273 against 237).  G = 8 where the launch keeps VF_MANY wavefronts all the same (twice
-// what the chip holds); a smaller field takes one group per wavefront, all of them resident at once.
+// k_constrain_apply 67 against 33, k_adv_face_bwd 273 against 237).  G = 8 where the launch keeps VF_MANY wavefronts
+// all the same (twice what the chip holds); a smaller field takes one group per wavefront, all of them resident
+// at once.  The step's three calls with eight groups / by the rule / with one (us): 96^3 279 / 249 / 251, 128^3
+// 376 / 352 / 350, 140^3 434 / 425 / 426, 160^3 541 / 536 / 546, 200^3 866 / 869 / 905.
 constexpr int VF_GROUPS = 8;
 constexpr size_t VF_MANY = 16384;
 inline bool vf_many(const size_t n[3]) { return (n[0] + n[1] + n[2]) / (64 * VF_GROUPS) >= VF_MANY; }

@@ -1022,8 +1022,10 @@ __device__ __forceinline__ void finalize_update(const FinUpdate &F, const LevelD
 // The first partials of the n <= FOLD_BRICKS bricks of a single grid, summed by every 128-thread
 // workgroup of the kernel that uses the sum, so that no finalize launch (3 to 4 us, most of it its
 // boundary and one trip to memory) stands between the producer and it.  load() issues the loads,
-// sum() adds; all threads call both.  The limit keeps what all workgroups read
-// together (8 n^2 bytes) well under the time of a launch: 8 MB from the L2s at 1024.
+// sum() adds; all threads call both.  What all workgroups read together grows with the square of the
+// bricks, 8 MB from the L2s at 1024, and the loads of a larger limit cost registers at every size.  Projections to 1e-6
+// with k_finalize / with the limit at 1024 / at 4096 (us): 95 bricks 901 / 848 / 856, 774 bricks 1368 / 1319 / 1336,
+// 1439 bricks 1593 / 1597 / 1579, 2152 bricks 2162 / 2163 / 2228.
 //
 // A breakdown that such a kernel finds is recorded in the flags that it tests on entry, by the workgroup of
 // brick 0 while others still enter.  So the two wavefronts of a workgroup don't go by flags of their own: sum()
@@ -1496,7 +1498,7 @@ __device__ __forceinline__ Row4Coef<T> row4_coef(const OpDesc<T> &A, const Row4N
     return row4_coef_join(row4_coef_load(A, N), N);
 }
 
-// jacobi_brick on the lane's four cells (same per-cell arithmetic); DOT adds rhs.zout of the
+// One sweep of the lane's four cells (k_jacobi_dot's arithmetic per cell); DOT adds rhs.zout of the
 // unknowns, in cell order, to part.
 template <int DOT, class T>
 __device__ __forceinline__ void jacobi_row4(const LevelDesc &L, const OpDesc<T> &A, const T *__restrict__ idiag,

@@ -704,7 +704,9 @@ static bool smooth_k_supported(int k) {
 // Levels that smooth with one multi-sweep launch per step: up to max_bricks stored bricks, and in FP64
 // with four sweeps (90 registers, 16 wavefronts: one workgroup per CU) no more than the CUs: on 224
 // bricks the pre-smoothing takes 10 us in one launch against 12 us sweep by sweep, the post-smoothing
-// with the prolongation 12 us against 18 us; a second round of workgroups would lose.
+// with the prolongation 12 us against 18 us; a second round of workgroups loses.  FP64 projections to 1e-6,
+// sweep by sweep / up to 256 bricks / on any level (ms): 1,439 bricks on the finest level 3.23 / 2.93 / 2.94,
+// 2,152 bricks 4.78 / 4.41 / 4.54, 3,737 bricks 6.10 / 5.68 / 5.98.
 template <class T>
 static bool smooth_k_level(int nbricks, int max_bricks, int k) {
     if (sizeof(T) == 8 && k == 4) max_bricks = std::min(max_bricks, 256);
@@ -910,7 +912,7 @@ static T *vcycle(shkz_ctx *C, Launcher &K, Problem &P, const T *rhs0, T *z0, T *
             // finest level: one sweep from zero, then plain sweeps (cheaper there than the fused
             // two-sweep kernel, whose on-the-fly neighbour values cost 12 extra loads per cell)
             if (f && first_done) {
-                // z = omega * idiag * rhs was written by the residual update (k_cg_update4z)
+                // z = omega * idiag * rhs was written by the residual update (k_cg_update4<1>, k_cg_update<T, 1>)
             } else if constexpr (sizeof(T) == 4)
                 K.go(f ? "smooth_first_L0" : "smooth_first_Lc", l, 3 * es, -usave(C, l, es),
                      row4_launch(L.nbricks, f).grid, row4_launch(L.nbricks, f).block,
@@ -1138,8 +1140,8 @@ static int krylov(shkz_ctx *C, Launcher &K, Problem &P, T *x, T *r, T *p, T *q, 
     // FP32 preconditioned form with fused kernels: the loop is rotated so that each iteration
     // ends with the operator apply of the next direction, formed in the same kernel
     // (k_apply_dot4p), and starts with the residual update that also performs the V-cycle's first
-    // sweep (k_cg_update4z); the direction alternates between two buffers, so one captured graph
-    // holds two iterations.  Same kernels' arithmetic, same results as the separate kernels.
+    // smoothing step (k_cg_update4<1 or 2>); the direction alternates between two buffers, so there are
+    // two graphs, of an iteration each.  Same kernels' arithmetic, same results as the separate kernels.
     const bool fused = sizeof(T) == 4 && precond && !keep_dir && C->fuse_krylov && P.kp2;
     const bool brick = P.smoother == SHKZ_SMOOTH_BRICK;
     // alpha and beta formed by the kernels that use them (single grids up to FOLD_BRICKS bricks), p.q
@@ -2426,8 +2428,10 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
 
 // Copies between the caller's (pageable) arrays and the device, complete on return.  One thread's copies go
 // through the runtime's staging buffer at the rate of its memcpy; from COPY_PARALLEL bytes on, pieces
-// are copied by up to four threads, each on a stream of its own (eight were no faster).  96x128x80, 39 MB: the
-// projection 3863 us with one thread, 2940 us here.
+// are copied by up to four threads, each on a stream of its own (eight were no faster).  Projections, one thread /
+// four (us): 32^3 719 / 865 (at best 706 / 712), 48^3 924 / 893, 56^3 (2.8 MB in, 3.5 out) 1087 / 1021, 60^3
+// 1152 / 1106, 64^3 1414 / 1126, 96^3 2793 / 2060.  Threads help from about 1 MB on, but by no more than 6% and not in
+// every run below 4 MB, where the line lies.
 struct HostCopy {
     void *dst;
     const void *src;
