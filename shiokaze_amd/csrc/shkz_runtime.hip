@@ -2387,18 +2387,20 @@ static int project_stages(shkz_ctx *C, const shkz_grid *grids, int ngrids, const
     const double t_solve = now_ms();
 
     // ---------------------------------------------------------------- per grid: scatter + update
-    launch_grids<OutputGrid>(K, "output", ngrids, OUT_THREADS,
-                             [&](int g, OutputGrid &F, double &bytes) {
-                                 GridJob &J = jobs[g];
-                                 const shkz_grid *in = J.in;
-                                 F = OutputGrid{J.G, F0.gl[g], in->pressure, in->pressure64,
-                                                J.scene ? J.scene->p : nullptr, J.cflag, in->unknown_out};
-                                 bytes += (double)J.M * (24 + (J.G.phi64 ? 8 : 4) + (in->solid ? 4 : 0) +
-                                                         (in->pressure ? 4 : 0) + (in->pressure64 ? 8 : 0) +
-                                                         (J.scene ? 8 : 0) + (in->unknown_out ? 2 : 0));
-                                 return output_blocks(J.G);
-                             },
-                             k_output, F0.desc, (const double *)P.x64);
+    for (const bool thin : {false, true})
+        launch_grids<OutputGrid>(K, "output", ngrids, OUT_THREADS,
+                                 [&](int g, OutputGrid &F, double &bytes) {
+                                     GridJob &J = jobs[g];
+                                     if (output_thin(J.G) != thin) return 0;
+                                     const shkz_grid *in = J.in;
+                                     F = OutputGrid{J.G, F0.gl[g], in->pressure, in->pressure64,
+                                                    J.scene ? J.scene->p : nullptr, J.cflag, in->unknown_out};
+                                     bytes += (double)J.M * (24 + (J.G.phi64 ? 8 : 4) + (in->solid ? 4 : 0) +
+                                                             (in->pressure ? 4 : 0) + (in->pressure64 ? 8 : 0) +
+                                                             (J.scene ? 8 : 0) + (in->unknown_out ? 2 : 0));
+                                     return output_blocks(J.G);
+                                 },
+                                 thin ? k_output<1> : k_output<0>, F0.desc, (const double *)P.x64);
     for (int g = 0; g < ngrids; ++g) {
         GridJob &J = jobs[g];
         if (J.scene) J.scene->has_pressure = true;
