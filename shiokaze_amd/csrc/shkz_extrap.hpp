@@ -360,13 +360,17 @@ __device__ __forceinline__ T acc(T v, double term) {
     return (T)((double)v + term);
 }
 
-// The solid sample and its derivative at p (nodal array), in the level set's type T.  Returns the
-// interpolated value where the point is inside (negative); 0 where it is not.
+// The solid sample and its derivative at the centre p of a face (nodal array), in the level set's type T: der and
+// true where the point is inside (negative).  The centre's corner (corner_of) is the face's own (i, j, k),
+// the last but one node where that lies past it, so the corners are loaded and tested without FP64.
 template <class T>
-__device__ __forceinline__ double solid_sample(const VelField &F, const double p[3], double der[3], bool &inside) {
+__device__ __forceinline__ bool inside_solid(const VelField &F, int i, int j, int k, const double p[3], double der[3]) {
 #pragma clang fp contract(off)
     const int s[3] = {F.w + 1, F.h + 1, F.d + 1};
-    const Corner c = corner_of(s, p);
+    Corner c;
+    c.i = i < F.w - 1 ? i : F.w - 1;
+    c.j = j < F.h - 1 ? j : F.h - 1;
+    c.k = k < F.d - 1 ? k : F.d - 1;
     const T *S = (const T *)F.solid;
     T v[8];
     unsigned q[8];
@@ -379,29 +383,25 @@ __device__ __forceinline__ double solid_sample(const VelField &F, const double p
     bool any_neg = false;
 #pragma unroll
     for (int n = 0; n < 8; ++n) any_neg = any_neg || v[n] < T(0);
-    if (!any_neg) {
-        inside = false;
-        return 0.0;
-    }
+    if (!any_neg) return false;
+    c = corner_of(s, p);
     double w[8];
     interp_weights(c, w);
     T val = T(0);
 #pragma unroll
     for (int n = 0; n < 8; ++n)
         if (w[n] != 0.0) val = acc<T>(val, (double)v[n] * w[n]);
-    inside = (double)val < 0.0;
-    if (inside) {
-        double dw[24];
-        deriv_weights(c, dw);
+    if (!((double)val < 0.0)) return false;
+    double dw[24];
+    deriv_weights(c, dw);
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            T r = T(0);
+    for (int a = 0; a < 3; ++a) {
+        T r = T(0);
 #pragma unroll
-            for (int n = 0; n < 8; ++n) r = acc<T>(r, dw[8 * a + n] * (double)v[n]);
-            der[a] = (double)r;
-        }
+        for (int n = 0; n < 8; ++n) r = acc<T>(r, dw[8 * a + n] * (double)v[n]);
+        der[a] = (double)r;
     }
-    return (double)val;
+    return true;
 }
 
 // Component b of the saved velocity at p (macarray_interpolator3.h:43-50): inactive faces read 0.
@@ -430,27 +430,6 @@ __device__ __forceinline__ double vel_sample(const VelField &F, const float *con
     return (double)val;
 }
 
-// Whether any of the eight solid nodes around the centre of face (a; i, j, k) is negative.  The centre's
-// corner (corner_of) is its own (i, j, k), the last but one node where that lies past it.
-template <class T>
-__device__ __forceinline__ bool near_solid(const VelField &F, int i, int j, int k) {
-    const int s[3] = {F.w + 1, F.h + 1, F.d + 1};
-    Corner c;
-    c.i = i < F.w - 1 ? i : F.w - 1;
-    c.j = j < F.h - 1 ? j : F.h - 1;
-    c.k = k < F.d - 1 ? k : F.d - 1;
-    unsigned q[8];
-    corner_indices(c, s, q);
-    const T *S = (const T *)F.solid;
-    T v[8];
-#pragma unroll
-    for (int n = 0; n < 8; ++n) v[n] = S[q[n]];
-    bool neg = false;
-#pragma unroll
-    for (int n = 0; n < 8; ++n) neg = neg || v[n] < T(0);
-    return neg;
-}
-
 // Activity code of a face whose constrained value waits in the side buffer (k_constrain_apply).
 constexpr uint8_t ACT_CONSTRAINED = 255;
 
@@ -462,20 +441,19 @@ constexpr uint8_t ACT_CONSTRAINED = 255;
 // ACT_CONSTRAINED.  The velocity arrays are only read here.
 //
 // Bound by issue: most of the faces are inactive and most of the others away from the solid, so the decode
-// divides by multiplying and the corner test needs no FP64 (256^3: 223 us before, 157 us).
+// divides by multiplying and the corner test needs no FP64 (256^3: 223 us before, 157 us).  The corners that the
+// test loads serve the interpolation too: with loads of its own for each, 130x140x150 faces near a solid everywhere
+// (random nodes) took 207 us a call, 179 here.
 __device__ __forceinline__ void constrain_face(const VelField &F, int a, size_t f, int t, float *X0, float *X1, float *X2,
                                                bool with_solid) {
 #pragma clang fp contract(off)
     int i, j, k;
     vf_decode(F, a, f, i, j, k);
-    if (with_solid && (F.solid64 ? near_solid<double>(F, i, j, k) : near_solid<float>(F, i, j, k))) {
+    if (with_solid) {
         const float *const Sv[3] = {F.vel[0], F.vel[1], F.vel[2]};
         const double p[3] = {i + 0.5 * (a != 0), j + 0.5 * (a != 1), k + 0.5 * (a != 2)};
         double der[3] = {0.0, 0.0, 0.0};
-        bool inside;
-        if (F.solid64) solid_sample<double>(F, p, der, inside);
-        else solid_sample<float>(F, p, der, inside);
-        if (inside) {
+        if (F.solid64 ? inside_solid<double>(F, i, j, k, p, der) : inside_solid<float>(F, i, j, k, p, der)) {
             double nrm[3];
 #pragma unroll
             for (int b = 0; b < 3; ++b) nrm[b] = vf_div_dx(F, der[b]);
