@@ -1,4 +1,4 @@
-// LinSolver's kept graphs.  After a failed build the solver reports the failure, holds nothing of it, and the next
+// LinSolver's kept graphs.  They are built for a system that comes again or takes long.  After a failed build the solver reports the failure, holds nothing of it, and the next
 // system replays graphs of its own size only; and the form of an iteration (two launches or five) follows the rows and non-zeros of each system, whatever
 // was solved before on the same arrays.  The HIP calls that ls_solve_device makes are stand-ins: a graph is a
 // record of its first kernel argument (the system's size) and its launches, and one chosen call fails.
@@ -13,7 +13,7 @@ namespace {
 struct Graph {
     int n = 0, nodes = 0;
 };
-int live_execs = 0, wrong_launches = 0, launches = 0, want_n = 0, polls = 0, nnz = 0;
+int live_execs = 0, wrong_launches = 0, launches = 0, want_n = 0, polls = 0, nnz = 0, chunks = 2, builds_done = 0, direct = 0;
 int calls_left = -1;  // the call that fails (counted over the building calls), -1: none
 bool fails() { return calls_left >= 0 && calls_left-- == 0; }
 }  // namespace
@@ -37,6 +37,7 @@ hipError_t hipGraphInstantiateWithFlags(hipGraphExec_t *e, hipGraph_t g, unsigne
     if (fails()) return hipErrorOutOfMemory;
     *e = (hipGraphExec_t) new Graph(*(Graph *)g);
     ++live_execs;
+    ++builds_done;
     return hipSuccess;
 }
 hipError_t hipGraphDestroy(hipGraph_t g) {
@@ -59,8 +60,8 @@ hipError_t hipMemcpyAsync(void *dst, const void *, size_t, hipMemcpyKind, hipStr
     std::memset(s, 0, sizeof(*s));
     s->maxit = 1000;
     s->nnz = nnz;
-    s->done = polls++ > 1;
-    s->iter = 8 * polls;  // the second chunk: long enough for the longer graph
+    s->done = polls >= chunks;
+    s->iter = LS_BUILD_AFTER * polls++;  // the second chunk: replayed, and long enough for the longer graph
     s->r0 = 1.0;
     s->rinf = 0.9;
     s->tol = 1e-6;
@@ -68,7 +69,10 @@ hipError_t hipMemcpyAsync(void *dst, const void *, size_t, hipMemcpyKind, hipStr
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) {
+    ++direct;
+    return hipSuccess;
+}
 hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
 }
@@ -104,7 +108,7 @@ static int after_failed_builds() {
             const int held = live_execs;
             const int again = solve(L, n);
             if (first != SHKZ_OK || other != SHKZ_ERR_DEVICE || held != 0 || again != SHKZ_OK || live_execs != 2 ||
-                wrong_launches || !launches || L.exec_n != n) {
+                wrong_launches || !launches || L.built.n != n) {
                 ++bad;
                 std::printf("n=%d, failure at call %d: %d %d %d, held %d, live %d, %d of %d launches of another graph\n", n, fail_at,
                             first, other, again, held, live_execs, wrong_launches, launches);
@@ -142,4 +146,35 @@ static int forms() {
     return bad;
 }
 
-int main(int argc, char **argv) { return argc > 1 && argv[1] == std::string("form") ? forms() : after_failed_builds(); }
+// Systems that converge within the first chunk: launched directly at first sight, replayed when they come again.
+static int short_solves() {
+    int bad = 0;
+    chunks = 1;
+    shkz_linsolver L;
+    LsScalars host;
+    L.host_s = &host;
+    const struct {
+        int n;
+        bool replayed, built;
+    } solves[] = {{100, false, false}, {100, true, true},  {100, true, false}, {99, false, false}, {100, true, false},
+                  {99, false, false},  {99, true, true},   {99, true, false},  {100, false, false}, {100, true, true},
+                  {LS_FOLD_ROWS + 5, false, false}, {LS_FOLD_ROWS + 5, true, true}};
+    for (const auto &x : solves) {
+        launches = wrong_launches = builds_done = direct = 0;
+        const int rc = solve(L, x.n);
+        const bool by_launches = direct > 8;  // (the set-up is launched in any case)
+        if (rc != SHKZ_OK || wrong_launches || (launches > 0) != x.replayed || by_launches == x.replayed ||
+            builds_done != (x.built ? 2 : 0)) {
+            ++bad;
+            std::printf("n=%d: %d, %d replays (%d wrong), %d launches, %d graphs built\n", x.n, rc, launches, wrong_launches, direct,
+                        builds_done);
+        }
+    }
+    if (!bad) std::printf("OK\n");
+    return bad;
+}
+
+int main(int argc, char **argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    return what == "form" ? forms() : what == "short" ? short_solves() : after_failed_builds();
+}

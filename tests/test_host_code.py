@@ -38,3 +38,7 @@ def test_host_copies_short_of_memory(tmp_path):
 
 def test_linsolver_form_follows_rows_and_nonzeros(tmp_path):
     build_and_run(tmp_path, "linsolve_graph_check", "form")
+
+
+def test_linsolver_short_solves_build_no_graph(tmp_path):
+    build_and_run(tmp_path, "linsolve_graph_check", "short")
